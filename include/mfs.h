@@ -346,7 +346,9 @@ typedef struct {
                       FP64 inner 1 -> 1 row, 2 -> 2 rows; with r, d, q
                       kept in registers: 3 -> 1 row (wg_size up to 512),
                       4 -> 2 rows (these need nint <= rows * wg_size for
-                      every cell, else MFS_ERR_ARG)                         */
+                      every cell, else MFS_ERR_ARG).  MIXED on cells of
+                      n <= 10 runs the matrix-core kernel, which has one
+                      shape, for every variant and wg_size accepted        */
   int fallback_wg_size;  /* MIXED: shape of the FP64 pass over the problems  */
   int fallback_variant;  /* the FP32 launch could not solve (0 = the FP64
                             autotuned shape, else as wg_size / variant)      */

@@ -15,9 +15,11 @@
 //    indices).  Blocks that couple to boundary nodes are zero here; their
 //    effect is in the right-hand side b = -K_IB g.
 //  * b, x: FP64 [interior node][3][24] per cell.
-//  * one task = (cell, group of 8 bases); a persistent kernel pulls tasks
-//    from an atomic queue (largest cells first) and runs FP32 Jacobi-PCG with
-//    FP64 refinement for its 8 right-hand sides, search directions in LDS.
+//  * one task = a cell and some of its bases; a persistent kernel pulls tasks
+//    from an atomic queue (largest cells first).  Mixed precision on cells of
+//    n <= 10 runs the matrix-core kernel of batch_mfma.hpp (FP32 Jacobi-PCG
+//    with FP64 refinement, 24 or 12 bases per task, K in its tiled layout);
+//    FP64, and mixed on larger cells, runs k_batch_solve (8 bases per task).
 //
 // Reference-trace mode (MFS_TRACE_REFERENCE) replaces the boundary data
 // hat_c * e_d by the reference's edge -> face hierarchy (MsFEM_Grid.h:
@@ -56,32 +58,24 @@ constexpr int RG = 8;    // right-hand sides per task
 // Row stride (values) of p in LDS, and of d when it lives there: the 3 x RG
 // values of a row plus padding.  A wave's lanes own consecutive rows, so its
 // reads of one component address consecutive rows; with packed rows (96 B
-// FP32, 192 B FP64) they had 2- / 4-way bank conflicts.  FP64 and the FP32
-// register variants use 16-byte reads: 208 B and 112 B rows put any 8 (or
-// 16) consecutive rows in distinct banks.  The FP32 slab variants use 104 B
-// rows (8-byte reads, distinct banks for 16 consecutive rows), which keeps
-// two workgroups per CU on cells of up to 729 rows.
-template <typename T, bool REG>
-constexpr int lds_row() { return sizeof(T) == 8 ? 3 * RG + 2 : REG ? 3 * RG + 4 : 3 * RG + 2; }
-template <typename T, bool REG>
-__device__ __forceinline__ int64_t lds_at(int v, int a, int r) { return (int64_t)v * lds_row<T, REG>() + a * RG + r; }
+// FP32, 192 B FP64) they had 2- / 4-way bank conflicts.  FP64 uses 16-byte
+// reads: 208 B rows put any 8 consecutive rows in distinct banks; FP32 104 B
+// rows (8-byte reads, distinct banks for 16 consecutive rows).
+constexpr int kLdsRow = 3 * RG + 2;
+__device__ __forceinline__ int64_t lds_at(int v, int a, int r) { return (int64_t)v * kLdsRow + a * RG + r; }
 constexpr int NB = 24;   // bases per cell
 constexpr int MAXN = 12; // largest supported cell subdivision (FP32 inner; FP64 inner: 10)
-// Kernel variants per precision, picked by the autotuner: the number of
-// rows a thread carries through the inner-iteration phases at once (more
-// rows keep more loads in flight per wave, fewer rows leave registers for
-// two waves per SIMD), and whether the per-row vectors r, d, q live in
-// registers (variants 3 and 4; only for batches whose cells all have
-// nint <= rows * workgroup size) or in a global scratch slab.  (Measured
-// and dropped: K rings of 5 stencil points, part of each row's K kept in
-// registers for the whole task, and forcing three or four waves per SIMD;
-// each costs more in spills than it hides in latency.)
+// Kernel variants of k_batch_solve per precision, picked by the autotuner:
+// the number of rows a thread carries through the inner-iteration phases at
+// once (more rows keep more loads in flight per wave, fewer rows leave
+// registers for two waves per SIMD), and whether the per-row vectors r, d, q
+// live in registers (FP64 variants 3 and 4; only for batches whose cells all
+// have nint <= rows * workgroup size) or in a global scratch slab.  In mixed
+// precision variants 3 and 4 exist for cells that the matrix-core kernel
+// takes (n <= 10), which then serves all four.
 constexpr int kRptF32[4] = {2, 3, 1, 2}, kRptF64[4] = {1, 2, 1, 2};
 constexpr bool kRegVar[4] = {false, false, true, true};
 constexpr int kVariants[2] = {4, 4};  // per precision: FP32 inner, FP64 inner
-// Register-resident variants keep d (the inner correction) in LDS behind p,
-// except the one-row FP32 variant, which has the registers for it.
-constexpr bool d_in_lds(bool fp64, int rpt) { return fp64 || rpt != 1; }
 // Largest workgroup of a variant: one register-resident row per thread
 // needs a thread per interior node, so that form takes up to 512 threads.
 constexpr int max_threads(bool reg, int rpt) { return reg && rpt == 1 ? 512 : 256; }
@@ -109,7 +103,24 @@ struct Cell {
   double ox, oy, oz;
   int64_t et0;  // reference-trace mode: first edge-profile entry (12*(n+1)*2 per cell)
   int64_t ft0;  // reference-trace mode: first face-trace entry (6*(n+1)^2*36 per cell)
+  int64_t kt0;  // first FP32 matrix value
 };
+
+// Record of a workgroup-uniform cell with the fields the solve kernels use in
+// scalar registers (K is read through a buffer resource formed from them).
+__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ Cell uniform_cell(const Cell* cells, int cell) {
+  Cell C = cells[cell];
+  C.n = __builtin_amdgcn_readfirstlane(C.n);
+  C.nint = __builtin_amdgcn_readfirstlane(C.nint);
+  C.int0 = uniform_i64(C.int0);
+  C.kt0 = uniform_i64(C.kt0);
+  return C;
+}
 
 // Coarse faces f = 2*ax + side (side 1: coordinate n); face coordinates
 // (u, v) run along the two other axes in increasing order.  Coarse edges
@@ -188,21 +199,28 @@ struct SolveArgs {
   int* flags;            // [cell][24]: bit0 not converged, bit1 guess rejected,
                          // bit2 FP32 inner solve failed, bit3 handed to the FP64 pass,
                          // bit4 FP64 solve from the guess failed and was redone from zero
-  // FP32 launch: tasks with a failed right-hand side are appended to the
-  // FP64 pass's list (count, then cells, then groups); FP64 pass: its task
-  // list and count (written by the FP32 launch), queue 0 only
-  int* fb_count;
-  int* fb_cell;
-  int* fb_group;
-  const int* ntasks_dev;
+  int list_failures;      // FP32 launch: an FP64 pass follows (sets flag bit 3)
+  const int* ntasks_dev;  // FP64 pass: length of its task list, queue 0 only
   double tol, inner_tol;
   int maxit;
   int inner_cap;  // iterations one inner solve may take before the RHS is
                   // declared failed in this precision (FP32: handed to FP64)
   int use_guess;
   int max_nint;  // largest cell of the batch (rows of the LDS vectors)
-  int stage_x;   // register variants: the residual pass stages the FP64 iterate in LDS
 };
+
+// FP32 matrix layout of the matrix-core kernel (batch_mfma.hpp): per 16
+// nodes, 12 chunks of 4 consecutive (stencil point, column) entries, 48
+// (node, row) pairs of 16 bytes each.
+constexpr int KT_CHUNKS = 12;                 // ceil(15 * 3 / 4)
+constexpr int KT_GROUP = KT_CHUNKS * 48 * 4;  // floats per 16 nodes
+constexpr int kMfmaMaxN = 10;                 // largest cell it takes
+__host__ __device__ constexpr int mfma_groups(int nint) { return (nint + 15) / 16; }
+__host__ __device__ constexpr int64_t k32_tile_floats(int nint) { return (int64_t)mfma_groups(nint) * KT_GROUP; }
+__host__ __device__ __forceinline__ int k32_tile_index(int v, int s, int a, int b) {
+  const int t = 3 * s + b;
+  return (((v >> 4) * KT_CHUNKS + (t >> 2)) * 48 + (v & 15) * 3 + a) * 4 + (t & 3);
+}
 
 __device__ __forceinline__ int interior_index(int i, int j, int k, int m) {
   return (i - 1) + m * ((j - 1) + m * (k - 1));
@@ -276,7 +294,7 @@ __global__ __launch_bounds__(256) void k_cell_assemble(const Cell* __restrict__ 
                                                        const uint32_t* __restrict__ g_ent,
                                                        const double* __restrict__ E, double nu, double h, int conv,
                                                        const double* __restrict__ ft, int64_t total_int,
-                                                       float* __restrict__ K32,
+                                                       int tiled, float* __restrict__ K32,
                                                        double* __restrict__ K64, float* __restrict__ dinv32,
                                                        double* __restrict__ dinv64, double* __restrict__ b64) {
   for (int64_t gv = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; gv < total_int;
@@ -298,7 +316,7 @@ __global__ __launch_bounds__(256) void k_cell_assemble(const Cell* __restrict__ 
     double bacc[3][NB];
     for (int a = 0; a < 3; a++)
       for (int q = 0; q < NB; q++) bacc[a][q] = 0.0;
-    float* K32c = K32 + C.int0 * (NS * 9);
+    float* K32c = K32 + C.kt0;
     double* K64c = K64 + C.int0 * (NS * 9);
     for (int s = 0; s < NS; s++) {
       const int ni = i + c_stencil[s][0], nj = j + c_stencil[s][1], nk = k + c_stencil[s][2];
@@ -319,7 +337,7 @@ __global__ __launch_bounds__(256) void k_cell_assemble(const Cell* __restrict__ 
         for (int b = 0; b < 3; b++) {
           const int64_t at = (int64_t)(s * 9 + 3 * a + b) * nint + v;
           K64c[at] = interior ? Kb[a][b] : 0.0;
-          K32c[at] = interior ? (float)Kb[a][b] : 0.0f;
+          K32c[tiled ? k32_tile_index(v, s, a, b) : at] = interior ? (float)Kb[a][b] : 0.0f;
         }
       if (!interior) {
         if (ft == nullptr) {
@@ -394,66 +412,11 @@ __device__ __forceinline__ int stencil_offset(int s, int m) {
 // neighbour's coordinates, its bounds test and a select.
 __device__ __forceinline__ int neighbour_row(int v, int off, int nint) { return min(max(v + off, 0), nint - 1); }
 
-// The same product for RPT rows of one thread at once (rows v[k]; rows with
-// ok[k] false are computed on row 0 and discarded by the caller).  The K
-// values of all RPT rows for the next stencil point are loaded while the
-// current point is applied, so a wave keeps RPT*9 loads in flight and the
-// row passes of one thread do not queue behind each other.
-template <typename KT, typename VT, int RPT, typename Load>
-__device__ __forceinline__ void stencil_rows(const KT* __restrict__ Kc, int nint, const int (&v)[RPT],
-                                             const bool (&ok)[RPT], int m, Load load, VT (&acc)[RPT][3][RG]) {
-  int vi[RPT];
-  const KT* kp[RPT];
-  KT kn[RPT][9];
-#pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    vi[q] = ok[q] ? v[q] : 0;
-    kp[q] = Kc + vi[q];
-#pragma unroll
-    for (int e = 0; e < 9; e++) kn[q][e] = kp[q][(int64_t)e * nint];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int r = 0; r < RG; r++) acc[q][a][r] = 0;
-  }
-#pragma unroll 1
-  for (int s = 0; s < NS; s++) {
-    VT kv[RPT][9];
-#pragma unroll
-    for (int q = 0; q < RPT; q++)
-#pragma unroll
-      for (int e = 0; e < 9; e++) kv[q][e] = (VT)kn[q][e];
-    if (s + 1 < NS) {
-#pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        kp[q] += (int64_t)9 * nint;
-#pragma unroll
-        for (int e = 0; e < 9; e++) kn[q][e] = kp[q][(int64_t)e * nint];
-      }
-    }
-    const int off = stencil_offset(s, m);
-#pragma unroll
-    for (int q = 0; q < RPT; q++) {
-      const int u = neighbour_row(vi[q], off, nint);
-#pragma unroll
-      for (int b = 0; b < 3; b++) {
-        VT pv[RG];
-        load(u, b, pv);
-#pragma unroll
-        for (int r = 0; r < RG; r++) {
-          acc[q][0][r] += kv[q][0 * 3 + b] * pv[r];
-          acc[q][1][r] += kv[q][1 * 3 + b] * pv[r];
-          acc[q][2][r] += kv[q][2 * 3 + b] * pv[r];
-        }
-      }
-    }
-  }
-}
-
-// stencil_rows for the slab variants: the same products in the same order,
-// with two K register sets used in turn (the next point's K is requested
-// into one while the other is applied, two points per loop trip), so no set
-// is copied from one point to the next.
+// The stencil product for RPT rows of one thread at once (rows v[k]; rows with
+// ok[k] false are computed on row 0 and discarded by the caller), for the slab
+// variants: two K register sets used in turn (the next point's K of all RPT
+// rows is requested into one while the other is applied, two points per loop
+// trip), so no set is copied from one point to the next.
 template <typename KT, typename VT, int RPT, typename Load>
 __device__ __forceinline__ void stencil_rows_pp(const KT* __restrict__ Kc, int nint, const int (&v)[RPT],
                                                 const bool (&ok)[RPT], int m, Load load, VT (&acc)[RPT][3][RG]) {
@@ -519,7 +482,7 @@ __device__ __forceinline__ void phase_spmv(const float* __restrict__ K32, const 
   const int tid = threadIdx.x, nth = blockDim.x;
   auto ld = [&](int u, int b, T (&pv)[RG]) {
 #pragma unroll
-    for (int r = 0; r < RG; r++) pv[r] = P[lds_at<T, false>(u, b, r)];
+    for (int r = 0; r < RG; r++) pv[r] = P[lds_at(u, b, r)];
   };
   constexpr int RP = RPT > 0 ? RPT : 1;
   for (int v0 = tid; v0 < nint; v0 += RP * nth) {
@@ -544,7 +507,7 @@ __device__ __forceinline__ void phase_spmv(const float* __restrict__ K32, const 
         for (int r = 0; r < RG; r++) {
           const int64_t e = ((int64_t)vr[q] * 3 + a) * RG + r;
           Q[e] = acc[q][a][r];
-          w[r] += (double)(acc[q][a][r] * P[lds_at<T, false>(vr[q], a, r)]);
+          w[r] += (double)(acc[q][a][r] * P[lds_at(vr[q], a, r)]);
         }
     }
   }
@@ -568,7 +531,7 @@ __device__ __forceinline__ void phase_update(int nint, const T* __restrict__ din
 #pragma unroll
         for (int r = 0; r < RG; r++) {
           const int64_t e = ((int64_t)v * 3 + a) * RG + r;
-          const T pe = P[lds_at<T, false>(v, a, r)];
+          const T pe = P[lds_at(v, a, r)];
           D[e] += alpha[r] * pe;
           const T rv = R[e] - alpha[r] * Q[e];
           R[e] = rv;
@@ -598,7 +561,7 @@ __device__ __forceinline__ void phase_direction(int nint, const T* __restrict__ 
 #pragma unroll
         for (int r = 0; r < RG; r++) {
           if (!((on >> r) & 1)) continue;
-          const int64_t e = ((int64_t)v * 3 + a) * RG + r, ep = lds_at<T, false>(v, a, r);
+          const int64_t e = ((int64_t)v * 3 + a) * RG + r, ep = lds_at(v, a, r);
           P[ep] = dv * R[e] + beta[r] * P[ep];
         }
       }
@@ -650,7 +613,7 @@ __device__ __forceinline__ void k_ring_request(const KT* __restrict__ Kc, int ni
       for (int e = 0; e < 9; e++) ring[p][q][e] = kr.at(q, p, e);
 }
 
-// stencil_rows with the K values of PF stencil points in flight: the ring
+// The same product with the K values of PF stencil points in flight: the ring
 // holds points 0 .. PF-1 on entry (k_ring_request, or the previous call),
 // and point (s + PF) mod 15 is requested right after point s is applied,
 // into the slot point s used (PF x RPT x 9 registers).  The ring thus wraps:
@@ -659,7 +622,7 @@ __device__ __forceinline__ void k_ring_request(const KT* __restrict__ Kc, int ni
 // point loop is unrolled, so the ring is indexed statically and needs no
 // copies.  A wave then waits for a K load once per PF points instead of
 // once per point; PF x RPT x 9 stays below the 63 vector loads a wave can
-// have outstanding.  Same arithmetic, in the same order, as stencil_rows.
+// have outstanding.  Same arithmetic, in the same order, as stencil_rows_pp.
 template <typename KT, typename VT, int RPT, int PF, typename Load>
 __device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int nint, const int (&v)[RPT],
                                                 const bool (&ok)[RPT], int m, Load load, KT (&ring)[PF][RPT][9],
@@ -713,13 +676,11 @@ __device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int n
 // reads the neighbours' entries).  Rows at or beyond nint (ok false) carry
 // values that are never used.
 template <typename T, int RPT, int PF>
-__device__ __forceinline__ void phase_spmv_reg(const float* __restrict__ K32, const double* __restrict__ K64, int nint,
-                                               int m, const T* P, T (&ring)[PF][RPT][9], T (&Qr)[RPT][3][RG],
+__device__ __forceinline__ void phase_spmv_reg(const T* __restrict__ K, int nint, int m, const T* P, T (&ring)[PF][RPT][9], T (&Qr)[RPT][3][RG],
                                                double (&w)[RG]) {
-  constexpr bool fp64 = std::is_same<T, double>::value;
   auto ld = [&](int u, int b, T (&pv)[RG]) {
 #pragma unroll
-    for (int r = 0; r < RG; r++) pv[r] = P[lds_at<T, true>(u, b, r)];
+    for (int r = 0; r < RG; r++) pv[r] = P[lds_at(u, b, r)];
   };
   int vr[RPT];
   bool ok[RPT];
@@ -728,10 +689,7 @@ __device__ __forceinline__ void phase_spmv_reg(const float* __restrict__ K32, co
     vr[q] = threadIdx.x + q * blockDim.x;
     ok[q] = vr[q] < nint;
   }
-  if constexpr (fp64)
-    stencil_rows_pf<double, double, RPT, PF>(K64, nint, vr, ok, m, ld, ring, Qr);
-  else
-    stencil_rows_pf<float, float, RPT, PF>(K32, nint, vr, ok, m, ld, ring, Qr);
+  stencil_rows_pf<T, T, RPT, PF>(K, nint, vr, ok, m, ld, ring, Qr);
   // the row's three components are summed in T before the FP64 partial
   // (one conversion and FP64 add per right-hand side instead of three)
 #pragma unroll
@@ -741,16 +699,16 @@ __device__ __forceinline__ void phase_spmv_reg(const float* __restrict__ K32, co
     for (int r = 0; r < RG; r++) {
       T t = 0;
 #pragma unroll
-      for (int a = 0; a < 3; a++) t += Qr[q][a][r] * P[lds_at<T, true>(vr[q], a, r)];
+      for (int a = 0; a < 3; a++) t += Qr[q][a][r] * P[lds_at(vr[q], a, r)];
       w[r] += (double)t;
     }
   }
 }
 
-template <typename T, int RPT, bool DLDS>
+template <typename T, int RPT>
 __device__ __forceinline__ void phase_update_reg(int nint, const T (&dv)[RPT][3], const T* P, const T (&Qr)[RPT][3][RG],
-                                                 T (&Rr)[RPT][3][RG], T* DL, T (&Dr)[RPT][3][RG],
-                                                 const T (&alpha)[RG], double (&w)[2 * RG]) {
+                                                 T (&Rr)[RPT][3][RG], T* DL, const T (&alpha)[RG],
+                                                 double (&w)[2 * RG]) {
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
     const int v = threadIdx.x + q * blockDim.x;
@@ -762,11 +720,8 @@ __device__ __forceinline__ void phase_update_reg(int nint, const T (&dv)[RPT][3]
     for (int a = 0; a < 3; a++)
 #pragma unroll
       for (int r = 0; r < RG; r++) {
-        const T pe = P[lds_at<T, true>(v, a, r)];
-        if constexpr (DLDS)
-          DL[lds_at<T, true>(v, a, r)] += alpha[r] * pe;
-        else
-          Dr[q][a][r] += alpha[r] * pe;
+        const T pe = P[lds_at(v, a, r)];
+        DL[lds_at(v, a, r)] += alpha[r] * pe;
         const T rv = Rr[q][a][r] - alpha[r] * Qr[q][a][r];
         Rr[q][a][r] = rv;
         const T z = dv[q][a] * rv;
@@ -793,7 +748,7 @@ __device__ __forceinline__ void phase_direction_reg(int nint, const T (&dv)[RPT]
 #pragma unroll
       for (int r = 0; r < RG; r++) {
         if (!((on >> r) & 1)) continue;
-        const int64_t e = lds_at<T, true>(v, a, r);
+        const int64_t e = lds_at(v, a, r);
         P[e] = dv[q][a] * Rr[q][a][r] + beta[r] * P[e];
       }
   }
@@ -966,20 +921,15 @@ void k_batch_solve(SolveArgs A) {
   T* D = REG ? nullptr : R + A.scr_stride;  // inner correction
   T* Q = REG ? nullptr : D + A.scr_stride;  // A p
   constexpr int RQ = REG ? RPT : 1;
+  static_assert(!REG || fp64, "the register-resident form is FP64");
   T Rr[RQ][3][RG], Qr[RQ][3][RG], dvr[RQ][3];
   // REG: the inner correction d of the owned rows, in LDS behind p (each
-  // thread touches only its own rows' entries) or in registers
-  constexpr bool kDInLds = REG && d_in_lds(fp64, RPT);
-  T Dr[RQ][3][RG];  // unused (and removed) when d is in LDS
-  T* DL = kDInLds ? P + (int64_t)A.max_nint * lds_row<T, REG>() : nullptr;
-  // REG with stage_x: the FP64 iterate of the task's rows for the residual
-  // pass, in the FP64 d region (free during that pass) or behind p
-  double* XS = !REG ? nullptr
-                    : (kDInLds && fp64) ? reinterpret_cast<double*>(DL)
-                                        : reinterpret_cast<double*>(P + (int64_t)A.max_nint * lds_row<T, REG>() *
-                                                                            (kDInLds ? 2 : 1));
+  // thread touches only its own rows' entries); during the residual pass the
+  // same region stages the iterate
+  T* DL = REG ? P + (int64_t)A.max_nint * kLdsRow : nullptr;
+  double* XS = reinterpret_cast<double*>(DL);
   // stencil points whose K values are in flight in the register forms
-  constexpr int kPrefetch = fp64 ? 1 : 3;
+  constexpr int kPrefetch = 1;
 
   int tried = 0;  // queues found empty (thread 0)
   const int home = blockIdx.x % NQ;
@@ -1011,9 +961,9 @@ void k_batch_solve(SolveArgs A) {
     if (task < 0) break;
     const int cell = __builtin_amdgcn_readfirstlane(A.task_cell[task]);
     const int grp = __builtin_amdgcn_readfirstlane(A.task_group[task]);
-    const Cell C = A.cells[cell];
+    const Cell C = uniform_cell(A.cells, cell);
     const int n = C.n, m = n - 1, nint = C.nint;
-    const float* K32 = A.K32 + C.int0 * (NS * 9);
+    const float* K32 = A.K32 + C.kt0;
     const double* K64 = A.K64 + C.int0 * (NS * 9);
     const double* b64 = A.b64 + C.int0 * (3 * NB);
     double* x64 = A.x64 + C.int0 * (3 * NB);
@@ -1087,25 +1037,22 @@ void k_batch_solve(SolveArgs A) {
           for (int r = 0; r < RG; r++) pv[r] = x64[(int64_t)u * 3 * NB + b * NB + q0 + r];
         };
         if constexpr (REG) {
-          // when the launch has room for it, the task's FP64 iterate is
-          // staged in LDS (own rows, one barrier), so the stencil reads its
-          // neighbours' values from there instead of from global memory
-          if (A.stage_x) {
+          // the task's FP64 iterate is staged in LDS (own rows, one barrier),
+          // so the stencil reads its neighbours' values from there instead
+          // of from global memory
 #pragma unroll
-            for (int q = 0; q < RQ; q++) {
-              const int v = tid + q * nth;
-              if (v >= nint) continue;
+          for (int q = 0; q < RQ; q++) {
+            const int v = tid + q * nth;
+            if (v >= nint) continue;
 #pragma unroll
-              for (int a = 0; a < 3; a++)
+            for (int a = 0; a < 3; a++)
 #pragma unroll
-                for (int r = 0; r < RG; r++)
-                  XS[lds_at<double, true>(v, a, r)] = x64[(int64_t)v * 3 * NB + a * NB + q0 + r];
-            }
-            __syncthreads();
+              for (int r = 0; r < RG; r++) XS[lds_at(v, a, r)] = x64[(int64_t)v * 3 * NB + a * NB + q0 + r];
           }
+          __syncthreads();
           auto lds_ld = [&](int u, int b, double (&pv)[RG]) {
 #pragma unroll
-            for (int r = 0; r < RG; r++) pv[r] = XS[lds_at<double, true>(u, b, r)];
+            for (int r = 0; r < RG; r++) pv[r] = XS[lds_at(u, b, r)];
           };
           // one owned row at a time (the accumulators are FP64)
 #pragma unroll
@@ -1113,13 +1060,10 @@ void k_batch_solve(SolveArgs A) {
             const int vr[1] = {tid + q * nth};
             const bool ok[1] = {vr[0] < nint};
             double acc[1][3][RG];
-            if (A.stage_x) {
-              // unrolled, with the next point's K in flight
-              double kr1[1][1][9];
-              k_ring_request<double, 1, 1>(K64, nint, vr, ok, kr1);
-              stencil_rows_pf<double, double, 1, 1>(K64, nint, vr, ok, m, lds_ld, kr1, acc);
-            } else
-              stencil_rows<double, double, 1>(K64, nint, vr, ok, m, ld, acc);
+            // unrolled, with the next point's K in flight
+            double kr1[1][1][9];
+            k_ring_request<double, 1, 1>(K64, nint, vr, ok, kr1);
+            stencil_rows_pf<double, double, 1, 1>(K64, nint, vr, ok, m, lds_ld, kr1, acc);
             if (!ok[0]) continue;
 #pragma unroll
             for (int a = 0; a < 3; a++)
@@ -1286,10 +1230,7 @@ void k_batch_solve(SolveArgs A) {
               for (int r = 0; r < RG; r++) {
                 const T rv = ((live >> r) & 1) ? (T)((double)Rr[q][a][r] * (double)inv[r]) : (T)0;
                 Rr[q][a][r] = rv;
-                if constexpr (kDInLds)
-                  DL[lds_at<T, true>(tid + q * nth, a, r)] = 0;
-                else
-                  Dr[q][a][r] = 0;
+                DL[lds_at(tid + q * nth, a, r)] = 0;
                 const T z = dvr[q][a] * rv;
                 w[r] += (double)(rv * z);
                 w[RG + r] += (double)(rv * rv);
@@ -1334,7 +1275,7 @@ void k_batch_solve(SolveArgs A) {
             for (int a = 0; a < 3; a++)
 #pragma unroll
               for (int r = 0; r < RG; r++) {
-                const int64_t e = lds_at<T, true>(v, a, r);
+                const int64_t e = lds_at(v, a, r);
                 const T z = dvr[q][a] * Rr[q][a][r];
                 P[e] = beta[r] != (T)0 ? z + beta[r] * P[e] : z;
               }
@@ -1345,7 +1286,7 @@ void k_batch_solve(SolveArgs A) {
             const T dv = dinv[v * 3 + a];
 #pragma unroll
             for (int r = 0; r < RG; r++) {
-              const int64_t e = ((int64_t)v * 3 + a) * RG + r, ep = lds_at<T, false>(v, a, r);
+              const int64_t e = ((int64_t)v * 3 + a) * RG + r, ep = lds_at(v, a, r);
               const T z = dv * R[e];
               P[ep] = beta[r] != (T)0 ? z + beta[r] * P[ep] : z;
             }
@@ -1367,10 +1308,7 @@ void k_batch_solve(SolveArgs A) {
             vr[q] = tid + q * nth;
             ok[q] = vr[q] < nint;
           }
-          if constexpr (fp64)
-            k_ring_request<double, RQ, kPrefetch>(K64, nint, vr, ok, kring);
-          else
-            k_ring_request<float, RQ, kPrefetch>(K32, nint, vr, ok, kring);
+          if constexpr (fp64) k_ring_request<double, RQ, kPrefetch>(K64, nint, vr, ok, kring);
         }
       }
       if (act && inner_cap > 0) do {
@@ -1381,7 +1319,7 @@ void k_batch_solve(SolveArgs A) {
 #pragma unroll
           for (int r = 0; r < RG; r++) w[r] = 0;
           if constexpr (REG)
-            phase_spmv_reg<T, RQ, kPrefetch>(K32, K64, nint, m, P, kring, Qr, w);
+            phase_spmv_reg<T, RQ, kPrefetch>(K64, nint, m, P, kring, Qr, w);
           else
             phase_spmv<T, RPT>(K32, K64, nint, m, P, Q, w);
           // alpha of right-hand side r computed in lane r, then broadcast
@@ -1402,7 +1340,7 @@ void k_batch_solve(SolveArgs A) {
 #pragma unroll
           for (int r = 0; r < 2 * RG; r++) w[r] = 0;
           if constexpr (REG)
-            phase_update_reg<T, RQ, kDInLds>(nint, dvr, P, Qr, Rr, DL, Dr, alpha, w);
+            phase_update_reg<T, RQ>(nint, dvr, P, Qr, Rr, DL, alpha, w);
           else
             phase_update<T, RPT>(nint, dinv, P, Q, R, D, alpha, w);
           // lane r < RG decides right-hand side r from its r.z (lane r) and
@@ -1476,7 +1414,7 @@ void k_batch_solve(SolveArgs A) {
             for (int r = 0; r < RG; r++)
               if (((live >> r) & 1) && !((capfail >> r) & 1) && !S.failed[r])
                 x64[(int64_t)v * 3 * NB + a * NB + q0 + r] +=
-                    S.scale[r] * (double)(kDInLds ? DL[lds_at<T, true>(v, a, r)] : Dr[q][a][r]);
+                    S.scale[r] * (double)DL[lds_at(v, a, r)];
         }
       } else
       for (int v = tid; v < nint; v += nth)
@@ -1502,21 +1440,14 @@ void k_batch_solve(SolveArgs A) {
       A.iters[cell * NB + q0 + r] = S.it[r];
       A.relres[cell * NB + q0 + r] = sqrt(S.rr64[r] / S.bb[r]);
       if (!(S.rr64[r] <= A.tol * A.tol * S.bb[r])) A.flags[cell * NB + q0 + r] |= 1;
-      if (S.failed[r]) A.flags[cell * NB + q0 + r] |= A.fb_count ? (4 | 8) : 4;
+      if (S.failed[r]) A.flags[cell * NB + q0 + r] |= 4;
       if (S.retried[r]) A.flags[cell * NB + q0 + r] |= 16;
-    }
-    if (A.fb_count && tid == 0) {
-      bool any = false;
-      for (int r = 0; r < RG; r++) any |= S.failed[r] != 0;
-      if (any) {
-        const int slot = __hip_atomic_fetch_add(A.fb_count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        A.fb_cell[slot] = cell;
-        A.fb_group[slot] = grp;
-      }
     }
     __syncthreads();
   }
 }
+
+#include "batch_mfma.hpp"
 
 __global__ void k_batch_reset(unsigned* queue, int* flags, int nflags, int* fb_count) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2051,6 +1982,9 @@ struct mfs_batch_s {
   int max_n = 0, max_nint = 0;
   int ntasks = 0;
   int seg[NQ + 1] = {};  // task ranges of the per-XCD queues
+  bool tiled = false;    // every cell has n <= 10: mixed precision runs the matrix-core kernel
+  int mseg[NQ + 1] = {};  // its task ranges
+  int64_t k32_total = 0;  // FP32 matrix values
   bool assembled = false;
   int tuned_wg[2] = {0, 0}, tuned_per_cu[2] = {0, 0};  // per precision (0 mixed, 1 FP64)
   int tuned_var[2] = {-1, -1};                        // kernel variant (rows per thread)
@@ -2078,6 +2012,8 @@ struct mfs_batch_s {
   int* d_flags = nullptr;
   int* d_task_cell = nullptr;
   int* d_task_group = nullptr;
+  int* d_mtask_cell = nullptr;  // tasks of the matrix-core kernel
+  int* d_mtask_group = nullptr;
   int* d_fb = nullptr;  // FP64 pass task list: count, cells[ntasks], groups[ntasks]
   unsigned* d_queue = nullptr;
   void* d_scr = nullptr;
@@ -2096,7 +2032,7 @@ static int batch_free(mfs_batch B) {
   if (B->ctx) (void)hipStreamSynchronize(B->ctx->stream);
   void* ptrs[] = {B->d_cells, B->d_int0, B->d_tmpls, B->d_gptr, B->d_gent, B->d_E, B->d_K32, B->d_K64,
                   B->d_dinv32, B->d_dinv64, B->d_b64, B->d_x64, B->d_iters, B->d_relres, B->d_flags,
-                  B->d_task_cell, B->d_task_group, B->d_fb, B->d_queue, B->d_scr, B->d_et, B->d_ft, B->d_face_order,
+                  B->d_task_cell, B->d_task_group, B->d_mtask_cell, B->d_mtask_group, B->d_fb, B->d_queue, B->d_scr, B->d_et, B->d_ft, B->d_face_order,
                   B->d_fstats, B->d_hat, B->d_report};
   for (void* p : ptrs) dfree(p);
   mfs_ctx c = B->ctx;
@@ -2202,10 +2138,13 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   }
   B->total_tets = t0;
   B->total_int = i0;
+  B->tiled = B->max_n <= kMfmaMaxN;
+  for (Cell& C : B->cells) {
+    C.kt0 = B->k32_total;
+    B->k32_total += B->tiled ? k32_tile_floats(C.nint) : (int64_t)NS * 9 * C.nint;
+  }
   B->et_total = e0;
   B->ft_total = f0;
-  for (int c = 0; c < d->n_cells; c++)
-    if (!(d->E[c] > 0) && false) break;
   // tasks: 3 per cell, largest cells first (stable by cell id)
   std::vector<int> order(d->n_cells);
   std::iota(order.begin(), order.end(), 0);
@@ -2223,6 +2162,18 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   }
   B->seg[NQ] = (int)tc.size();
   B->ntasks = (int)tc.size();
+  std::vector<int> mc, mg;
+  if (B->tiled) {
+    for (int q = 0; q < NQ; q++) {
+      B->mseg[q] = (int)mc.size();
+      for (size_t i = q; i < order.size(); i += NQ)
+        for (int g = 0; g < NB / mfma_task_rhs(B->cells[order[i]].nint); g++) {
+          mc.push_back(order[i]);
+          mg.push_back(g);
+        }
+    }
+    B->mseg[NQ] = (int)mc.size();
+  }
   int st = MFS_OK;
   auto alloc = [&](void** p, size_t bytes) {
     if (st == MFS_OK) st = dmalloc(p, bytes);
@@ -2233,7 +2184,7 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   alloc((void**)&B->d_gptr, sizeof(int64_t) * gptr_all.size());
   alloc((void**)&B->d_gent, sizeof(uint32_t) * std::max<size_t>(1, gent_all.size()));
   alloc((void**)&B->d_E, sizeof(double) * t0);
-  alloc((void**)&B->d_K32, sizeof(float) * NS * 9 * i0);
+  alloc((void**)&B->d_K32, sizeof(float) * B->k32_total);
   alloc((void**)&B->d_K64, sizeof(double) * NS * 9 * i0);
   alloc((void**)&B->d_dinv32, sizeof(float) * 3 * i0);
   alloc((void**)&B->d_dinv64, sizeof(double) * 3 * i0);
@@ -2244,6 +2195,10 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   alloc((void**)&B->d_flags, sizeof(int) * NB * d->n_cells);
   alloc((void**)&B->d_task_cell, sizeof(int) * B->ntasks);
   alloc((void**)&B->d_task_group, sizeof(int) * B->ntasks);
+  if (B->tiled) {
+    alloc((void**)&B->d_mtask_cell, sizeof(int) * mc.size());
+    alloc((void**)&B->d_mtask_group, sizeof(int) * mc.size());
+  }
   alloc((void**)&B->d_fb, sizeof(int) * (1 + 2 * (size_t)B->ntasks));
   alloc((void**)&B->d_queue, sizeof(unsigned) * NQ * QSTRIDE);
   alloc((void**)&B->d_report, sizeof(unsigned long long) * 6);
@@ -2267,6 +2222,10 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   MFS_HIP(hipMemcpyAsync(B->d_E, d->E, sizeof(double) * t0, hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemcpyAsync(B->d_task_cell, tc.data(), sizeof(int) * B->ntasks, hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemcpyAsync(B->d_task_group, tg.data(), sizeof(int) * B->ntasks, hipMemcpyHostToDevice, s));
+  if (B->tiled) {
+    MFS_HIP(hipMemcpyAsync(B->d_mtask_cell, mc.data(), sizeof(int) * mc.size(), hipMemcpyHostToDevice, s));
+    MFS_HIP(hipMemcpyAsync(B->d_mtask_group, mg.data(), sizeof(int) * mg.size(), hipMemcpyHostToDevice, s));
+  }
   if (B->d_face_order)
     MFS_HIP(hipMemcpyAsync(B->d_face_order, order.data(), sizeof(int) * d->n_cells, hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemsetAsync(B->d_x64, 0, sizeof(double) * 3 * NB * i0, s));
@@ -2318,7 +2277,7 @@ extern "C" int mfs_batch_assemble(mfs_batch B) {
   }
   const unsigned grid = (unsigned)std::min<int64_t>(65536, (B->total_int + 255) / 256);
   k_cell_assemble<<<grid, 256, 0, s>>>(B->d_cells, B->ncells, B->d_int0, B->d_tmpls, B->d_gptr, B->d_gent, B->d_E,
-                                       B->nu, B->h, B->conv, B->d_ft, B->total_int, B->d_K32, B->d_K64,
+                                       B->nu, B->h, B->conv, B->d_ft, B->total_int, B->tiled ? 1 : 0, B->d_K32, B->d_K64,
                                        B->d_dinv32, B->d_dinv64, B->d_b64);
   MFS_HIP(hipGetLastError());
   MFS_HIP(hipStreamSynchronize(s));
@@ -2369,36 +2328,29 @@ static void boundary_functions(const mfs_batch_s* B, const std::vector<double>& 
       }
 }
 
-// p, and for the register-resident variants also d, per workgroup
+// Dynamic LDS of k_batch_solve: p, and for the register-resident variants
+// also d (where the residual pass stages the FP64 iterate).
 static size_t lds_bytes(mfs_batch B, int prec, int var) {
-  const int rpt = prec == MFS_PREC_F64 ? kRptF64[var] : kRptF32[var];
-  const bool dl = kRegVar[var] && d_in_lds(prec == MFS_PREC_F64, rpt);
-  const int row = prec == MFS_PREC_F64 ? (kRegVar[var] ? lds_row<double, true>() : lds_row<double, false>())
-                                        : (kRegVar[var] ? lds_row<float, true>() : lds_row<float, false>());
-  return (size_t)B->max_nint * row * (prec == MFS_PREC_F64 ? 8 : 4) * (dl ? 2 : 1);
+  return (size_t)B->max_nint * kLdsRow * (prec == MFS_PREC_F64 ? 8 : 4) * (kRegVar[var] ? 2 : 1);
 }
-
-// The residual pass of the register variants stages the task's FP64 iterate
-// in LDS: FP64 in the d region (free during that pass), FP32 one row per
-// thread (already one workgroup per CU) in a region behind p, when it fits.
-static size_t stage_x_extra(mfs_batch B, int prec, int var) {
-  if (!kRegVar[var] || prec == MFS_PREC_F64) return 0;
-  return (size_t)B->max_nint * lds_row<double, true>() * 8;
+// ... and of the matrix-core kernel: p and the inverse diagonal of the
+// largest task
+static size_t mfma_lds_bytes(mfs_batch B) {
+  size_t need = 0;
+  for (int n = 2; n <= B->max_n; n++) {
+    const int nint = (n - 1) * (n - 1) * (n - 1);
+    need = std::max(need, sizeof(float) * (size_t)nint * 3 * (mfma_task_rhs(nint) + 1 + 4 * mfma_d_lds(mfma_task_rhs(nint))));
+  }
+  return need;
 }
-static bool stage_x(mfs_batch B, int prec, int var) {
-  if (!kRegVar[var]) return false;
-  if (prec != MFS_PREC_F64 && kRptF32[var] != 1) return false;
-  return lds_bytes(B, prec, var) + stage_x_extra(B, prec, var) <= 160 * 1024 - 8192;
-}
-static size_t launch_lds(mfs_batch B, int prec, int var) {
-  return lds_bytes(B, prec, var) + (stage_x(B, prec, var) ? stage_x_extra(B, prec, var) : 0);
-}
+static bool use_mfma(mfs_batch B, int prec) { return prec == MFS_PREC_MIXED && B->tiled; }
 
 // Per-workgroup scratch for a launch shape; must run before any capture.
 static int batch_scratch(mfs_batch B, int precision, int per_cu, int var) {
   const int grid = B->ctx->cu_count * per_cu;
   const int64_t stride = (int64_t)B->max_nint * 3 * RG;
-  const size_t need = kRegVar[var] ? 0 : (size_t)grid * 3 * stride * (precision == MFS_PREC_F64 ? 8 : 4);
+  const size_t need =
+      kRegVar[var] || use_mfma(B, precision) ? 0 : (size_t)grid * 3 * stride * (precision == MFS_PREC_F64 ? 8 : 4);
   if (need > B->scr_bytes) {
     MFS_HIP(hipStreamSynchronize(B->ctx->stream));
     dfree(B->d_scr);
@@ -2412,7 +2364,15 @@ static int batch_scratch(mfs_batch B, int precision, int per_cu, int var) {
 
 // Launch reset + persistent solve on the context stream (capturable: no
 // allocation, no memset; the queue and flags are cleared by a kernel).
-static const void* batch_kernel(int precision, int var) {
+static const void* batch_kernel(mfs_batch B, int precision, int var) {
+  if (use_mfma(B, precision)) {
+    switch (mfma_class(B->max_nint)) {
+      case 0: return (const void*)k_batch_solve_mfma<0>;
+      case 1: return (const void*)k_batch_solve_mfma<1>;
+      case 2: return (const void*)k_batch_solve_mfma<2>;
+      default: return (const void*)k_batch_solve_mfma<3>;
+    }
+  }
   if (precision == MFS_PREC_F64) {
     switch (var) {
       case 0: return (const void*)k_batch_solve<double, kRptF64[0], kRegVar[0]>;
@@ -2421,12 +2381,15 @@ static const void* batch_kernel(int precision, int var) {
       default: return (const void*)k_batch_solve<double, kRptF64[3], kRegVar[3]>;
     }
   }
-  switch (var) {
-    case 0: return (const void*)k_batch_solve<float, kRptF32[0], kRegVar[0]>;
-    case 1: return (const void*)k_batch_solve<float, kRptF32[1], kRegVar[1]>;
-    case 2: return (const void*)k_batch_solve<float, kRptF32[2], kRegVar[2]>;
-    default: return (const void*)k_batch_solve<float, kRptF32[3], kRegVar[3]>;
-  }
+  return var == 0 ? (const void*)k_batch_solve<float, kRptF32[0], false>
+                  : (const void*)k_batch_solve<float, kRptF32[1], false>;
+}
+// Threads and dynamic LDS of a launch (the matrix-core kernel's are its own).
+static int launch_threads(mfs_batch B, int precision, int wg) {
+  return use_mfma(B, precision) ? 64 * mfma_waves(mfma_class(B->max_nint)) : wg;
+}
+static size_t launch_lds(mfs_batch B, int precision, int var) {
+  return use_mfma(B, precision) ? mfma_lds_bytes(B) : lds_bytes(B, precision, var);
 }
 
 // A variant takes workgroups up to its thread bound; the register-resident
@@ -2452,7 +2415,8 @@ static int batch_launch(mfs_batch B, const mfs_batch_solve_desc* d, int wg, int 
     return MFS_ERR_ARG;
   }
   const size_t lds = launch_lds(B, d->precision, var);
-  const size_t need = kRegVar[var] ? 0 : (size_t)grid * 3 * stride * (d->precision == MFS_PREC_F64 ? 8 : 4);
+  const bool mfma = use_mfma(B, d->precision);
+  const size_t need = kRegVar[var] || mfma ? 0 : (size_t)grid * 3 * stride * (d->precision == MFS_PREC_F64 ? 8 : 4);
   if (need > B->scr_bytes) {
     set_error("mfs_batch_solve: scratch not allocated for this launch shape");
     return MFS_ERR_ARG;
@@ -2464,12 +2428,13 @@ static int batch_launch(mfs_batch B, const mfs_batch_solve_desc* d, int wg, int 
   }
   SolveArgs A;
   A.cells = B->d_cells;
-  A.task_cell = fb ? B->d_fb + 1 : B->d_task_cell;
-  A.task_group = fb ? B->d_fb + 1 + B->ntasks : B->d_task_group;
+  A.task_cell = fb ? B->d_fb + 1 : mfma ? B->d_mtask_cell : B->d_task_cell;
+  A.task_group = fb ? B->d_fb + 1 + B->ntasks : mfma ? B->d_mtask_group : B->d_task_group;
   A.ntasks = B->ntasks;
   // MFS_ONE_QUEUE=1 keeps the cell-size order in a single queue (A/B runs)
   static const bool one_queue = std::getenv("MFS_ONE_QUEUE") && std::getenv("MFS_ONE_QUEUE")[0] == '1';
-  for (int q = 0; q <= NQ; q++) A.seg[q] = one_queue ? (q == 0 ? 0 : B->ntasks) : B->seg[q];
+  const int* seg = mfma ? B->mseg : B->seg;
+  for (int q = 0; q <= NQ; q++) A.seg[q] = one_queue ? (q == 0 ? 0 : seg[NQ]) : seg[q];
   A.queue = B->d_queue;
   A.K32 = B->d_K32;
   A.K64 = B->d_K64;
@@ -2481,14 +2446,11 @@ static int batch_launch(mfs_batch B, const mfs_batch_solve_desc* d, int wg, int 
   A.scr64 = (double*)B->d_scr;
   A.scr_stride = stride;
   A.max_nint = B->max_nint;
-  A.stage_x = stage_x(B, d->precision, var) ? 1 : 0;
   A.iters = B->d_iters;
   A.relres = B->d_relres;
   A.flags = B->d_flags;
   const bool list_failures = pass == BL_MAIN_LIST && d->precision == MFS_PREC_MIXED;
-  A.fb_count = list_failures ? B->d_fb : nullptr;
-  A.fb_cell = list_failures ? B->d_fb + 1 : nullptr;
-  A.fb_group = list_failures ? B->d_fb + 1 + B->ntasks : nullptr;
+  A.list_failures = list_failures ? 1 : 0;
   A.ntasks_dev = fb ? B->d_fb : nullptr;
   A.tol = d->tol;
   A.inner_tol = d->inner_tol > 0 ? d->inner_tol : 1e-4;
@@ -2500,7 +2462,14 @@ static int batch_launch(mfs_batch B, const mfs_batch_solve_desc* d, int wg, int 
   k_batch_reset<<<std::max(1, (B->ncells * NB + 255) / 256), 256, 0, s>>>(
       B->d_queue, B->d_flags, fb ? 0 : B->ncells * NB, list_failures ? B->d_fb : nullptr);
   void* args[] = {&A};
-  MFS_HIP(hipLaunchKernel(batch_kernel(d->precision, var), dim3(grid), dim3(wg), args, lds, s));
+  MFS_HIP(hipLaunchKernel(batch_kernel(B, d->precision, var), dim3(grid), dim3(launch_threads(B, d->precision, wg)), args,
+                          lds, s));
+  if (list_failures) {
+    const int ngroups = B->ncells * (NB / RG);
+    k_list_failures<<<(ngroups + 255) / 256, 256, 0, s>>>(B->d_flags, ngroups, B->d_fb, B->d_fb + 1,
+                                                          B->d_fb + 1 + B->ntasks);
+    MFS_HIP(hipGetLastError());
+  }
   return MFS_OK;
 }
 
@@ -2528,7 +2497,8 @@ static int batch_check_desc(mfs_batch B, const mfs_batch_solve_desc* d) {
 // least 1.
 static int resident_per_cu(mfs_batch B, int precision, int wg, int var) {
   const size_t lds = launch_lds(B, precision, var);
-  const void* fn = batch_kernel(precision, var);
+  const void* fn = batch_kernel(B, precision, var);
+  wg = launch_threads(B, precision, wg);
   (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, wg, lds) != hipSuccess) nb = 1;
@@ -2705,6 +2675,8 @@ extern "C" int mfs_batch_autotune(mfs_batch B, const mfs_batch_solve_desc* d, in
   for (int var = 0; var < kVariants[t]; var++)
   for (int wg : {64, 128, 192, 256, 320, 384, 448, 512}) {
     if (!variant_fits(B, d->precision, var, wg)) continue;
+    // the matrix-core kernel has one shape, whatever variant is asked for
+    if (use_mfma(B, d->precision) && !(var == 0 && wg == 256)) continue;
     const int res = resident_per_cu(B, d->precision, wg, var);
     for (int pc : {res, res - 1}) {
       if (pc < 1 || (pc == res - 1 && res == 1)) continue;

@@ -270,8 +270,6 @@ __device__ void tet_grads(const int (&ijk)[4][3], double hf, double (&g)[4][3], 
   V = fabs(det) / 6.0;
 }
 
-// Step index of axis a in the tet's axis order (xyz,xzy,yxz,yzx,zxy,zyx).
-__device__ constexpr int kStepOf[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {2, 0, 1}, {1, 2, 0}, {2, 1, 0}};
 
 // Elastic block (I=i, J=j) of a tet: textbook V(lam dI_a dJ_b + mu dI_b dJ_a +
 // mu delta dI.dJ); the reference convention is its transpose.
@@ -1456,8 +1454,8 @@ __global__ void k_batch_reset(unsigned* queue, int* flags, int nflags, int* fb_c
   for (int i = t; i < nflags; i += gridDim.x * blockDim.x) flags[i] = 0;
 }
 
-// Coarse Galerkin matrices Kc = Phi^T K Phi (24x24 per cell), FP64, by an
-// element loop: one workgroup per cell, tets processed one at a time.
+// Coarse Galerkin matrices Kc = Phi^T K Phi (24x24 per cell), FP64, one
+// workgroup of 4 waves per cell.
 // form MFS_BASIS_COMPONENTWISE: the coarse functions are Psi_{c,a} =
 // e_a (sum_d phi_{c,d})_a (the reference's use of one vector basis per
 // coarse node, component by component) and the coarse element is the
@@ -1465,138 +1463,146 @@ __global__ void k_batch_reset(unsigned* queue, int* flags, int nflags, int* fb_c
 // (MsFEM_Grid.h:3837-3975), integrated exactly over the fine tets: the
 // textbook Galerkin product, blockwise transposed in the reference
 // convention.
-__global__ __launch_bounds__(256) void k_galerkin(const Cell* __restrict__ cells, const double* __restrict__ E,
-                                                  double nu, double h, int conv, const double* __restrict__ x64,
-                                                  const double* __restrict__ ft, int form,
-                                                  double* __restrict__ Kc) {
-  // GT tets per round: three barriers per round instead of per tet
-  constexpr int GT = 8;
-  __shared__ double phi[GT][12][NB];  // element values of the 24 bases
-  __shared__ double KeS[6][12][12];   // unit-modulus element matrix of each of the 6 tet shapes
-  __shared__ double KP[GT][12][NB];
-  __shared__ double Eg[GT];
-  __shared__ int Pg[GT];
-  const int cell = blockIdx.x, tid = threadIdx.x;
-  const Cell C = cells[cell];
-  const int n = C.n, m = n - 1;
-  const double hf = h / n;
+//
+// On a tet the gradient of a P1 function is its difference along the tet's
+// three axis-parallel edges, G[a][b] = d_b u_a, and the element form is
+//   u^T Ke w = sum_ab Gu[a][b] H[a][b],
+//   H[a][b] = mu Gw[a][b] + X Gw[b][a] + delta_ab Y tr Gw,
+// (X, Y) = (mu, lambda) in the textbook convention, (lambda, mu) in the
+// reference's.  Both are symmetric, so Kc is a sum of rank-1 terms over 9
+// gradient entries per tet: a contraction for v_mfma_f64_16x16x4.  A lane
+// owns one hex (of 4, the instruction's k) and columns l % 16 and
+// 16 + l % 8: it loads the hex's 8 nodes, forms G and H of the 6 tets in
+// registers and feeds them as A and B operands, with no LDS and no barrier
+// in the loop.  The three upper tiles (columns 0-15 x 0-15, 0-15 x 16-23,
+// 16-23 x 16-23) hold the symmetric result.
+//
+// Bound by FP64 MFMA issue (27 instructions of 64 cycles per 4 tets; the
+// last two tiles use half their columns).  4,096 cells of 8^3: 4.1 ms, 16^3
+// cells of n = 6..10: 5.4 ms; an element loop through LDS with three barriers
+// per 8 tets took 20.0 and 26.0 ms.
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+
+// The value (3 components) of coarse function q at fine node (i, j, k).
+__device__ __forceinline__ void coarse_function_at(const double* __restrict__ xc, const double* __restrict__ ftc, int n,
+                                                   double rn, int form, int i, int j, int k, int q, double (&v)[3]) {
+  const int m = n - 1, c = q / 3, d = q - 3 * c;
+  const bool comp = form == MFS_BASIS_COMPONENTWISE;
+  if (i >= 1 && i <= m && j >= 1 && j <= m && k >= 1 && k <= m) {
+    const double* x = xc + (unsigned)(interior_index(i, j, k, m) * 3 * NB);
+    if (!comp) {
+#pragma unroll
+      for (int a = 0; a < 3; a++) v[a] = x[a * NB + q];
+    } else {
+      const double* xd = x + d * NB + 3 * c;
+      const double sum = xd[0] + xd[1] + xd[2];
+#pragma unroll
+      for (int a = 0; a < 3; a++) v[a] = a == d ? sum : 0.0;
+    }
+  } else if (ftc) {
+    face_trace_at(ftc, n, i, j, k, q, v);
+    if (comp) {
+      double sum = 0.0;
+      for (int dd = 0; dd < 3; dd++) {
+        double g[3];
+        face_trace_at(ftc, n, i, j, k, 3 * c + dd, g);
+        sum += d == 0 ? g[0] : d == 1 ? g[1] : g[2];
+      }
+#pragma unroll
+      for (int a = 0; a < 3; a++) v[a] = a == d ? sum : 0.0;
+    }
+  } else {  // hat_c e_d, in either form
+    const double X = i * rn, Y = j * rn, Z = k * rn;
+    const double hat = ((c & 1) ? X : 1 - X) * ((c & 2) ? Y : 1 - Y) * ((c & 4) ? Z : 1 - Z);
+#pragma unroll
+    for (int a = 0; a < 3; a++) v[a] = a == d ? hat : 0.0;
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_galerkin(const Cell* __restrict__ cells, const double* __restrict__ E, double nu, double h, int conv,
+                const double* __restrict__ x64, const double* __restrict__ ft, int form, double* __restrict__ Kc) {
+  __shared__ double red[4][3][256];
+  const int cell = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const Cell C = uniform_cell(cells, cell);
+  const int n = C.n, nh = n * n * n;
+  const double hf = h / n, rn = 1.0 / n;
   const double lamf = nu / ((1.0 + nu) * (1.0 - 2.0 * nu)), muf = 1.0 / (2.0 * (1.0 + nu));
-  const int econv = form == MFS_BASIS_COMPONENTWISE ? (int)MFS_ELEM_TEXTBOOK : conv;
-  // register tiles: wave wv accumulates tets 2wv, 2wv+1 of every round; lane
-  // l owns the 3x3 tile (rows 3(l/8).., columns 3(l%8)..) of the 24x24 sum
-  const int wv = tid >> 6, ln = tid & 63, ti = ln >> 3, tj = ln & 7;
-  double acc[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-  const int ntet = 6 * n * n * n;
-  // every tet of the cell is a translate of one of 6 shapes: Ke = E_t KeS[shape]
-  if (tid < 6 * 16) {
-    const int p = tid / 16, I = (tid / 4) % 4, J = tid % 4;
-    int ijk[4][3];
-    tet_nodes(p, n, ijk);  // hex 0, shape p
-    double gr[4][3], V;
-    tet_grads(ijk, hf, gr, V);
-    double Kb[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    elastic_block(gr[I], gr[J], V * lamf, V * muf, econv, Kb);
-    for (int a = 0; a < 3; a++)
-      for (int b = 0; b < 3; b++) KeS[p][3 * I + a][3 * J + b] = Kb[a][b];
+  const bool textbook = form == MFS_BASIS_COMPONENTWISE || conv == MFS_ELEM_TEXTBOOK;
+  const double fx = textbook ? muf : lamf, fy = textbook ? lamf : muf;
+  const double* xc = x64 + C.int0 * 3 * NB;
+  const double* ftc = ft ? ft + C.ft0 : nullptr;
+  const double* Ec = E + C.tet0;
+  const int kk = lane >> 4, qa = lane & 15, qb = 16 + (lane & 7);
+  f64x4_t t00 = {0, 0, 0, 0}, t01 = {0, 0, 0, 0}, t11 = {0, 0, 0, 0};
+  for (int quad = wave; 4 * quad < nh; quad += 4) {
+    const int hex = 4 * quad + kk, hx = min(hex, nh - 1);  // (past the last hex: weight 0)
+    const int ci = hx % n, cj = (hx / n) % n, ck = hx / (n * n);
+    double va[8][3], vb[8][3];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int i = ci + (q & 1), j = cj + ((q >> 1) & 1), k = ck + (q >> 2);
+      coarse_function_at(xc, ftc, n, rn, form, i, j, k, qa, va[q]);
+      coarse_function_at(xc, ftc, n, rn, form, i, j, k, qb, vb[q]);
+    }
+#pragma unroll
+    for (int p = 0; p < 6; p++) {
+      // axis order of tet p (xyz, xzy, yxz, yzx, zxy, zyx) and its path of hex corners
+      const int p0 = p / 2, p1 = p % 2 == 0 ? (p0 == 0 ? 1 : 0) : (p0 == 2 ? 1 : 2), p2 = 3 - p0 - p1;
+      const int c1 = 1 << p0, c2 = c1 | (1 << p1);
+      // volume hf^3 / 6 and the 1 / hf of both gradients
+      const double w = hex < nh ? Ec[6 * hx + p] * (hf / 6.0) : 0.0;
+      const double wm = w * muf, wx = w * fx, wy = w * fy;
+      double ga[3][3], gb[3][3];
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        ga[a][p0] = va[c1][a] - va[0][a];
+        ga[a][p1] = va[c2][a] - va[c1][a];
+        ga[a][p2] = va[7][a] - va[c2][a];
+        gb[a][p0] = vb[c1][a] - vb[0][a];
+        gb[a][p1] = vb[c2][a] - vb[c1][a];
+        gb[a][p2] = vb[7][a] - vb[c2][a];
+      }
+      const double tra = wy * (ga[0][0] + ga[1][1] + ga[2][2]), trb = wy * (gb[0][0] + gb[1][1] + gb[2][2]);
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          double ha = wm * ga[a][b] + wx * ga[b][a], hb = wm * gb[a][b] + wx * gb[b][a];
+          if (a == b) {
+            ha += tra;
+            hb += trb;
+          }
+          t00 = __builtin_amdgcn_mfma_f64_16x16x4f64(ga[a][b], ha, t00, 0, 0, 0);
+          t01 = __builtin_amdgcn_mfma_f64_16x16x4f64(ga[a][b], hb, t01, 0, 0, 0);
+          t11 = __builtin_amdgcn_mfma_f64_16x16x4f64(gb[a][b], hb, t11, 0, 0, 0);
+        }
+    }
   }
-  for (int t0 = 0; t0 < ntet; t0 += GT) {
-    // element basis values of GT tets (zero past the last tet)
-    for (int q = tid; q < GT * 12 * NB; q += blockDim.x) {
-      const int g = q / (12 * NB), p = (q / NB) % 12, bq = q % NB;
-      const int t = t0 + g;
-      double val = 0.0;
-      if (t < ntet) {
-        // vertex v of the tet: the hex corner plus one along every axis
-        // stepped within the first v steps of the tet's axis order
-        const int vtx = p / 3, a = p % 3;
-        const int hex = t / 6, pm = t % 6;
-        const int i = hex % n + (vtx > kStepOf[pm][0]), j = (hex / n) % n + (vtx > kStepOf[pm][1]),
-                  k = hex / (n * n) + (vtx > kStepOf[pm][2]);
-        if (i >= 1 && i <= m && j >= 1 && j <= m && k >= 1 && k <= m) {
-          val = x64[(C.int0 + interior_index(i, j, k, m)) * 3 * NB + a * NB + bq];
-        } else {
-          double gv[3];
-          if (ft)
-            face_trace_at(ft + C.ft0, n, i, j, k, bq, gv);
-          else
-            hat_trace_at(n, i, j, k, bq, gv);
-          val = gv[a];
-        }
-      }
-      phi[g][p][bq] = val;
-    }
-    // moduli and shapes of the round's tets (modulus 0 past the last tet)
-    if (tid < GT) {
-      const int t = t0 + tid;
-      Eg[tid] = t < ntet ? E[C.tet0 + t] : 0.0;
-      Pg[tid] = t < ntet ? t % 6 : 0;
-    }
-    __syncthreads();
-    if (form == MFS_BASIS_COMPONENTWISE) {
-      // Psi_{c,a2}[p] = (p's component == a2) * sum_d phi_{c,d}[p]
-      for (int q = tid; q < GT * 12 * 8; q += blockDim.x) {
-        const int g = q / 96, p = (q / 8) % 12, c = q % 8;
-        const double sum = phi[g][p][3 * c] + phi[g][p][3 * c + 1] + phi[g][p][3 * c + 2];
-        for (int a2 = 0; a2 < 3; a2++) phi[g][p][3 * c + a2] = (p % 3 == a2) ? sum : 0.0;
-      }
-      __syncthreads();
-    }
-    {
-      // KP = Ke phi: one 3x3 tile (rows 3pb.., columns 3cb..) of one tet per thread
-      static_assert(GT * 4 * 8 == 256, "one KP tile per thread");
-      const int g = tid >> 5, pb = (tid >> 3) & 3, cb = tid & 7;
-      const int shp = Pg[g];
-      const double et = Eg[g];
-      double kp[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+  // accumulator r of a lane: row 4 r + lane / 16, column lane % 16
 #pragma unroll
-      for (int u = 0; u < 12; u++) {
-        double kr[3], pr[3];
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-          kr[r] = KeS[shp][3 * pb + r][u];
-          pr[r] = phi[g][u][3 * cb + r];
-        }
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) kp[r][c] += kr[r] * pr[c];
-      }
-#pragma unroll
-      for (int r = 0; r < 3; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) KP[g][3 * pb + r][3 * cb + c] = et * kp[r][c];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int gg = 0; gg < 2; gg++) {
-      const int g = 2 * wv + gg;
-#pragma unroll
-      for (int p = 0; p < 12; p++) {
-        double a[3], b[3];
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-          a[r] = phi[g][p][3 * ti + r];
-          b[r] = KP[g][p][3 * tj + r];
-        }
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) acc[r][c] += a[r] * b[c];
-      }
-    }
-    __syncthreads();
+  for (int r = 0; r < 4; r++) {
+    const int at = (4 * r + kk) * 16 + (lane & 15);
+    red[wave][0][at] = t00[r];
+    red[wave][1][at] = t01[r];
+    red[wave][2][at] = t11[r];
   }
-  // sum the four waves' tiles (phi is free now), then store
-  double* red = &phi[0][0][0];  // 4 x 576 doubles fit in GT*12*NB
-#pragma unroll
-  for (int r = 0; r < 3; r++)
-#pragma unroll
-    for (int c = 0; c < 3; c++) red[wv * NB * NB + (3 * ti + r) * NB + 3 * tj + c] = acc[r][c];
   __syncthreads();
   const bool bt = form == MFS_BASIS_COMPONENTWISE && conv == MFS_ELEM_REFERENCE;
-  for (int pr = tid; pr < NB * NB; pr += blockDim.x) {
+  for (int pr = tid; pr < NB * NB; pr += 256) {
     const int bi = pr / NB, bj = pr % NB;
-    const double v = (red[pr] + red[NB * NB + pr]) + (red[2 * NB * NB + pr] + red[3 * NB * NB + pr]);
+    int t, at;
+    if (bi < 16 && bj < 16) {
+      t = 0;
+      at = bi * 16 + bj;
+    } else if (bi >= 16 && bj >= 16) {
+      t = 2;
+      at = (bi - 16) * 16 + bj - 16;
+    } else {
+      t = 1;
+      at = min(bi, bj) * 16 + max(bi, bj) - 16;
+    }
+    const double v = (red[0][t][at] + red[1][t][at]) + (red[2][t][at] + red[3][t][at]);
     const int out = bt ? (3 * (bi / 3) + bj % 3) * NB + 3 * (bj / 3) + bi % 3 : pr;
     Kc[(int64_t)cell * NB * NB + out] = v;
   }
@@ -2024,6 +2030,7 @@ struct mfs_batch_s {
   unsigned long long* d_fstats = nullptr;  // [0] worst relative residual bits, [1] failures
   double* d_hat = nullptr;  // learned guess: the hat interpolant of one cell's entries
   int64_t hat_len = 0;
+  double* d_kc = nullptr;   // coarse matrices, from the first mfs_batch_coarse_matrices on
   unsigned long long* d_report = nullptr;  // k_batch_report's six sums
 };
 
@@ -2033,7 +2040,7 @@ static int batch_free(mfs_batch B) {
   void* ptrs[] = {B->d_cells, B->d_int0, B->d_tmpls, B->d_gptr, B->d_gent, B->d_E, B->d_K32, B->d_K64,
                   B->d_dinv32, B->d_dinv64, B->d_b64, B->d_x64, B->d_iters, B->d_relres, B->d_flags,
                   B->d_task_cell, B->d_task_group, B->d_mtask_cell, B->d_mtask_group, B->d_fb, B->d_queue, B->d_scr, B->d_et, B->d_ft, B->d_face_order,
-                  B->d_fstats, B->d_hat, B->d_report};
+                  B->d_fstats, B->d_hat, B->d_kc, B->d_report};
   for (void* p : ptrs) dfree(p);
   mfs_ctx c = B->ctx;
   delete B;
@@ -2754,13 +2761,12 @@ extern "C" int mfs_batch_coarse_matrices(mfs_batch B, double* Kc) {
   MFS_CHECK_ARG(B && Kc, "mfs_batch_coarse_matrices: bad argument");
   MFS_CHECK_ARG(B->assembled, "mfs_batch_coarse_matrices: call mfs_batch_assemble first");
   hipStream_t s = B->ctx->stream;
-  double* d_kc;
-  MFS_TRY(dmalloc((void**)&d_kc, sizeof(double) * NB * NB * B->ncells));
+  if (!B->d_kc) MFS_TRY(dmalloc((void**)&B->d_kc, sizeof(double) * NB * NB * B->ncells));
+  double* d_kc = B->d_kc;
   k_galerkin<<<B->ncells, 256, 0, s>>>(B->d_cells, B->d_E, B->nu, B->h, B->conv, B->d_x64, B->d_ft, B->form, d_kc);
   MFS_HIP(hipGetLastError());
   MFS_HIP(hipMemcpyAsync(Kc, d_kc, sizeof(double) * NB * NB * B->ncells, hipMemcpyDeviceToHost, s));
   MFS_HIP(hipStreamSynchronize(s));
-  dfree(d_kc);
   return MFS_OK;
 }
 

@@ -70,3 +70,35 @@ def test_iteration_cap_and_failure_list(ctx):
     handed = (fl & 8) != 0
     assert handed.sum() == rep.n_precision_fallback > 0
     B.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 5])
+@pytest.mark.parametrize("trace", [mfs.TRACE_Q1, mfs.TRACE_REFERENCE])
+@pytest.mark.parametrize("form", [mfs.BASIS_PER_DIRECTION, mfs.BASIS_COMPONENTWISE])
+@pytest.mark.parametrize("convention", [mfs.ELEM_REFERENCE, mfs.ELEM_TEXTBOOK])
+def test_coarse_matrices_equal_the_product_with_the_downloaded_bases(ctx, n, trace, form, convention):
+    """Kc = Phi^T K Phi with the library's own Phi and K summed from the
+    oracle's element matrices (hex counts 8, 27, 125: whole and ragged groups
+    of four).  Both are FP64 sums of at most 6 n^3 * 144 products, so they
+    agree to 1e-12 of the largest entry."""
+    h = 0.5
+    E = [np.exp(0.7 * np.random.default_rng([7, c]).standard_normal(6 * n ** 3)) for c in range(2)]
+    B = mfs.Batch(ctx, [n, n], [[0, 0, 0], [h, 0, 0]], h, np.concatenate(E), 0.3, convention=convention, trace=trace,
+                  coarse_basis=form)
+    B.assemble()
+    B.solve(precision=mfs.PREC_F64, tol=1e-9)
+    Kc = B.coarse_matrices()
+    assert np.array_equal(Kc, B.coarse_matrices())
+    xyz, tets = mfs.mesh_box(n, h=(h / n,) * 3)
+    econv = mfs.ELEM_TEXTBOOK if form == mfs.BASIS_COMPONENTWISE else convention
+    for c in range(2):
+        K = np.zeros((3 * len(xyz), 3 * len(xyz)))
+        for t, T in enumerate(tets):
+            d = (3 * T[:, None] + np.arange(3)).ravel()
+            K[np.ix_(d, d)] += orc.elem_elastic(xyz[T], E[c][t], 0.3, econv)
+        Phi = B.basis(c)
+        ref = Phi @ K @ Phi.T
+        if form == mfs.BASIS_COMPONENTWISE and convention == mfs.ELEM_REFERENCE:
+            ref = ref.reshape(8, 3, 8, 3).transpose(0, 3, 2, 1).reshape(24, 24)
+        assert np.abs(Kc[c] - ref).max() <= 1e-12 * np.abs(ref).max()
+    B.close()

@@ -78,6 +78,9 @@ constexpr bool kRegVar[4] = {false, false, true, true};
 constexpr int kVariants[2] = {4, 4};  // per precision: FP32 inner, FP64 inner
 // Largest workgroup of a variant: one register-resident row per thread
 // needs a thread per interior node, so that form takes up to 512 threads.
+// (One slab row per thread on 512 threads, two waves per SIMD where p leaves
+// room for one workgroup per CU, was slower: 1,000 cells of 10^3 74.9
+// against 65.4 ms, bound by the slab's traffic.)
 constexpr int max_threads(bool reg, int rpt) { return reg && rpt == 1 ? 512 : 256; }
 // Waves per SIMD a variant is compiled for: two where its registers allow
 // it (the compiler then spills cold code instead of dropping to one).
@@ -2515,8 +2518,18 @@ static int resident_per_cu(mfs_batch B, int precision, int wg, int var) {
 
 static int pick_shape(mfs_batch B, const mfs_batch_solve_desc* d, int* wg, int* per_cu, int* var) {
   const int t = d->precision == MFS_PREC_F64 ? 1 : 0;
-  const int wgs = d->wg_size ? d->wg_size : (B->tuned_wg[t] ? B->tuned_wg[t] : 256);
+  int wgs = d->wg_size ? d->wg_size : (B->tuned_wg[t] ? B->tuned_wg[t] : 256);
   *var = d->variant > 0 ? d->variant - 1 : (B->tuned_var[t] >= 0 ? B->tuned_var[t] : 0);
+  // FP64 with nothing asked for and nothing tuned: the register-resident
+  // kernel with a thread per row wherever every cell fits it (n <= 8; d and p
+  // take 143 KB of LDS there).  Against the slab kernel on 256 threads: 512
+  // cells of 8^3 5.1 / 15.7 ms, 1,000 cells of 5^3 1.17 / 3.29 ms, of n =
+  // 3..7 3.9 / 6.0 ms.
+  const int rows = (B->max_nint + 63) / 64 * 64;
+  if (t == 1 && !d->wg_size && d->variant <= 0 && B->tuned_var[t] < 0 && variant_fits(B, d->precision, 2, rows)) {
+    wgs = rows;
+    *var = 2;
+  }
   *wg = wgs;
   *per_cu = (!d->wg_size && B->tuned_per_cu[t]) ? B->tuned_per_cu[t] : resident_per_cu(B, d->precision, wgs, *var);
   return MFS_OK;

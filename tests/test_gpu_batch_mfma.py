@@ -102,3 +102,19 @@ def test_coarse_matrices_equal_the_product_with_the_downloaded_bases(ctx, n, tra
             ref = ref.reshape(8, 3, 8, 3).transpose(0, 3, 2, 1).reshape(24, 24)
         assert np.abs(Kc[c] - ref).max() <= 1e-12 * np.abs(ref).max()
     B.close()
+
+
+@pytest.mark.parametrize("sizes", [[8, 2], [9, 3], [5, 5]])
+def test_fp64_default_shape_matches_the_slab_kernel(ctx, sizes):
+    """FP64 with no shape asked for (register-resident up to n = 8, slab
+    above) against the slab kernel asked for by name: both stop at a true
+    relative residual of 1e-10, condition numbers below 1e2."""
+    B, *_ = batch(ctx, sizes, 8)
+    rep = B.solve(precision=mfs.PREC_F64, tol=1e-10)
+    assert rep.n_not_converged == 0 and rep.max_true_relres <= 1e-10
+    x = [B.basis(c) for c in range(len(sizes))]
+    B.solve(precision=mfs.PREC_F64, tol=1e-10, variant=1, wg_size=256)
+    for c in range(len(sizes)):
+        ref = B.basis(c)
+        assert np.linalg.norm(x[c] - ref) <= 1e-8 * np.linalg.norm(ref)
+    B.close()

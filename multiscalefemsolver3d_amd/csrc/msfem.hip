@@ -102,7 +102,6 @@ struct Cell {
   int nint;     // interior nodes (n-1)^3
   int64_t tet0; // first tet in E
   int64_t int0; // first interior node (global numbering over cells)
-  int tmpl;     // template id
   double ox, oy, oz;
   int64_t et0;  // reference-trace mode: first edge-profile entry (12*(n+1)*2 per cell)
   int64_t ft0;  // reference-trace mode: first face-trace entry (6*(n+1)^2*36 per cell)
@@ -138,14 +137,12 @@ __host__ __device__ __forceinline__ int edge_id(int dir, int axa, int sa, int ax
 }
 constexpr int FT_NODE = 36;  // face-trace values per face node: [a][lc][d]
 
-// Boundary value (3 components) of basis q = 3c + d at boundary node
-// (i, j, k) of an n-cell from its face traces: any face holding both the
-// node and corner c (they agree on shared edges), 0 when none does.
-__host__ __device__ __forceinline__ void face_trace_at(const double* ft_cell, int n, int i, int j, int k, int q,
-                                                       double (&g)[3]) {
-  const int c = q / 3, d = q % 3;
+// Face-trace values of corner c at boundary node (i, j, k) of an n-cell: entry
+// a * 12 + d is component a of basis 3c + d.  Any face holding both the node
+// and the corner (they agree on shared edges); null when none does (0).
+__host__ __device__ __forceinline__ const double* face_trace_of(const double* ft_cell, int n, int i, int j, int k,
+                                                                int c) {
   const int idx[3] = {i, j, k};
-  g[0] = g[1] = g[2] = 0.0;
   for (int ax = 0; ax < 3; ax++) {
     const int side = idx[ax] == 0 ? 0 : (idx[ax] == n ? 1 : -1);
     if (side < 0 || ((c >> ax) & 1) != side) continue;
@@ -153,10 +150,16 @@ __host__ __device__ __forceinline__ void face_trace_at(const double* ft_cell, in
     face_axes(ax, A1, A2);
     const int lc = ((c >> A1) & 1) + 2 * ((c >> A2) & 1);
     const int64_t w = idx[A1] + (int64_t)(n + 1) * idx[A2];
-    const double* base = ft_cell + (((int64_t)(2 * ax + side) * (n + 1) * (n + 1) + w) * FT_NODE) + 3 * lc + d;
-    for (int a = 0; a < 3; a++) g[a] = base[a * 12];
-    return;
+    return ft_cell + (((int64_t)(2 * ax + side) * (n + 1) * (n + 1) + w) * FT_NODE) + 3 * lc;
   }
+  return nullptr;
+}
+// Boundary value (3 components) of basis q = 3c + d at boundary node
+// (i, j, k) of an n-cell from its face traces.
+__host__ __device__ __forceinline__ void face_trace_at(const double* ft_cell, int n, int i, int j, int k, int q,
+                                                       double (&g)[3]) {
+  const double* base = face_trace_of(ft_cell, n, i, j, k, q / 3);
+  for (int a = 0; a < 3; a++) g[a] = base ? base[a * 12 + q % 3] : 0.0;
 }
 
 // Q1 boundary value hat_c(x) e_d.
@@ -167,12 +170,6 @@ __host__ __device__ __forceinline__ void hat_trace_at(int n, int i, int j, int k
   g[0] = g[1] = g[2] = 0.0;
   g[d] = hat;
 }
-
-struct Tmpl {  // per distinct n: gather lists of interior rows x stencil
-  int n;
-  int64_t ptr0;  // offset into g_ptr (nint*NS+1 entries)
-  int64_t ent0;  // offset into g_ent
-};
 
 // Task queues: one per XCD.  Workgroups are dispatched round-robin over the
 // 8 XCDs, so workgroup b pulls from queue b % 8 first; all three tasks of a
@@ -229,13 +226,6 @@ __device__ __forceinline__ int interior_index(int i, int j, int k, int m) {
   return (i - 1) + m * ((j - 1) + m * (k - 1));
 }
 
-// ---------------------------------------------------------------------------
-// Cell assembly: one thread per (cell, interior node).  For each stencil
-// block, sum the element contributions (template gather lists, ascending
-// tet order) with gradients recomputed from the structured fine geometry.
-// Interior-neighbour blocks go to K (FP64 and FP32); boundary-neighbour
-// blocks update b = -K_IB g for the 24 bases.
-// ---------------------------------------------------------------------------
 __device__ void tet_nodes(int t, int n, int (&ijk)[4][3]) {
   const int hex = t / 6, p = t % 6;
   int c[3] = {hex % n, (hex / n) % n, hex / (n * n)};
@@ -288,87 +278,258 @@ __device__ __forceinline__ void elastic_block(const double* dI, const double* dJ
     }
 }
 
-__global__ __launch_bounds__(256) void k_cell_assemble(const Cell* __restrict__ cells, int ncells,
-                                                       const int64_t* __restrict__ node_cell_ptr,
-                                                       const Tmpl* __restrict__ tmpls,
-                                                       const int64_t* __restrict__ g_ptr,
-                                                       const uint32_t* __restrict__ g_ent,
-                                                       const double* __restrict__ E, double nu, double h, int conv,
-                                                       const double* __restrict__ ft, int64_t total_int,
-                                                       int tiled, float* __restrict__ K32,
-                                                       double* __restrict__ K64, float* __restrict__ dinv32,
-                                                       double* __restrict__ dinv64, double* __restrict__ b64) {
-  for (int64_t gv = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; gv < total_int;
-       gv += (int64_t)gridDim.x * blockDim.x) {
-    // find the cell (binary search over cumulative interior counts)
-    int lo = 0, hi = ncells - 1;
-    while (lo < hi) {
-      int mid = (lo + hi + 1) >> 1;
-      if (node_cell_ptr[mid] <= gv) lo = mid;
-      else hi = mid - 1;
-    }
-    const Cell C = cells[lo];
-    const Tmpl T = tmpls[C.tmpl];
-    const int n = C.n, m = n - 1, nint = C.nint;
-    const int v = (int)(gv - C.int0);
-    const int i = v % m + 1, j = (v / m) % m + 1, k = v / (m * m) + 1;
-    const double hf = h / n;
-    const double lamf = nu / ((1.0 + nu) * (1.0 - 2.0 * nu)), muf = 1.0 / (2.0 * (1.0 + nu));
-    double bacc[3][NB];
+// ---------------------------------------------------------------------------
+// Cell assembly: one workgroup per cell, one thread per interior node.
+//
+// A tet steps from a hex corner along its three axes p0, p1, p2; times h the
+// gradients of its hat functions are -e_p0, e_p0 - e_p1, e_p1 - e_p2, e_p2.
+// The block of stencil point s is therefore a signed sum of the moduli of
+// the 4, 6 (or, on the diagonal, 24) tets that hold both nodes:
+//   S[a][b] = sum_t w_t gI[a] gJ[b],  w = E h / 6,
+//   K[a][b] = F S[a][b] + H S[b][a] + delta_ab mu tr S,
+// (F, H) = (lambda, mu) in the textbook convention, (mu, lambda) in the
+// reference's.  A thread loads the 24 moduli around its node once; the signs
+// are compile-time constants.  Blocks towards boundary nodes are stored as 0
+// and enter b = -K_IB g instead (formed again in a loop over the stencil, so
+// that the 72 sums of b exist once in the code).
+//
+// Bound by its stores (2.3 KB per node: K in FP64 and FP32, b) and, at nodes
+// next to the boundary, by b.  16^3 cells of n = 6..10: 2.7 ms (3.0 with the
+// moduli read from global memory instead of LDS); the gather over per-template
+// lists with the element recomputed per contribution took 3.9 ms.
+// ---------------------------------------------------------------------------
+// corner of local vertex I of tet p (bits x, y, z), and its gradient's signs
+__host__ __device__ constexpr int tet_axis(int p, int s) {
+  return s == 0 ? p / 2 : s == 1 ? (p % 2 == 0 ? (p / 2 == 0 ? 1 : 0) : (p / 2 == 2 ? 1 : 2))
+                                 : 3 - tet_axis(p, 0) - tet_axis(p, 1);
+}
+__host__ __device__ constexpr int tet_corner(int p, int I) {
+  int c = 0;
+  for (int s = 0; s < I; s++) c |= 1 << tet_axis(p, s);
+  return c;
+}
+__host__ __device__ constexpr int tet_sign(int p, int I, int a) {
+  return (I > 0 && tet_axis(p, I - 1) == a ? 1 : 0) - (I < 3 && tet_axis(p, I) == a ? 1 : 0);
+}
+// vertex J of tet p at the offset of stencil point s from vertex I, or -1
+__host__ __device__ constexpr int tet_partner(int p, int I, int s) {
+  for (int J = 0; J < 4; J++) {
+    bool same = true;
     for (int a = 0; a < 3; a++)
-      for (int q = 0; q < NB; q++) bacc[a][q] = 0.0;
-    float* K32c = K32 + C.kt0;
-    double* K64c = K64 + C.int0 * (NS * 9);
-    for (int s = 0; s < NS; s++) {
-      const int ni = i + c_stencil[s][0], nj = j + c_stencil[s][1], nk = k + c_stencil[s][2];
-      double Kb[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-      const int64_t slot = (int64_t)v * NS + s;
-      for (int64_t q = g_ptr[T.ptr0 + slot]; q < g_ptr[T.ptr0 + slot + 1]; q++) {
-        const uint32_t ce = g_ent[T.ent0 + q];
-        const int t = (int)(ce >> 4), li = (ce >> 2) & 3, lj = ce & 3;
-        int ijk[4][3];
-        tet_nodes(t, n, ijk);
-        double g[4][3], V;
-        tet_grads(ijk, hf, g, V);
-        const double Et = E[C.tet0 + t];
-        elastic_block(g[li], g[lj], V * Et * lamf, V * Et * muf, conv, Kb);
+      same = same && ((tet_corner(p, J) >> a) & 1) - ((tet_corner(p, I) >> a) & 1) == kStencil[s][a];
+    if (same) return J;
+  }
+  return -1;
+}
+// The tets of one off-diagonal stencil point for the boundary loop: tet p,
+// the node's corner in its hex, and the two gradients' signs (2 bits each:
+// sign + 1).
+struct PointTets {
+  int count;
+  uint32_t code[6];  // p | corner << 3 | (gI[a] + 1) << (6 + 2a) | (gJ[a] + 1) << (12 + 2a); padded with zero signs
+};
+struct StencilTets {
+  PointTets pt[NS];
+};
+constexpr StencilTets make_stencil_tets() {
+  StencilTets T{};
+  for (int s = 0; s < NS; s++) {
+    if (s == S_CENTER) continue;
+    for (int p = 0; p < 6; p++)
+      for (int I = 0; I < 4; I++) {
+        const int J = tet_partner(p, I, s);
+        if (J < 0) continue;
+        uint32_t c = (uint32_t)p | (uint32_t)tet_corner(p, I) << 3;
+        for (int a = 0; a < 3; a++)
+          c |= (uint32_t)(tet_sign(p, I, a) + 1) << (6 + 2 * a) | (uint32_t)(tet_sign(p, J, a) + 1) << (12 + 2 * a);
+        T.pt[s].code[T.pt[s].count++] = c;
       }
-      const bool interior = ni >= 1 && ni <= m && nj >= 1 && nj <= m && nk >= 1 && nk <= m;
+    for (int e = T.pt[s].count; e < 6; e++) T.pt[s].code[e] = 0x15u << 6 | 0x15u << 12;
+  }
+  return T;
+}
+__constant__ constexpr StencilTets c_tets = make_stencil_tets();
+
+// S of stencil point s from the 24 moduli around a node (w[4 p + I])
+template <int S_>
+__device__ __forceinline__ void point_sums(const double (&w)[24], double (&S)[3][3]) {
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) S[a][b] = 0.0;
+#pragma unroll
+  for (int p = 0; p < 6; p++)
+#pragma unroll
+    for (int I = 0; I < 4; I++) {
+      const int J = tet_partner(p, I, S_);
+      if (J < 0) continue;
+#pragma unroll
       for (int a = 0; a < 3; a++)
+#pragma unroll
         for (int b = 0; b < 3; b++) {
-          const int64_t at = (int64_t)(s * 9 + 3 * a + b) * nint + v;
-          K64c[at] = interior ? Kb[a][b] : 0.0;
-          K32c[tiled ? k32_tile_index(v, s, a, b) : at] = interior ? (float)Kb[a][b] : 0.0f;
+          const int sg = tet_sign(p, I, a) * tet_sign(p, J, b);
+          if (sg > 0) S[a][b] += w[4 * p + I];
+          if (sg < 0) S[a][b] -= w[4 * p + I];
         }
-      if (!interior) {
+    }
+}
+struct CellK {  // where one cell's matrix goes
+  double* K64;
+  float* K32;
+  int nint, m, tiled;
+  double F, H, mu;
+};
+__device__ __forceinline__ double block_entry(const CellK& C, const double (&S)[3][3], int a, int b) {
+  double v = C.F * S[a][b] + C.H * S[b][a];
+  if (a == b) v += C.mu * (S[0][0] + S[1][1] + S[2][2]);
+  return v;
+}
+
+// Stencil points S_ .. 14 of node v = (i, j, k); pend holds the FP32 values of
+// the last four points, stored as 16-byte chunks of the tiled layout.
+template <int S_>
+__device__ __forceinline__ void store_points(const CellK& C, const double (&w)[24], int v, int i, int j, int k,
+                                             float (&pend)[3][12], double (&diag)[3]) {
+  if constexpr (S_ < NS) {
+    const int ni = i + kStencil[S_][0], nj = j + kStencil[S_][1], nk = k + kStencil[S_][2];
+    const bool in = ni >= 1 && ni <= C.m && nj >= 1 && nj <= C.m && nk >= 1 && nk <= C.m;
+    double S[3][3];
+    point_sums<S_>(w, S);
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        const double kv = in ? block_entry(C, S, a, b) : 0.0;
+        const int64_t at = (int64_t)(S_ * 9 + 3 * a + b) * C.nint + v;
+        C.K64[at] = kv;
+        if (C.tiled)
+          pend[a][3 * (S_ % 4) + b] = (float)kv;
+        else
+          C.K32[at] = (float)kv;
+        if (S_ == S_CENTER && a == b) diag[a] = kv;
+      }
+    }
+    if (C.tiled && (S_ % 4 == 3 || S_ == NS - 1)) {
+#pragma unroll
+      for (int q = 0; q < 3; q++)  // chunks of entries 3 (S_ - S_ % 4) + 4 q ..
+        if (3 * (S_ - S_ % 4) + 4 * q < 3 * NS)
+#pragma unroll
+          for (int a = 0; a < 3; a++)
+            *reinterpret_cast<float4*>(C.K32 + k32_tile_index(v, S_ - S_ % 4 + (4 * q) / 3, a, (4 * q) % 3)) =
+                make_float4(pend[a][4 * q], pend[a][4 * q + 1], pend[a][4 * q + 2], pend[a][4 * q + 3]);
+    }
+    store_points<S_ + 1>(C, w, v, i, j, k, pend, diag);
+  }
+}
+
+constexpr int kAsmThreads = 128;  // 125 .. 729 nodes per cell: few idle lanes
+__global__ __launch_bounds__(kAsmThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_cell_assemble(const Cell* __restrict__ cells, const double* __restrict__ E, double nu, double h, int conv,
+                     const double* __restrict__ ft, int tiled, float* __restrict__ K32, double* __restrict__ K64,
+                     float* __restrict__ dinv32, double* __restrict__ dinv64, double* __restrict__ b64) {
+  const Cell C = uniform_cell(cells, blockIdx.x);
+  const int n = C.n, m = n - 1, nint = C.nint;
+  const double hf = h / n, rn = 1.0 / n;
+  const double lam = nu / ((1.0 + nu) * (1.0 - 2.0 * nu)), mu = 1.0 / (2.0 * (1.0 + nu));
+  CellK ck;
+  ck.K64 = K64 + C.int0 * (NS * 9);
+  ck.K32 = K32 + C.kt0;
+  ck.nint = nint;
+  ck.m = m;
+  ck.tiled = tiled;
+  ck.F = conv == MFS_ELEM_TEXTBOOK ? lam : mu;
+  ck.H = conv == MFS_ELEM_TEXTBOOK ? mu : lam;
+  ck.mu = mu;
+  // the cell's moduli, times h / 6, in LDS: every one is read 4 times by the
+  // nodes of its tet and again for b
+  extern __shared__ double w_lds[];
+  for (int t = threadIdx.x; t < 6 * n * n * n; t += kAsmThreads) w_lds[t] = E[C.tet0 + t] * (hf / 6.0);
+  __syncthreads();
+  for (int v = threadIdx.x; v < nint; v += kAsmThreads) {
+    const int i = v % m + 1, j = (v / m) % m + 1, k = v / (m * m) + 1;
+    {
+      double w[24];
+#pragma unroll
+      for (int p = 0; p < 6; p++)
+#pragma unroll
+        for (int I = 0; I < 4; I++) {
+          const int c = tet_corner(p, I);
+          const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
+          w[4 * p + I] = w_lds[6 * hex + p];
+        }
+      float pend[3][12];
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int q = 0; q < 12; q++) pend[a][q] = 0.f;
+      double diag[3];
+      store_points<0>(ck, w, v, i, j, k, pend, diag);
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        dinv64[(C.int0 + v) * 3 + a] = 1.0 / diag[a];
+        dinv32[(C.int0 + v) * 3 + a] = (float)(1.0 / diag[a]);
+      }
+    }
+    double bacc[3][NB];
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int q = 0; q < NB; q++) bacc[a][q] = 0.0;
+    if (i == 1 || i == m || j == 1 || j == m || k == 1 || k == m) {
+#pragma unroll 1
+      for (int s = 0; s < NS; s++) {
+        const int ni = i + c_stencil[s][0], nj = j + c_stencil[s][1], nk = k + c_stencil[s][2];
+        if (ni >= 1 && ni <= m && nj >= 1 && nj <= m && nk >= 1 && nk <= m) continue;
+        double S[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+        for (int e = 0; e < 6; e++) {
+          const uint32_t code = c_tets.pt[s].code[e];
+          const int p = code & 7, c = (code >> 3) & 7;
+          const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
+          const double w = w_lds[6 * hex + p];
+#pragma unroll
+          for (int a = 0; a < 3; a++) {
+            const double wa = w * (double)((int)((code >> (6 + 2 * a)) & 3) - 1);
+#pragma unroll
+            for (int b = 0; b < 3; b++) S[a][b] += wa * (double)((int)((code >> (12 + 2 * b)) & 3) - 1);
+          }
+        }
+        double Kb[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+#pragma unroll
+          for (int b = 0; b < 3; b++) Kb[a][b] = block_entry(ck, S, a, b);
         if (ft == nullptr) {
           // g for basis (c, d) at this boundary node: hat_c(x) e_d
-          const double X = (double)ni / n, Y = (double)nj / n, Z = (double)nk / n;
+          const double X = ni == n ? 1.0 : ni * rn, Y = nj == n ? 1.0 : nj * rn, Z = nk == n ? 1.0 : nk * rn;
+#pragma unroll
           for (int c = 0; c < 8; c++) {
             const double hat = ((c & 1) ? X : 1 - X) * ((c & 2) ? Y : 1 - Y) * ((c & 4) ? Z : 1 - Z);
-            if (hat == 0.0) continue;
+#pragma unroll
             for (int d = 0; d < 3; d++)
+#pragma unroll
               for (int a = 0; a < 3; a++) bacc[a][3 * c + d] -= Kb[a][d] * hat;
           }
         } else {
           // g from the face traces (reference-trace mode): full vectors
 #pragma unroll
-          for (int q = 0; q < NB; q++) {
-            double g[3];
-            face_trace_at(ft + C.ft0, n, ni, nj, nk, q, g);
-            for (int a = 0; a < 3; a++) bacc[a][q] -= Kb[a][0] * g[0] + Kb[a][1] * g[1] + Kb[a][2] * g[2];
+          for (int c = 0; c < 8; c++) {
+            const double* g = face_trace_of(ft + C.ft0, n, ni, nj, nk, c);
+            if (!g) continue;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+              for (int a = 0; a < 3; a++)
+                bacc[a][3 * c + d] -= Kb[a][0] * g[d] + Kb[a][1] * g[12 + d] + Kb[a][2] * g[24 + d];
           }
         }
       }
-      if (s == S_CENTER)
-        for (int a = 0; a < 3; a++) {
-          dinv64[(C.int0 + v) * 3 + a] = 1.0 / Kb[a][a];
-          dinv32[(C.int0 + v) * 3 + a] = (float)(1.0 / Kb[a][a]);
-        }
     }
-    double* bv = b64 + (C.int0 + v) * (3 * NB);
+    double2* bv = reinterpret_cast<double2*>(b64 + (C.int0 + v) * (3 * NB));
+#pragma unroll
     for (int a = 0; a < 3; a++)
-      for (int q = 0; q < NB; q++) bv[a * NB + q] = bacc[a][q];
+#pragma unroll
+      for (int q = 0; q < NB; q += 2) bv[(a * NB + q) / 2] = make_double2(bacc[a][q], bacc[a][q + 1]);
   }
 }
 
@@ -1515,7 +1676,7 @@ __device__ __forceinline__ void coarse_function_at(const double* __restrict__ xc
       for (int a = 0; a < 3; a++) v[a] = a == d ? sum : 0.0;
     }
   } else {  // hat_c e_d, in either form
-    const double X = i * rn, Y = j * rn, Z = k * rn;
+    const double X = i == n ? 1.0 : i * rn, Y = j == n ? 1.0 : j * rn, Z = k == n ? 1.0 : k * rn;
     const double hat = ((c & 1) ? X : 1 - X) * ((c & 2) ? Y : 1 - Y) * ((c & 4) ? Z : 1 - Z);
 #pragma unroll
     for (int a = 0; a < 3; a++) v[a] = a == d ? hat : 0.0;
@@ -1986,7 +2147,6 @@ struct mfs_batch_s {
   double h = 1.0, nu = 0.3;
   int conv = MFS_ELEM_REFERENCE;
   std::vector<Cell> cells;
-  std::vector<int64_t> int0;  // per cell
   int64_t total_int = 0, total_tets = 0;
   int max_n = 0, max_nint = 0;
   int ntasks = 0;
@@ -2005,10 +2165,6 @@ struct mfs_batch_s {
   double trace_ms = 0.0;       // device time of the edge + face launches
   // device
   Cell* d_cells = nullptr;
-  int64_t* d_int0 = nullptr;
-  Tmpl* d_tmpls = nullptr;
-  int64_t* d_gptr = nullptr;
-  uint32_t* d_gent = nullptr;
   double* d_E = nullptr;
   float* d_K32 = nullptr;
   double* d_K64 = nullptr;
@@ -2040,7 +2196,7 @@ struct mfs_batch_s {
 static int batch_free(mfs_batch B) {
   if (!B) return MFS_OK;
   if (B->ctx) (void)hipStreamSynchronize(B->ctx->stream);
-  void* ptrs[] = {B->d_cells, B->d_int0, B->d_tmpls, B->d_gptr, B->d_gent, B->d_E, B->d_K32, B->d_K64,
+  void* ptrs[] = {B->d_cells, B->d_E, B->d_K32, B->d_K64,
                   B->d_dinv32, B->d_dinv64, B->d_b64, B->d_x64, B->d_iters, B->d_relres, B->d_flags,
                   B->d_task_cell, B->d_task_group, B->d_mtask_cell, B->d_mtask_group, B->d_fb, B->d_queue, B->d_scr, B->d_et, B->d_ft, B->d_face_order,
                   B->d_fstats, B->d_hat, B->d_kc, B->d_report};
@@ -2077,54 +2233,8 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   B->trace = d->trace;
   B->form = d->coarse_basis;
   if (d->trace_tol > 0) B->trace_tol = d->trace_tol;
-  // templates per distinct n
-  std::map<int, int> tmpl_of;
-  std::vector<Tmpl> tmpls;
-  std::vector<int64_t> gptr_all;
-  std::vector<uint32_t> gent_all;
-  for (int c = 0; c < d->n_cells; c++) {
-    const int n = d->cell_n[c];
-    if (tmpl_of.count(n)) continue;
-    const int s = n + 1, m = n - 1;
-    std::vector<double> xyz(3 * (size_t)s * s * s);
-    std::vector<int32_t> tets(4 * 6 * (size_t)n * n * n);
-    mfs_mesh_box(n, n, n, 0, 0, 0, 1, 1, 1, xyz.data(), tets.data());
-    Pattern P;
-    build_pattern((int64_t)s * s * s, 6ll * n * n * n, tets.data(), P);
-    GatherLists G;
-    build_gather_lists(P, 6ll * n * n * n, tets.data(), G);
-    Tmpl T;
-    T.n = n;
-    T.ptr0 = (int64_t)gptr_all.size();
-    T.ent0 = (int64_t)gent_all.size();
-    int64_t base = 0;
-    gptr_all.push_back(0);
-    for (int k = 1; k <= m; k++)
-      for (int j = 1; j <= m; j++)
-        for (int i = 1; i <= m; i++) {
-          const int row = i + s * (j + s * k);
-          for (int st = 0; st < NS; st++) {
-            const int col = (i + h_stencil[st][0]) + s * ((j + h_stencil[st][1]) + s * (k + h_stencil[st][2]));
-            const int32_t* b0 = P.col.data() + P.rowptr[row];
-            const int32_t* e0 = P.col.data() + P.rowptr[row + 1];
-            const int32_t* f = std::lower_bound(b0, e0, col);
-            if (f == e0 || *f != col) {
-              set_error("mfs_batch_create: stencil point missing from the cell pattern");
-              batch_free(B);
-              return MFS_ERR_ARG;
-            }
-            const int64_t slot = f - P.col.data();
-            for (int64_t q = G.ptr[slot]; q < G.ptr[slot + 1]; q++) gent_all.push_back(G.entry[q]);
-            base += G.ptr[slot + 1] - G.ptr[slot];
-            gptr_all.push_back(base);
-          }
-        }
-    tmpl_of[n] = (int)tmpls.size();
-    tmpls.push_back(T);
-  }
   // cells
   B->cells.resize(d->n_cells);
-  B->int0.resize(d->n_cells);
   int64_t t0 = 0, i0 = 0, e0 = 0, f0 = 0;
   for (int c = 0; c < d->n_cells; c++) {
     Cell& C = B->cells[c];
@@ -2136,11 +2246,9 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
     C.nint = (C.n - 1) * (C.n - 1) * (C.n - 1);
     C.tet0 = t0;
     C.int0 = i0;
-    C.tmpl = tmpl_of[C.n];
     C.ox = d->cell_origin[3 * c];
     C.oy = d->cell_origin[3 * c + 1];
     C.oz = d->cell_origin[3 * c + 2];
-    B->int0[c] = i0;
     t0 += 6ll * C.n * C.n * C.n;
     i0 += C.nint;
     B->max_n = std::max(B->max_n, C.n);
@@ -2189,10 +2297,6 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
     if (st == MFS_OK) st = dmalloc(p, bytes);
   };
   alloc((void**)&B->d_cells, sizeof(Cell) * d->n_cells);
-  alloc((void**)&B->d_int0, sizeof(int64_t) * d->n_cells);
-  alloc((void**)&B->d_tmpls, sizeof(Tmpl) * tmpls.size());
-  alloc((void**)&B->d_gptr, sizeof(int64_t) * gptr_all.size());
-  alloc((void**)&B->d_gent, sizeof(uint32_t) * std::max<size_t>(1, gent_all.size()));
   alloc((void**)&B->d_E, sizeof(double) * t0);
   alloc((void**)&B->d_K32, sizeof(float) * B->k32_total);
   alloc((void**)&B->d_K64, sizeof(double) * NS * 9 * i0);
@@ -2225,10 +2329,6 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   hipStream_t s = ctx->stream;
   MFS_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_stencil), h_stencil, sizeof(h_stencil)));
   MFS_HIP(hipMemcpyAsync(B->d_cells, B->cells.data(), sizeof(Cell) * d->n_cells, hipMemcpyHostToDevice, s));
-  MFS_HIP(hipMemcpyAsync(B->d_int0, B->int0.data(), sizeof(int64_t) * d->n_cells, hipMemcpyHostToDevice, s));
-  MFS_HIP(hipMemcpyAsync(B->d_tmpls, tmpls.data(), sizeof(Tmpl) * tmpls.size(), hipMemcpyHostToDevice, s));
-  MFS_HIP(hipMemcpyAsync(B->d_gptr, gptr_all.data(), sizeof(int64_t) * gptr_all.size(), hipMemcpyHostToDevice, s));
-  MFS_HIP(hipMemcpyAsync(B->d_gent, gent_all.data(), sizeof(uint32_t) * gent_all.size(), hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemcpyAsync(B->d_E, d->E, sizeof(double) * t0, hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemcpyAsync(B->d_task_cell, tc.data(), sizeof(int) * B->ntasks, hipMemcpyHostToDevice, s));
   MFS_HIP(hipMemcpyAsync(B->d_task_group, tg.data(), sizeof(int) * B->ntasks, hipMemcpyHostToDevice, s));
@@ -2285,10 +2385,11 @@ extern "C" int mfs_batch_assemble(mfs_batch B) {
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
   }
-  const unsigned grid = (unsigned)std::min<int64_t>(65536, (B->total_int + 255) / 256);
-  k_cell_assemble<<<grid, 256, 0, s>>>(B->d_cells, B->ncells, B->d_int0, B->d_tmpls, B->d_gptr, B->d_gent, B->d_E,
-                                       B->nu, B->h, B->conv, B->d_ft, B->total_int, B->tiled ? 1 : 0, B->d_K32, B->d_K64,
-                                       B->d_dinv32, B->d_dinv64, B->d_b64);
+  const size_t asm_lds = sizeof(double) * 6 * B->max_n * B->max_n * B->max_n;  // 83 KB at n = 12
+  (void)hipFuncSetAttribute((const void*)k_cell_assemble, hipFuncAttributeMaxDynamicSharedMemorySize, (int)asm_lds);
+  k_cell_assemble<<<B->ncells, kAsmThreads, asm_lds, s>>>(B->d_cells, B->d_E, B->nu, B->h, B->conv, B->d_ft,
+                                                    B->tiled ? 1 : 0, B->d_K32, B->d_K64, B->d_dinv32, B->d_dinv64,
+                                                    B->d_b64);
   MFS_HIP(hipGetLastError());
   MFS_HIP(hipStreamSynchronize(s));
   B->assembled = true;

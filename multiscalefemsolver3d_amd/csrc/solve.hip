@@ -649,93 +649,191 @@ __global__ void k_combine(const T* __restrict__ V, const double* __restrict__ y,
 // ---------------------------------------------------------------------------
 // Preconditioned MINRES for symmetric (possibly indefinite) A with SPD M =
 // diag(A) (Elman, Silvester & Wathen, "Finite Elements and Fast Iterative
-// Solvers", Algorithm 2.4).  The scalar recurrence (Lanczos norms, Givens
-// rotations, eta) stays on the device: a one-thread kernel per step updates
-// it, and the host reads the stop record every 8 steps; updates of steps
-// launched past the stopping one leave x unchanged.
+// Solvers", Algorithm 2.4), two kernels per step like the PCG:
+//  k_mr_spmv(t):    from k_mr_lanczos(t-1)'s partials ||v_t||_M; the Givens
+//                   rotation of step t-1, w and x of step t-1 (own rows);
+//                   q = A z_t and partials of z_t . q
+//  k_mr_lanczos(t): delta from those partials; v_{t+1}, u_{t+1} = D^-1 v_{t+1}
+//                   and partials of u . v
+// z_t = u_t / ||v_t||_M is never stored: the products read u and scale the
+// result.  Every block evaluates the scalar recurrence from the state that
+// the previous k_mr_spmv wrote to the other of two buffers; block 0 writes
+// the new one.  Once a step has stopped, later kernels change nothing.
+// The recurrence as seven launches per step (product, dot, its sum, Lanczos,
+// its sum, rotation, update), launched one by one, took 21.2 us per step on
+// the 20^3 elastic cube in FP32 and 26.8 in FP64; two launches replayed from a
+// graph 11.9 and 16.9 (40^3: 28.5 and 45.5, now 16.4 and 34.5).
 // ---------------------------------------------------------------------------
-// MINRES recurrence scalars on the device (doubles): the Lanczos norms, the
-// Givens rotation of the last two steps, eta, the update coefficients of
-// the current step, and the stop record (-1 while running, else the index of
-// the last step whose update applies; kMsBad = 1 when that step's rotation
-// failed and its update must not apply either).
-enum {
-  kMsG, kMsGPrev, kMsC, kMsCPrev, kMsSPrev, kMsS, kMsEta, kMsEta0, kMsA1, kMsA2, kMsA3, kMsCEta, kMsInvG, kMsRtol,
-  kMsStop, kMsBad, kMsCount
+struct MinresState {
+  double G, GPrev, C, CPrev, SPrev, S, Eta, Eta0, Rtol;
+  int k;         // k_mr_spmv launches that have run
+  int maxsteps;
+  int stop;      // -1 while running, else the steps taken
+  int bad;       // 1: a rotation failed, 2: the starting norm is zero, 3: it is not finite
 };
 
-// one thread: rotation of step `step` from delta (dh[1]) and ||v_{j+1}||_M^2 (dh[2])
-__global__ void k_minres_rot(const double* __restrict__ dh, double* __restrict__ ms, int step) {
-  if (threadIdx.x != 0 || blockIdx.x != 0 || ms[kMsStop] >= 0.0) return;
-  const double delta = dh[1], g_next = sqrt(fmax(dh[2], 0.0));
-  const double g = ms[kMsG], c = ms[kMsC], c_prev = ms[kMsCPrev], s_prev = ms[kMsSPrev], s_cur = ms[kMsS];
-  const double a0 = c * delta - c_prev * s_cur * g;
-  const double a1 = sqrt(a0 * a0 + g_next * g_next);
-  if (!isfinite(delta) || !isfinite(g_next) || !(a1 > 0)) {
-    ms[kMsBad] = 1.0;
-    ms[kMsStop] = step;
-    return;
-  }
-  const double c_next = a0 / a1, s_next = g_next / a1, eta = ms[kMsEta];
-  ms[kMsA1] = a1;
-  ms[kMsA2] = s_cur * delta + c_prev * c * g;
-  ms[kMsA3] = s_prev * g;
-  ms[kMsCEta] = c_next * eta;
-  ms[kMsInvG] = g_next > 0 ? 1.0 / g_next : 0.0;
-  const double eta_next = -s_next * eta;
-  ms[kMsEta] = eta_next;
-  ms[kMsCPrev] = c;
-  ms[kMsC] = c_next;
-  ms[kMsSPrev] = s_cur;
-  ms[kMsS] = s_next;
-  ms[kMsGPrev] = g;
-  ms[kMsG] = g_next;
-  if (fabs(eta_next) <= ms[kMsRtol] * ms[kMsEta0] || g_next == 0) ms[kMsStop] = step;
+__global__ void k_mr_init(MinresState* st, double rtol, int maxsteps) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  MinresState m = {};
+  m.C = m.CPrev = 1.0;
+  m.Rtol = rtol;
+  m.maxsteps = maxsteps;
+  m.stop = -1;
+  *st = m;
 }
 
-// v_new = q - (delta/g) v - (g/g_prev) v_old; z_new = dinv v_new;
-// per-block partial of z_new . v_new.   delta from device memory.
-template <typename T>
-__global__ __launch_bounds__(256) void k_minres_lanczos(const T* __restrict__ q, const T* __restrict__ v,
-                                                        const T* __restrict__ v_old, T* __restrict__ v_new,
-                                                        T* __restrict__ z_new, const T* __restrict__ dinv,
-                                                        const double* __restrict__ delta,
-                                                        const double* __restrict__ ms, int64_t n,
-                                                        double* __restrict__ partials) {
-  const double g = ms[kMsG], g_prev = ms[kMsGPrev];
-  const T c1 = (T)(delta[0] / g), c2 = g_prev > 0 ? (T)(g / g_prev) : (T)0;
+template <typename T, int BS, typename CI>
+__global__ __launch_bounds__(256) void k_mr_spmv(const int64_t* __restrict__ slice_base,
+                                                 const int32_t* __restrict__ slice_width,
+                                                 const CI* __restrict__ col, const T* __restrict__ val,
+                                                 const T* __restrict__ u, const T* __restrict__ u_prev,
+                                                 const T* __restrict__ w_old, const T* __restrict__ w,
+                                                 T* __restrict__ w_new, T* __restrict__ x, T* __restrict__ q,
+                                                 int64_t nb, int64_t n_slices, const MinresState* __restrict__ st_in,
+                                                 MinresState* __restrict__ st_out, const double* __restrict__ delta,
+                                                 const double* __restrict__ part_g, unsigned g_g,
+                                                 double* __restrict__ part_d, int xcd) {
+  MinresState m = *st_in;
+  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+  double pre[1][4];
+  partials_issue<1, 4>(part_g, g_g, pre);
+  if (m.stop >= 0) {
+    if (writer) *st_out = m;
+    return;
+  }
+  const int64_t slice = (int64_t)xcd_block(xcd) * 4 + threadIdx.x / 64;
+  const int lane = threadIdx.x & 63;
+  const int64_t r = slice * 64 + lane;
+  const bool own = r < nb;
+  const double dlt = *delta;
+  // everything that does not depend on the scalars is loaded first
+  T acc[BS], uo[BS], up[BS], wo[BS], wc[BS], xo[BS];
+#pragma unroll
+  for (int a = 0; a < BS; a++) acc[a] = uo[a] = up[a] = wo[a] = wc[a] = xo[a] = 0;
+  if (own)
+#pragma unroll
+    for (int a = 0; a < BS; a++) {
+      const int64_t i = BS * r + a;
+      uo[a] = u[i];
+      up[a] = u_prev[i];
+      wo[a] = w_old[i];
+      wc[a] = w[i];
+      xo[a] = x[i];
+    }
+  if (slice < n_slices)
+    sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb, [&](int64_t i) { return u[i]; }, acc);
+  double tot[1];
+  partials_finish<1, 4>(part_g, g_g, pre, tot);
+  const double g_next = sqrt(fmax(tot[0], 0.0));
+  const bool first = m.k == 0;
+  bool update = false;
+  T ia1 = 0, ta2 = 0, ta3 = 0, tc = 0, tz = 0;
+  if (first) {
+    if (!(tot[0] == tot[0]) || isinf(g_next)) {
+      m.bad = 3;
+      m.stop = 0;
+    } else if (!(g_next > 0)) {
+      m.bad = 2;
+      m.stop = 0;
+    }
+    m.G = m.Eta = m.Eta0 = g_next;
+  } else {
+    const double g = m.G, c = m.C, c_prev = m.CPrev, s_prev = m.SPrev, s_cur = m.S;
+    const double a0 = c * dlt - c_prev * s_cur * g;
+    const double a1 = sqrt(a0 * a0 + g_next * g_next);
+    if (!isfinite(dlt) || !(tot[0] == tot[0]) || !isfinite(g_next) || !(a1 > 0)) {
+      m.bad = 1;
+      m.stop = m.k;
+    } else {
+      const double c_next = a0 / a1, s_next = g_next / a1;
+      update = true;
+      ia1 = (T)(1.0 / a1);
+      ta2 = (T)(s_cur * dlt + c_prev * c * g);
+      ta3 = (T)(s_prev * g);
+      tc = (T)(c_next * m.Eta);
+      tz = (T)(1.0 / g);
+      const double eta = -s_next * m.Eta;
+      m.Eta = eta;
+      m.CPrev = c;
+      m.C = c_next;
+      m.SPrev = s_cur;
+      m.S = s_next;
+      m.GPrev = g;
+      m.G = g_next;
+      if (fabs(eta) <= m.Rtol * m.Eta0 || g_next == 0 || m.k >= m.maxsteps) m.stop = m.k;
+    }
+  }
+  m.k++;
+  if (writer) *st_out = m;
+  if (update && own)
+#pragma unroll
+    for (int a = 0; a < BS; a++) {
+      const int64_t i = BS * r + a;
+      const T wn = (tz * up[a] - ta3 * wo[a] - ta2 * wc[a]) * ia1;
+      w_new[i] = wn;
+      x[i] = xo[a] + tc * wn;
+    }
+  if (m.stop >= 0) return;
+  const T inv = (T)(1.0 / m.G);
   T red[1] = {0};
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+  if (own)
+#pragma unroll
+    for (int a = 0; a < BS; a++) {
+      const T qa = inv * acc[a];
+      q[BS * r + a] = qa;
+      red[0] += qa * (inv * uo[a]);
+    }
+  block_partials<T, 1>(red, part_d);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_mr_lanczos(const T* __restrict__ q, const T* __restrict__ v,
+                                                    const T* __restrict__ v_old, T* __restrict__ v_new,
+                                                    T* __restrict__ u_new, const T* __restrict__ dinv, int64_t n,
+                                                    const MinresState* __restrict__ st, const double* __restrict__ part_d,
+                                                    unsigned g_d, double* __restrict__ delta,
+                                                    double* __restrict__ part_g, int xcd, unsigned g1, int bs) {
+  const int stop = st->stop;
+  const double g = st->G, g_prev = st->GPrev;
+  double pre[1][5];
+  partials_issue<1, 5>(part_d, g_d, pre);
+  if (stop >= 0) return;
+  int64_t e0, e1;
+  update_range(n, xcd, g1, bs, 256, e0, e1);
+  const int64_t i0 = e0 + threadIdx.x;
+  T qv[4], vv[4], ov[4], dv[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int64_t i = i0 + k * 256;
+    const bool in = i < e1;
+    qv[k] = in ? q[i] : (T)0;
+    vv[k] = in ? v[i] : (T)0;
+    ov[k] = in ? v_old[i] : (T)0;
+    dv[k] = dinv && in ? dinv[i] : (T)1;
+  }
+  double d[1];
+  partials_finish<1, 5>(part_d, g_d, pre, d);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *delta = d[0];
+  const T c1 = (T)(d[0] / g), c2 = g_prev > 0 ? (T)(g / g_prev) : (T)0;
+  T red[1] = {0};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int64_t i = i0 + k * 256;
+    if (i >= e1) continue;
+    const T vn = qv[k] - c1 * vv[k] - c2 * ov[k];
+    v_new[i] = vn;
+    const T un = dv[k] * vn;
+    u_new[i] = un;
+    red[0] += un * vn;
+  }
+  for (int64_t i = i0 + 1024; i < e1; i += 256) {  // chunks beyond 1,024 elements
     const T vn = q[i] - c1 * v[i] - c2 * v_old[i];
     v_new[i] = vn;
-    const T zn = dinv ? dinv[i] * vn : vn;
-    z_new[i] = zn;
-    red[0] += zn * vn;
+    const T un = dinv ? dinv[i] * vn : vn;
+    u_new[i] = un;
+    red[0] += un * vn;
   }
-  write_block_partials<T, 1>(red, partials);
-}
-// w_new = (z - a3 w_old - a2 w) / a1; x += (c eta) w_new; z_next *= 1/g_next
-template <typename T>
-__global__ __launch_bounds__(256) void k_minres_update(const T* __restrict__ z, const T* __restrict__ w,
-                                                       const T* __restrict__ w_old, T* __restrict__ w_new,
-                                                       T* __restrict__ x, T* __restrict__ z_next,
-                                                       const double* __restrict__ ms, int step, int64_t n) {
-  // steps after the stopping one, and a step whose rotation failed, change nothing
-  const double stop = ms[kMsStop];
-  if (stop >= 0.0 && ((double)step > stop || ms[kMsBad] != 0.0)) return;
-  const T ia1 = (T)(1.0 / ms[kMsA1]), ta2 = (T)ms[kMsA2], ta3 = (T)ms[kMsA3], tc = (T)ms[kMsCEta],
-          tg = (T)ms[kMsInvG];
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const T wn = (z[i] - ta3 * w_old[i] - ta2 * w[i]) * ia1;
-    w_new[i] = wn;
-    x[i] += tc * wn;
-    z_next[i] *= tg;
-  }
-}
-template <typename T>
-__global__ void k_scale_vec(T* __restrict__ a, double s, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    a[i] *= (T)s;
+  block_partials<T, 1>(red, part_g);
 }
 template <typename T>
 __global__ void k_minres_start(const T* __restrict__ r, T* __restrict__ v, T* __restrict__ z, const T* __restrict__ dinv,
@@ -755,6 +853,166 @@ __global__ void k_minres_start(const T* __restrict__ r, T* __restrict__ v, T* __
   }
   write_block_partials<T, 1>(red, partials);
 }
+
+template <typename T>
+struct MinresEngine {
+  mfs_mat A = nullptr;
+  int64_t n = 0;
+  const T *val = nullptr, *dinv = nullptr;
+  // rhs (then u), x, v[3], w[3], u, A z
+  T* buf[10] = {};
+  T *V[3] = {}, *W[3] = {}, *U[2] = {}, *x = nullptr, *q = nullptr;
+  MinresState* st = nullptr;  // two records, by step parity
+  double* delta = nullptr;
+  double* tot = nullptr;  // [z.q, u.v] summed by k_finish_sums when fin
+  ReduceScratch red;
+  unsigned g_spmv = 0, g_vec = 0;
+  bool fin = false, use_graph = true;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  static constexpr int kChunk = 12;  // steps per graph: a multiple of the buffers' period 6
+
+  double* part_d() { return red.partials; }
+  double* part_g() { return red.partials + g_spmv; }
+
+  int init(mfs_mat A_) {
+    A = A_;
+    n = A->n();
+    const bool f64 = std::is_same<T, double>::value;
+    if (!f64 && !A->val32_valid) MFS_TRY(mat_refresh_derived(A));
+    val = f64 ? (const T*)A->d_val64 : (const T*)A->d_val32;
+    dinv = f64 ? (const T*)A->d_dinv64 : (const T*)A->d_dinv32;
+    g_spmv = (unsigned)spmv_grid(A);
+    const int64_t cus = std::max(A->ctx->cu_count, 64);
+    g_vec = (unsigned)std::min<int64_t>(4 * cus, std::max<int64_t>(cus, (n + 1023) / 1024));
+    fin = (uint64_t)g_spmv * g_vec > 2000000ull;  // as the PCG: sum the partials once
+    if (const char* e = std::getenv("MFS_FINISH_SUMS")) fin = e[0] == '1';
+    for (T*& b : buf) MFS_TRY(dmalloc((void**)&b, sizeof(T) * n));
+    MFS_TRY(dmalloc((void**)&st, 2 * sizeof(MinresState)));
+    MFS_TRY(dmalloc((void**)&delta, 8 * sizeof(double)));
+    tot = delta + 4;
+    MFS_TRY(reduce_scratch_alloc(red, (int64_t)g_spmv + g_vec + 64));
+    U[1] = buf[0];
+    x = buf[1];
+    for (int k = 0; k < 3; k++) {
+      V[k] = buf[2 + k];
+      W[k] = buf[5 + k];
+    }
+    U[0] = buf[8];
+    q = buf[9];
+    const char* e = std::getenv("MFS_NO_GRAPH");
+    use_graph = !(e && e[0] == '1');
+    if (!use_graph) return MFS_OK;
+    hipStream_t s = A->ctx->stream;
+    MFS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    for (int t = 0; t < kChunk; t++) launch_step(s, t);
+    MFS_HIP(hipStreamEndCapture(s, &graph));
+    MFS_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    return MFS_OK;
+  }
+
+  template <int BS, typename CI>
+  void launch_spmv(hipStream_t s, int t, const CI* col) {
+    k_mr_spmv<T, BS, CI><<<g_spmv, 256, 0, s>>>(
+        A->d_slice_base, A->d_slice_width, col, val, U[t % 2], U[(t + 1) % 2], W[(t + 2) % 3], W[t % 3], W[(t + 1) % 3],
+        x, q, A->nb, A->sell.n_slices, st + t % 2, st + (t + 1) % 2, delta, fin ? tot + 1 : part_g(), fin ? 1u : g_vec,
+        part_d(), A->xcd_map);
+  }
+  void launch_step(hipStream_t s, int t) {
+    if (A->d_col16) {
+      if (A->bs == 1)
+        launch_spmv<1>(s, t, A->d_col16);
+      else
+        launch_spmv<3>(s, t, A->d_col16);
+    } else {
+      if (A->bs == 1)
+        launch_spmv<1>(s, t, A->d_col);
+      else
+        launch_spmv<3>(s, t, A->d_col);
+    }
+    if (fin) k_finish_sums<<<1, 256, 0, s>>>(part_d(), g_spmv, tot);
+    k_mr_lanczos<T><<<g_vec, 256, 0, s>>>(q, V[(t + 1) % 3], V[t % 3], V[(t + 2) % 3], U[(t + 1) % 2], dinv, n,
+                                          st + (t + 1) % 2, fin ? tot : part_d(), fin ? 1u : g_spmv, delta, part_g(),
+                                          A->xcd_map, g_spmv, A->bs);
+    if (fin) k_finish_sums<<<1, 256, 0, s>>>(part_g(), g_vec, tot + 1);
+  }
+
+  // One run on A d = rhs (rhs in buf[0], d returned in buf[1]) to relative
+  // (M^-1-norm) tolerance rtol or maxsteps.
+  int run(double rtol, int maxsteps, int* steps, double* est_rel) {
+    hipStream_t s = A->ctx->stream;
+    k_minres_start<T><<<g_vec, 256, 0, s>>>(buf[0], V[1], U[0], dinv, x, V[0], W[1], W[0], n, part_g());
+    k_mr_init<<<1, 64, 0, s>>>(st, rtol, maxsteps);
+    if (fin) k_finish_sums<<<1, 256, 0, s>>>(part_g(), g_vec, tot + 1);
+    MFS_HIP(hipGetLastError());
+    for (hipEvent_t& e : ev)
+      if (!e) MFS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    MinresState* hs = (MinresState*)A->ctx->pinned;
+    auto submit = [&](int slot) -> int {
+      if (use_graph) {
+        MFS_HIP(hipGraphLaunch(exec, s));
+      } else {
+        for (int t = 0; t < kChunk; t++) launch_step(s, t);
+        MFS_HIP(hipGetLastError());
+      }
+      MFS_HIP(hipMemcpyAsync(hs + slot, st, sizeof(MinresState), hipMemcpyDeviceToHost, s));  // kChunk is even
+      MFS_HIP(hipEventRecord(ev[slot], s));
+      return MFS_OK;
+    };
+    // while the estimate is far above the tolerance the next chunk is queued
+    // before the host waits for this one
+    int head = 0, inflight = 1;
+    bool ahead = false;
+    MFS_TRY(submit(0));
+    for (;;) {
+      if (ahead && inflight == 1) {
+        MFS_TRY(submit(head ^ 1));
+        inflight = 2;
+      }
+      MFS_HIP(hipEventSynchronize(ev[head]));
+      inflight--;
+      const MinresState& m = hs[head];
+      if (m.stop >= 0) break;
+      ahead = std::fabs(m.Eta) > 2.0 * m.Rtol * m.Eta0 && m.k + kChunk < m.maxsteps;
+      head ^= 1;
+      if (inflight == 0) {
+        MFS_TRY(submit(head));
+        inflight = 1;
+      }
+    }
+    const MinresState m = hs[head];
+    if (inflight) MFS_HIP(hipStreamSynchronize(s));
+    if (m.bad == 1 || m.bad == 3) return MFS_ERR_NONFINITE;
+    if (m.bad == 2) {
+      *est_rel = 0.0;
+      return MFS_OK;
+    }
+    *steps += m.stop;
+    *est_rel = std::fabs(m.Eta) / m.Eta0;
+    return MFS_OK;
+  }
+
+  void destroy() {
+    if (exec) (void)hipGraphExecDestroy(exec);
+    if (graph) (void)hipGraphDestroy(graph);
+    exec = nullptr;
+    graph = nullptr;
+    for (hipEvent_t& e : ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    for (T*& b : buf) {
+      dfree(b);
+      b = nullptr;
+    }
+    dfree(st);
+    dfree(delta);
+    st = nullptr;
+    delta = nullptr;
+    reduce_scratch_free(red);
+  }
+};
 
 // ---------------------------------------------------------------------------
 // BiCGStab with right Jacobi preconditioning (van der Vorst 1992; the
@@ -1196,8 +1454,8 @@ struct mfs_solver_s {
   PcgEngine<float> cg32;
   bool has64 = false, has32 = false;
   // GMRES
-  // MINRES vectors: rhs / z_next, x, v[3], w[3], z, A z
-  void* mr[10] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  MinresEngine<double> mr64;
+  MinresEngine<float> mr32;
   void* V = nullptr;   // (m+1) * n in the inner precision
   void* w = nullptr;
   void* z = nullptr;
@@ -1232,7 +1490,8 @@ extern "C" int mfs_solver_destroy(mfs_solver S) {
   dfree(S->b64);
   dfree(S->r64);
   dfree(S->dout);
-  for (void* v : S->mr) dfree(v);
+  S->mr64.destroy();
+  S->mr32.destroy();
   dfree(S->V);
   dfree(S->w);
   dfree(S->z);
@@ -1282,11 +1541,12 @@ extern "C" int mfs_solver_create(mfs_mat A, const mfs_solve_desc* desc, mfs_solv
     else
       tryit(S->bs32.init(A, true));
   } else if (desc->method == MFS_MINRES) {
-    const size_t sv = desc->precision == MFS_PREC_F64 ? 8 : 4;
-    if (desc->precision == MFS_PREC_MIXED && !A->val32_valid) tryit(mat_refresh_derived(A));
-    for (void*& v : S->mr) tryit(dmalloc(&v, sv * n));
-    tryit(dmalloc((void**)&S->dh, 8 * 64));
-    if (s == MFS_OK) tryit(reduce_scratch_alloc(S->redg, 2 * 1024 + 64));
+    if (s == MFS_OK) {
+      if (desc->precision == MFS_PREC_F64)
+        tryit(S->mr64.init(A));
+      else
+        tryit(S->mr32.init(A));
+    }
   } else if (desc->method != MFS_GMRES) {
     if (s == MFS_OK && desc->precision == MFS_PREC_F64) {
       S->has64 = true;
@@ -1498,95 +1758,6 @@ static int gmres_cycle(mfs_solver S, const T* val, const T* dinv, T* rhs, double
   return MFS_OK;
 }
 
-// One MINRES run on A d = rhs (rhs in mr[0]; d returned in mr[1]), to
-// relative (M^-1-norm) tolerance rtol or maxsteps.  Returns the steps taken.
-template <typename T>
-static int minres_run(mfs_solver S, const T* dinv, double rtol, int maxsteps, int* steps, double* est_rel) {
-  hipStream_t s = S->A->ctx->stream;
-  mfs_mat A = S->A;
-  const int64_t n = S->n;
-  const int prec = std::is_same<T, double>::value ? MFS_F64 : MFS_F32;
-  T* rhs = (T*)S->mr[0];
-  T* x = (T*)S->mr[1];
-  T* v[3] = {(T*)S->mr[2], (T*)S->mr[3], (T*)S->mr[4]};  // v_{j-1}, v_j, v_{j+1}
-  T* w[3] = {(T*)S->mr[5], (T*)S->mr[6], (T*)S->mr[7]};  // w_{j-1}, w_j, w_{j+1}
-  T* zbuf[2] = {(T*)S->mr[8], nullptr};
-  T* Az = (T*)S->mr[9];
-  for (void* b : S->mr)
-    if (!b) {
-      set_error("minres: work vector not allocated");
-      return MFS_ERR_ARG;
-    }
-  if (!S->dh || !S->redg.partials) {
-    set_error("minres: reduction scratch not allocated");
-    return MFS_ERR_ARG;
-  }
-  const unsigned gv = grid_for(n, 1024);
-  double* hp = (double*)A->ctx->pinned;
-  // z buffers: z_j in zbuf[0]; z_{j+1} in the spare v slot is not possible,
-  // so z_{j+1} goes to rhs (rhs is consumed by the start kernel).
-  T* zj = zbuf[0];
-  T* znext = rhs;
-  k_minres_start<T><<<gv, 256, 0, s>>>(rhs, v[1], zj, dinv, x, v[0], w[1], w[0], n, S->redg.partials);
-  k_finish_sums<<<1, 256, 0, s>>>(S->redg.partials, gv, S->dh);
-  MFS_HIP(hipMemcpyAsync(hp, S->dh, 8, hipMemcpyDeviceToHost, s));
-  MFS_HIP(hipStreamSynchronize(s));
-  const double g = std::sqrt(std::max(hp[0], 0.0));
-  if (!(g > 0) || !std::isfinite(g)) {
-    *est_rel = std::isfinite(g) ? 0.0 : 1.0;
-    return std::isfinite(g) ? MFS_OK : MFS_ERR_NONFINITE;
-  }
-  // recurrence state on the device; the host checks it every kSync steps
-  // (steps launched past the stopping one leave x unchanged)
-  constexpr int kSync = 8;
-  double* ms = S->dh + 8;
-  {
-    double init[kMsCount] = {};
-    init[kMsG] = g;
-    init[kMsC] = init[kMsCPrev] = 1.0;
-    init[kMsEta] = init[kMsEta0] = g;
-    init[kMsRtol] = rtol;
-    init[kMsStop] = -1.0;
-    for (int q = 0; q < kMsCount; q++) hp[q] = init[q];
-    MFS_HIP(hipMemcpyAsync(ms, hp, sizeof(double) * kMsCount, hipMemcpyHostToDevice, s));
-  }
-  k_scale_vec<T><<<gv, 256, 0, s>>>(zj, 1.0 / g, n);
-  int j = 0;
-  double stop = -1.0, bad = 0.0;
-  while (j < maxsteps && stop < 0.0) {
-    const int nb = std::min(kSync, maxsteps - j);
-    for (int t = 0; t < nb; t++, j++) {
-      MFS_TRY(spmv_launch(A, prec, zj, Az, s));
-      // delta = <A z_j, z_j>
-      k_multidot<T><<<dim3(gv, 1), 256, 0, s>>>(zj, Az, n, S->redg.partials);
-      k_finish_sums<<<1, 256, 0, s>>>(S->redg.partials, gv, S->dh + 1);
-      k_minres_lanczos<T><<<gv, 256, 0, s>>>(Az, v[1], v[0], v[2], znext, dinv, S->dh + 1, ms, n,
-                                             S->redg.partials);
-      k_finish_sums<<<1, 256, 0, s>>>(S->redg.partials, gv, S->dh + 2);
-      k_minres_rot<<<1, 64, 0, s>>>(S->dh, ms, j);
-      k_minres_update<T><<<gv, 256, 0, s>>>(zj, w[1], w[0], w[2], x, znext, ms, j, n);
-      // rotate the buffers: v_{j-1} <- v_j, v_j <- v_{j+1} (the same for w), z
-      std::swap(v[0], v[1]);
-      std::swap(v[1], v[2]);
-      std::swap(w[0], w[1]);
-      std::swap(w[1], w[2]);
-      std::swap(zj, znext);
-    }
-    MFS_HIP(hipGetLastError());
-    MFS_HIP(hipMemcpyAsync(hp, ms, sizeof(double) * kMsCount, hipMemcpyDeviceToHost, s));
-    MFS_HIP(hipStreamSynchronize(s));
-    stop = hp[kMsStop];
-    bad = hp[kMsBad];
-  }
-  if (bad != 0.0) return MFS_ERR_NONFINITE;
-  if (stop >= 0.0) j = (int)stop + 1;
-  const double eta = hp[kMsEta], eta0 = hp[kMsEta0];
-  // the correction must end in mr[1]: x never moves
-  *steps += j;
-  *est_rel = std::fabs(eta) / eta0;
-  return MFS_OK;
-}
-
 __global__ void k_add_f64(double* __restrict__ x, const double* __restrict__ u, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     x[i] += u[i];
@@ -1748,15 +1919,14 @@ extern "C" int mfs_solver_run(mfs_solver S, mfs_vec b, mfs_vec x, mfs_solve_repo
       double est = 1;
       int steps = 0, st2;
       if (d.precision == MFS_PREC_F64) {
-        MFS_HIP(hipMemcpyAsync(S->mr[0], S->r64, 8 * n, hipMemcpyDeviceToDevice, s));
-        st2 = minres_run<double>(S, A->d_dinv64, 0.5 * d.tol * std::sqrt(bb) / rn, d.maxit - iters, &steps, &est);
-        if (st2 == MFS_OK) k_add_f64<<<gv, 256, 0, s>>>(S->x64, (const double*)S->mr[1], n);
+        MFS_HIP(hipMemcpyAsync(S->mr64.buf[0], S->r64, 8 * n, hipMemcpyDeviceToDevice, s));
+        st2 = S->mr64.run(0.5 * d.tol * std::sqrt(bb) / rn, d.maxit - iters, &steps, &est);
+        if (st2 == MFS_OK) k_add_f64<<<gv, 256, 0, s>>>(S->x64, S->mr64.x, n);
       } else {
-        float* dummy = (float*)S->mr[2];
-        k_demote_scaled<<<gv, 256, 0, s>>>(S->r64, 1.0 / rn, (float*)S->mr[0], dummy, n);
+        k_demote_scaled<<<gv, 256, 0, s>>>(S->r64, 1.0 / rn, S->mr32.buf[0], S->mr32.x, n);
         const double itol = std::min(0.5, std::max(d.inner_tol, 0.5 * d.tol / rel));
-        st2 = minres_run<float>(S, A->d_dinv32, itol, d.maxit - iters, &steps, &est);
-        if (st2 == MFS_OK) k_promote_add<<<gv, 256, 0, s>>>(S->x64, (const float*)S->mr[1], nullptr, rn, n);
+        st2 = S->mr32.run(itol, d.maxit - iters, &steps, &est);
+        if (st2 == MFS_OK) k_promote_add<<<gv, 256, 0, s>>>(S->x64, S->mr32.x, nullptr, rn, n);
       }
       if (st2 != MFS_OK) {
         status = st2;

@@ -144,12 +144,12 @@ __device__ __forceinline__ unsigned xcd_block(int on) {
 }
 
 // Element range [e0, e1) of this block of a vector-update kernel that
-// feeds a SELL kernel of grid g1 (256 block rows of bs elements per block).
+// feeds a SELL kernel of grid g1 (rpb elements of the vector per block).
 // With the XCD slice order (xcd = 1) the update blocks running on XCD x
 // split the rows that the SELL kernel's blocks on XCD x own, so the values
 // written are gathered next from the same L2; otherwise equal contiguous
 // chunks.  Chunks are multiples of gran elements.
-__device__ __forceinline__ void update_range(int64_t n, int xcd, unsigned g1, int bs, int gran, int64_t& e0,
+__device__ __forceinline__ void update_range(int64_t n, int xcd, unsigned g1, int rpb, int gran, int64_t& e0,
                                              int64_t& e1) {
   const unsigned G = gridDim.x, b = blockIdx.x;
   if (!xcd || G < 8) {
@@ -161,7 +161,7 @@ __device__ __forceinline__ void update_range(int64_t n, int xcd, unsigned g1, in
   const unsigned x = b & 7u, k = b >> 3, cnt = (G - x + 7) / 8;
   const unsigned per = g1 >> 3, rem = g1 & 7u;
   const int64_t s1 = (int64_t)x * per + min(x, rem), c1 = per + (x < rem ? 1 : 0);
-  const int64_t r0 = min(n, s1 * 256 * bs), r1 = min(n, (s1 + c1) * 256 * bs);
+  const int64_t r0 = min(n, s1 * rpb), r1 = min(n, (s1 + c1) * rpb);
   const int64_t chunk = ((r1 - r0 + cnt - 1) / cnt + gran - 1) / gran * gran;
   e0 = min(r1, r0 + (int64_t)k * chunk);
   e1 = min(r1, e0 + chunk);
@@ -279,6 +279,46 @@ __device__ __forceinline__ void sell_row_pair(int64_t sb, int w, const CI* __res
   }
 }
 
+// Component a of the block row product of sell_row_x<T, 3>, with the same
+// operations in the same order.  A lane holds 3 of an entry's 9 values, so U
+// can be larger: fewer, wider latencies per row.
+template <typename T, int U, typename XL, typename CI>
+__device__ __forceinline__ T sell_row_component(const int64_t* __restrict__ slice_base,
+                                                const int32_t* __restrict__ slice_width, const CI* __restrict__ col,
+                                                const T* __restrict__ val, int64_t slice, int lane, int a, XL xl) {
+  constexpr int C = 64;
+  T acc = 0;
+  const int64_t sb = slice_base[slice];
+  const int w = slice_width[slice];
+  const CI* cp = col + sb + lane;
+  const int32_t rbase = sizeof(CI) == 2 ? (int32_t)(slice * C + lane) : 0;
+  const T* vp = val + sb * 9 + 3 * a * C + lane;
+  for (int j0 = 0; j0 < w; j0 += U) {
+    int32_t c[U];
+    T v[U][3];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int j = min(j0 + u, w - 1);
+      const bool in = j0 + u < w;
+      c[u] = (int32_t)cp[(int64_t)j * C] + rbase;  // read by three waves: through the caches
+#pragma unroll
+      for (int e = 0; e < 3; e++) {
+        const T t = __builtin_nontemporal_load(vp + ((int64_t)j * 9 + e) * C);
+        v[u][e] = in ? t : (T)0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      T xv[3];
+#pragma unroll
+      for (int b = 0; b < 3; b++) xv[b] = xl((int64_t)3 * c[u] + b);
+#pragma unroll
+      for (int b = 0; b < 3; b++) acc += v[u][b] * xv[b];
+    }
+  }
+  return acc;
+}
+
 template <typename T, int BS, typename CI>
 __device__ __forceinline__ void sell_row(const int64_t* __restrict__ slice_base, const int32_t* __restrict__ slice_width,
                                          const CI* __restrict__ col, const T* __restrict__ val,
@@ -292,6 +332,9 @@ int spmv_dot_launch(mfs_mat A, int prec, const void* x, void* y, double* partial
 int spmv_residual_launch(mfs_mat A, int prec, const void* x, void* r, const void* b, double* partials,
                          unsigned* counter, double* out, hipStream_t s);
 int64_t spmv_grid(mfs_mat A);
+// The iteration kernels' form for small systems of 3x3 blocks: one slice per
+// block, a wave per component, instead of a wave per slice.
+bool sell_component_waves(mfs_mat A, bool f64);
 }  // namespace mfs
 
 // Fence-free two-stage reductions: a kernel writes one partial per block and

@@ -703,6 +703,19 @@ int spmv_residual_launch(mfs_mat A, int prec, const void* x, void* r, const void
   return spmv_mode_launch<2>(A, prec, x, r, b, partials, counter, out, s);
 }
 int64_t spmv_grid(mfs_mat A) { return (A->sell.n_slices + 3) / 4; }
+
+// A wave per component while a wave per slice leaves the chip without enough
+// waves to hide a row's chain of index, gather and value latencies.  us per
+// PCG iteration, a wave per slice -> a wave per component, over the slices:
+//   FP32:  77 12.5 -> 10.7   145 12.0 ->  9.8 (MINRES)   562 13.9 -> 14.4
+//   FP64:  77 18.2 -> 12.5   245 22.0 -> 12.7           1077 37.3 -> 32.0
+//        2073 54.5 -> 54.8  3547 78.5 -> 92.6
+// Past the line the operand gathers, made three times, cost more.
+bool sell_component_waves(mfs_mat A, bool f64) {
+  if (A->bs != 3) return false;
+  if (const char* e = std::getenv("MFS_COMPONENT_WAVES")) return e[0] == '1';  // force either way (tests)
+  return A->sell.n_slices <= (f64 ? 1200 : 400);
+}
 }  // namespace mfs
 
 extern "C" int mfs_spmv(mfs_mat A, int prec, mfs_vec x, mfs_vec y) {

@@ -92,6 +92,25 @@ __device__ __forceinline__ void block_partials(T (&v)[NV], double* __restrict__ 
         (red[threadIdx.x][0] + red[threadIdx.x][1]) + (red[threadIdx.x][2] + red[threadIdx.x][3]);
 }
 
+// a.b of a block row from its components' waves, added in the order that a
+// thread with all of them has: v holds component `wave`'s pair; the sum goes
+// to wave 0, zero to the others.
+template <typename T>
+__device__ __forceinline__ void component_dot(const T (&v)[2], T& dot) {
+  __shared__ T ex[2][2][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (wave == 1 || wave == 2)
+    for (int k = 0; k < 2; k++) ex[wave - 1][k][lane] = v[k];
+  __syncthreads();
+  if (wave == 0) {
+    dot += ex[0][0][lane] * ex[0][1][lane];
+    dot += ex[1][0][lane] * ex[1][1][lane];
+  } else {
+    dot = 0;
+  }
+}
+constexpr int kCompGroup = 9;  // entries per latency of sell_row_component
+
 // K1: from K2's partials (r.z, r.r): stop test, beta = rz / rz_prev;
 // p_new = z + beta p_old (own rows written), q = A p_new, per-block partial
 // of p_new.q.  Scalar rows compute q = A z + beta A p_old (both products in
@@ -99,7 +118,11 @@ __device__ __forceinline__ void block_partials(T (&v)[NV], double* __restrict__ 
 // issued while the partials of the previous kernel are still in flight.
 // 3x3 blocks form p_new on the fly for the gathered columns once beta is
 // known (two operand gathers per block column would cost 30 more registers).
-template <typename T, int BS, typename CI>
+//
+// CW (sell_component_waves): a block computes one slice, wave a < 3 its
+// component a, by the operations of the other form in the same order (only
+// the partials' FP64 sums are regrouped).
+template <typename T, int BS, bool CW, typename CI>
 __global__ __launch_bounds__(256) void k_cg_dir_spmv(const int64_t* __restrict__ slice_base,
                                                      const int32_t* __restrict__ slice_width,
                                                      const CI* __restrict__ col, const T* __restrict__ val,
@@ -107,10 +130,14 @@ __global__ __launch_bounds__(256) void k_cg_dir_spmv(const int64_t* __restrict__
                                                      T* __restrict__ p_new, T* __restrict__ q, int64_t nb,
                                                      int64_t n_slices, CgState* st, const double* __restrict__ part_rz,
                                                      unsigned g_rz, double* __restrict__ part_pq, int xcd) {
+  constexpr int NA = CW ? 1 : BS;
   const int was_done = st->done;
-  const int64_t slice = (int64_t)xcd_block(xcd) * 4 + threadIdx.x / 64;
+  const int wave = threadIdx.x / 64;
+  const int64_t slice = CW ? (int64_t)xcd_block(xcd) : (int64_t)xcd_block(xcd) * 4 + wave;
   const int lane = threadIdx.x & 63;
   const int64_t r = slice * 64 + lane;
+  const int a0 = CW ? wave : 0;
+  const bool own = r < nb && (!CW || wave < BS);
   // the slice's start and width are loaded with the stop flag and the
   // partials, ahead of the branch on the flag
   const bool in_range = slice < n_slices;
@@ -119,12 +146,12 @@ __global__ __launch_bounds__(256) void k_cg_dir_spmv(const int64_t* __restrict__
   double pre[2][2];
   partials_issue<2, 2>(part_rz, g_rz, pre);
   if (was_done) return;
-  T az[BS], ap[BS], zo[BS], po[BS];
+  T az[NA], ap[NA], zo[NA], po[NA];
 #pragma unroll
-  for (int a = 0; a < BS; a++) az[a] = ap[a] = zo[a] = po[a] = 0;
+  for (int a = 0; a < NA; a++) az[a] = ap[a] = zo[a] = po[a] = 0;
   if constexpr (BS == 1) {
     sell_row_pair<T, BS>(sb, w, col, val, z, p_old, slice, lane, az, ap);
-    if (r < nb) {
+    if (own) {
       zo[0] = z[r];
       po[0] = p_old[r];
     }
@@ -152,29 +179,37 @@ __global__ __launch_bounds__(256) void k_cg_dir_spmv(const int64_t* __restrict__
   if (done != CG_RUN) return;
   if constexpr (BS != 1) {
     // az = A p_new with the operand z_j + beta p_j formed on the fly
-    if (slice < n_slices)
-      sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb,
-                        [&](int64_t i) { return z[i] + beta * p_old[i]; }, az);
-    if (r < nb) {
+    if (own) {
 #pragma unroll
-      for (int a = 0; a < BS; a++) {
-        zo[a] = z[BS * r + a];
-        po[a] = p_old[BS * r + a];
+      for (int a = 0; a < NA; a++) {
+        zo[a] = z[BS * r + a0 + a];
+        po[a] = p_old[BS * r + a0 + a];
       }
     }
+    if constexpr (CW) {
+      if (wave < BS)
+        az[0] = sell_row_component<T, kCompGroup>(slice_base, slice_width, col, val, slice, lane, wave,
+                                                  [&](int64_t i) { return z[i] + beta * p_old[i]; });
+    } else if (slice < n_slices) {
+      sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb,
+                        [&](int64_t i) { return z[i] + beta * p_old[i]; }, az);
+    }
   }
-  T red[1] = {0};
-  if (r < nb) {
+  T red[1] = {0}, pq[2] = {0, 0};
+  if (own) {
 #pragma unroll
-    for (int a = 0; a < BS; a++) {
-      const int64_t i = BS * r + a;
+    for (int a = 0; a < NA; a++) {
+      const int64_t i = BS * r + a0 + a;
       const T pn = zo[a] + beta * po[a];
       const T qa = az[a] + beta * ap[a];
       p_new[i] = pn;
       q[i] = qa;
       red[0] += qa * pn;
+      pq[0] = qa;
+      pq[1] = pn;
     }
   }
+  if constexpr (CW) component_dot(pq, red[0]);
   block_partials<T, 1>(red, part_pq);
 }
 
@@ -186,14 +221,14 @@ __global__ __launch_bounds__(256) void k_cg_update(T* __restrict__ x, const T* _
                                                    T* __restrict__ z, const T* __restrict__ q,
                                                    const T* __restrict__ dinv, int64_t n, CgState* st,
                                                    const double* __restrict__ part_pq, unsigned g_pq,
-                                                   double* __restrict__ part_rz, int xcd, unsigned g1, int bs) {
+                                                   double* __restrict__ part_rz, int xcd, unsigned g1, int rpb) {
   const int was_done = st->done;
   const double rz = st->rz1;
   double pre[1][5];
   partials_issue<1, 5>(part_pq, g_pq, pre);
   if (was_done) return;
   int64_t e0, e1;
-  update_range(n, xcd, g1, bs, 256, e0, e1);
+  update_range(n, xcd, g1, rpb, 256, e0, e1);
   const int64_t i0 = e0 + threadIdx.x;
   // first pass: four elements per thread, loaded together
   T xv[4], pv[4], rv[4], qv[4], dv[4];
@@ -349,6 +384,8 @@ struct PcgEngine {
   CgState* st = nullptr;
   ReduceScratch red;
   unsigned g_spmv = 0, g_vec = 0;
+  bool split = false;  // K1: one slice per block (sell_component_waves)
+  int rpb = 0;         // vector elements per block of K1
   int chunk = 16;
   bool use_graph = true;
   // external buffers (mfs_solve_noalloc): no graph, no events; the host
@@ -384,7 +421,9 @@ struct PcgEngine {
     if (!f64 && !A->val32_valid) MFS_TRY(mat_refresh_derived(A));
     val = f64 ? (const T*)A->d_val64 : (const T*)A->d_val32;
     dinv = precond ? (f64 ? (const T*)A->d_dinv64 : (const T*)A->d_dinv32) : nullptr;
-    g_spmv = (unsigned)spmv_grid(A);
+    split = sell_component_waves(A, std::is_same<T, double>::value);
+    g_spmv = (unsigned)(split ? A->sell.n_slices : spmv_grid(A));
+    rpb = A->bs * (split ? 64 : 256);
     // update-kernel grid: about 4 elements per thread (its loop keeps 4 in
     // flight) but at least one block per CU; fewer blocks also means fewer
     // partial sums for every block of the next kernel to add up
@@ -428,26 +467,18 @@ struct PcgEngine {
 
   // K1 with 16-bit row-relative columns when the matrix has them
   void launch_k1(hipStream_t s, T* p_old, T* p_new) {
-    const int64_t ns = A->sell.n_slices;
-    if (A->d_col16) {
-      if (A->bs == 1)
-        k_cg_dir_spmv<T, 1, int16_t><<<g_spmv, 256, 0, s>>>(A->d_slice_base, A->d_slice_width, A->d_col16, val, z,
-                                                            p_old, p_new, q, A->nb, ns, st, rz_src(), rz_g(),
-                                                            part_pq(), A->xcd_map);
-      else
-        k_cg_dir_spmv<T, 3, int16_t><<<g_spmv, 256, 0, s>>>(A->d_slice_base, A->d_slice_width, A->d_col16, val, z,
-                                                            p_old, p_new, q, A->nb, ns, st, rz_src(), rz_g(),
-                                                            part_pq(), A->xcd_map);
-    } else {
-      if (A->bs == 1)
-        k_cg_dir_spmv<T, 1, int32_t><<<g_spmv, 256, 0, s>>>(A->d_slice_base, A->d_slice_width, A->d_col, val, z,
-                                                            p_old, p_new, q, A->nb, ns, st, rz_src(), rz_g(),
-                                                            part_pq(), A->xcd_map);
-      else
-        k_cg_dir_spmv<T, 3, int32_t><<<g_spmv, 256, 0, s>>>(A->d_slice_base, A->d_slice_width, A->d_col, val, z,
-                                                            p_old, p_new, q, A->nb, ns, st, rz_src(), rz_g(),
-                                                            part_pq(), A->xcd_map);
-    }
+    if (A->d_col16)
+      A->bs == 1 ? launch_k1<1>(s, p_old, p_new, A->d_col16) : launch_k1<3>(s, p_old, p_new, A->d_col16);
+    else
+      A->bs == 1 ? launch_k1<1>(s, p_old, p_new, A->d_col) : launch_k1<3>(s, p_old, p_new, A->d_col);
+  }
+  template <int BS, typename CI>
+  void launch_k1(hipStream_t s, T* p_old, T* p_new, const CI* col) {
+    auto kern = k_cg_dir_spmv<T, BS, false, CI>;
+    if constexpr (BS == 3)
+      if (split) kern = k_cg_dir_spmv<T, BS, true, CI>;
+    kern<<<g_spmv, 256, 0, s>>>(A->d_slice_base, A->d_slice_width, col, val, z, p_old, p_new, q, A->nb,
+                                A->sell.n_slices, st, rz_src(), rz_g(), part_pq(), A->xcd_map);
   }
 
   void launch_iteration(hipStream_t s, int parity) {
@@ -456,7 +487,7 @@ struct PcgEngine {
     launch_k1(s, p_old, p_new);
     finish_pq(s);
     k_cg_update<T><<<g_vec, 256, 0, s>>>(x, p_new, r, z, q, dinv, n, st, pq_src(), pq_g(), part_rz(), A->xcd_map,
-                                         g_spmv, A->bs);
+                                         g_spmv, rpb);
     finish_rz(s);
   }
 
@@ -682,7 +713,7 @@ __global__ void k_mr_init(MinresState* st, double rtol, int maxsteps) {
   *st = m;
 }
 
-template <typename T, int BS, typename CI>
+template <typename T, int BS, bool CW, typename CI>
 __global__ __launch_bounds__(256) void k_mr_spmv(const int64_t* __restrict__ slice_base,
                                                  const int32_t* __restrict__ slice_width,
                                                  const CI* __restrict__ col, const T* __restrict__ val,
@@ -701,27 +732,35 @@ __global__ __launch_bounds__(256) void k_mr_spmv(const int64_t* __restrict__ sli
     if (writer) *st_out = m;
     return;
   }
-  const int64_t slice = (int64_t)xcd_block(xcd) * 4 + threadIdx.x / 64;
+  constexpr int NA = CW ? 1 : BS;  // CW: as in k_cg_dir_spmv
+  const int wave = threadIdx.x / 64;
+  const int64_t slice = CW ? (int64_t)xcd_block(xcd) : (int64_t)xcd_block(xcd) * 4 + wave;
   const int lane = threadIdx.x & 63;
   const int64_t r = slice * 64 + lane;
-  const bool own = r < nb;
+  const int a0 = CW ? wave : 0;
+  const bool own = r < nb && (!CW || wave < BS);
   const double dlt = *delta;
   // everything that does not depend on the scalars is loaded first
-  T acc[BS], uo[BS], up[BS], wo[BS], wc[BS], xo[BS];
+  T acc[NA], uo[NA], up[NA], wo[NA], wc[NA], xo[NA];
 #pragma unroll
-  for (int a = 0; a < BS; a++) acc[a] = uo[a] = up[a] = wo[a] = wc[a] = xo[a] = 0;
+  for (int a = 0; a < NA; a++) acc[a] = uo[a] = up[a] = wo[a] = wc[a] = xo[a] = 0;
   if (own)
 #pragma unroll
-    for (int a = 0; a < BS; a++) {
-      const int64_t i = BS * r + a;
+    for (int a = 0; a < NA; a++) {
+      const int64_t i = BS * r + a0 + a;
       uo[a] = u[i];
       up[a] = u_prev[i];
       wo[a] = w_old[i];
       wc[a] = w[i];
       xo[a] = x[i];
     }
-  if (slice < n_slices)
+  if constexpr (CW) {
+    if (wave < BS)
+      acc[0] = sell_row_component<T, kCompGroup>(slice_base, slice_width, col, val, slice, lane, wave,
+                                                 [&](int64_t i) { return u[i]; });
+  } else if (slice < n_slices) {
     sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb, [&](int64_t i) { return u[i]; }, acc);
+  }
   double tot[1];
   partials_finish<1, 4>(part_g, g_g, pre, tot);
   const double g_next = sqrt(fmax(tot[0], 0.0));
@@ -767,22 +806,25 @@ __global__ __launch_bounds__(256) void k_mr_spmv(const int64_t* __restrict__ sli
   if (writer) *st_out = m;
   if (update && own)
 #pragma unroll
-    for (int a = 0; a < BS; a++) {
-      const int64_t i = BS * r + a;
+    for (int a = 0; a < NA; a++) {
+      const int64_t i = BS * r + a0 + a;
       const T wn = (tz * up[a] - ta3 * wo[a] - ta2 * wc[a]) * ia1;
       w_new[i] = wn;
       x[i] = xo[a] + tc * wn;
     }
   if (m.stop >= 0) return;
   const T inv = (T)(1.0 / m.G);
-  T red[1] = {0};
+  T red[1] = {0}, qz[2] = {0, 0};
   if (own)
 #pragma unroll
-    for (int a = 0; a < BS; a++) {
+    for (int a = 0; a < NA; a++) {
       const T qa = inv * acc[a];
-      q[BS * r + a] = qa;
+      q[BS * r + a0 + a] = qa;
       red[0] += qa * (inv * uo[a]);
+      qz[0] = qa;
+      qz[1] = inv * uo[a];
     }
+  if constexpr (CW) component_dot(qz, red[0]);
   block_partials<T, 1>(red, part_d);
 }
 
@@ -792,14 +834,14 @@ __global__ __launch_bounds__(256) void k_mr_lanczos(const T* __restrict__ q, con
                                                     T* __restrict__ u_new, const T* __restrict__ dinv, int64_t n,
                                                     const MinresState* __restrict__ st, const double* __restrict__ part_d,
                                                     unsigned g_d, double* __restrict__ delta,
-                                                    double* __restrict__ part_g, int xcd, unsigned g1, int bs) {
+                                                    double* __restrict__ part_g, int xcd, unsigned g1, int rpb) {
   const int stop = st->stop;
   const double g = st->G, g_prev = st->GPrev;
   double pre[1][5];
   partials_issue<1, 5>(part_d, g_d, pre);
   if (stop >= 0) return;
   int64_t e0, e1;
-  update_range(n, xcd, g1, bs, 256, e0, e1);
+  update_range(n, xcd, g1, rpb, 256, e0, e1);
   const int64_t i0 = e0 + threadIdx.x;
   T qv[4], vv[4], ov[4], dv[4];
 #pragma unroll
@@ -867,7 +909,7 @@ struct MinresEngine {
   double* tot = nullptr;  // [z.q, u.v] summed by k_finish_sums when fin
   ReduceScratch red;
   unsigned g_spmv = 0, g_vec = 0;
-  bool fin = false, use_graph = true;
+  bool fin = false, use_graph = true, split = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[2] = {nullptr, nullptr};
@@ -883,7 +925,8 @@ struct MinresEngine {
     if (!f64 && !A->val32_valid) MFS_TRY(mat_refresh_derived(A));
     val = f64 ? (const T*)A->d_val64 : (const T*)A->d_val32;
     dinv = f64 ? (const T*)A->d_dinv64 : (const T*)A->d_dinv32;
-    g_spmv = (unsigned)spmv_grid(A);
+    split = sell_component_waves(A, std::is_same<T, double>::value);
+    g_spmv = (unsigned)(split ? A->sell.n_slices : spmv_grid(A));
     const int64_t cus = std::max(A->ctx->cu_count, 64);
     g_vec = (unsigned)std::min<int64_t>(4 * cus, std::max<int64_t>(cus, (n + 1023) / 1024));
     fin = (uint64_t)g_spmv * g_vec > 2000000ull;  // as the PCG: sum the partials once
@@ -914,7 +957,10 @@ struct MinresEngine {
 
   template <int BS, typename CI>
   void launch_spmv(hipStream_t s, int t, const CI* col) {
-    k_mr_spmv<T, BS, CI><<<g_spmv, 256, 0, s>>>(
+    auto kern = k_mr_spmv<T, BS, false, CI>;
+    if constexpr (BS == 3)
+      if (split) kern = k_mr_spmv<T, BS, true, CI>;
+    kern<<<g_spmv, 256, 0, s>>>(
         A->d_slice_base, A->d_slice_width, col, val, U[t % 2], U[(t + 1) % 2], W[(t + 2) % 3], W[t % 3], W[(t + 1) % 3],
         x, q, A->nb, A->sell.n_slices, st + t % 2, st + (t + 1) % 2, delta, fin ? tot + 1 : part_g(), fin ? 1u : g_vec,
         part_d(), A->xcd_map);
@@ -934,7 +980,7 @@ struct MinresEngine {
     if (fin) k_finish_sums<<<1, 256, 0, s>>>(part_d(), g_spmv, tot);
     k_mr_lanczos<T><<<g_vec, 256, 0, s>>>(q, V[(t + 1) % 3], V[t % 3], V[(t + 2) % 3], U[(t + 1) % 2], dinv, n,
                                           st + (t + 1) % 2, fin ? tot : part_d(), fin ? 1u : g_spmv, delta, part_g(),
-                                          A->xcd_map, g_spmv, A->bs);
+                                          A->xcd_map, g_spmv, A->bs * (split ? 64 : 256));
     if (fin) k_finish_sums<<<1, 256, 0, s>>>(part_g(), g_vec, tot + 1);
   }
 
@@ -1185,7 +1231,7 @@ __global__ __launch_bounds__(256) void k_bs_update(T* __restrict__ x, T* __restr
                                                    const T* __restrict__ s, const T* __restrict__ t,
                                                    const T* __restrict__ r0, const T* __restrict__ dinv, int64_t n,
                                                    BsState* st, const double* __restrict__ part_b, unsigned g_b,
-                                                   double* __restrict__ part_c, int xcd, unsigned g1, int bs) {
+                                                   double* __restrict__ part_c, int xcd, unsigned g1, int rpb) {
   const int was_done = st->done;
   const T alpha = (T)st->alpha, beta = (T)st->beta;
   double pre[2][4];
@@ -1194,7 +1240,7 @@ __global__ __launch_bounds__(256) void k_bs_update(T* __restrict__ x, T* __restr
   // the rows that this XCD's blocks of k_bs_dir_spmv gather next; the loads
   // of the first 4 elements per thread are issued before omega is known
   int64_t e0, e1;
-  update_range(n, xcd, g1, bs, 64, e0, e1);
+  update_range(n, xcd, g1, rpb, 64, e0, e1);
   const int64_t i0 = e0 + threadIdx.x;
   T xv[4], rv[4], wv[4], vv[4], sv[4], tv[4], r0v[4], dv[4];
 #pragma unroll
@@ -1364,7 +1410,7 @@ struct BsEngine {
     spmv(s, 1);
     if (fin) k_finish_sums<<<2, 256, 0, s>>>(part_b, g_spmv, tot + 1);
     k_bs_update<T><<<g_vec, 256, 0, s>>>(x, r, rh, wh, vh, sv, t, r0, dinv, n, st, src_b(), fin ? 1u : g_spmv,
-                                         part_c, A->xcd_map, g_spmv, A->bs);
+                                         part_c, A->xcd_map, g_spmv, 256 * A->bs);
     if (fin) k_finish_sums<<<2, 256, 0, s>>>(part_c, g_vec, tot + 3);
   }
 
@@ -2048,7 +2094,7 @@ int time_cg_kernel(PcgEngine<T>& E, int kernel, int reps, double* avg_ms, double
       E.launch_k1(s, E.pbuf[0], E.pbuf[1]);
     } else {
       k_cg_update<T><<<E.g_vec, 256, 0, s>>>(E.x, E.pbuf[1], E.r, E.z, E.q, E.dinv, n, E.st, E.pq_src(), E.pq_g(),
-                                             E.part_rz(), E.A->xcd_map, E.g_spmv, E.A->bs);
+                                             E.part_rz(), E.A->xcd_map, E.g_spmv, E.rpb);
     }
   }
   MFS_HIP(hipEventRecord(e1, s));

@@ -40,48 +40,73 @@ struct MrState {
 
 enum { MR_RUN = 0, MR_CONV = 1, MR_BREAK = 2, MR_MAXIT = 3 };
 
-// Sum of NQ values' per-block partials part[q*G + b] in block order, done by
-// every block of the consuming kernel (identical totals).  The first P
-// partials of every value are loaded together (NQ*P loads in flight per
-// thread; G <= 256*P needs no more), so the NQ sums cost one memory latency
-// instead of one each.
+// Sum of NQ values' per-block partials part[q*G + b], done by every block of
+// the consuming kernel (identical totals).  Wave w sums the values w, w + 4,
+// ..: a block's 12 sums (6 systems, r.z and r.r) cost three wave sums in line
+// instead of twelve.  The first P partials of a lane are loaded together.
 template <int NQ, int P>
 __device__ __forceinline__ void mr_sum_partials(const double* __restrict__ part, unsigned G, double (&tot)[NQ]) {
-  __shared__ double red[NQ][4];
+  __shared__ double red[NQ];
+  constexpr int M = (NQ + 3) / 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double pre[NQ][P];
+  double pre[M][P];
 #pragma unroll
-  for (int q = 0; q < NQ; q++)
+  for (int m = 0; m < M; m++)
 #pragma unroll
     for (int u = 0; u < P; u++) {
-      const unsigned b = threadIdx.x + u * 256;
-      pre[q][u] = b < G ? part[(size_t)q * G + b] : 0.0;
+      const unsigned b = lane + u * 64;
+      const int q = wave + 4 * m;
+      pre[m][u] = q < NQ && b < G ? part[(size_t)q * G + b] : 0.0;
     }
 #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    double s = pre[q][0];
+  for (int m = 0; m < M; m++) {
+    const int q = wave + 4 * m;
+    double s = pre[m][0];
 #pragma unroll
-    for (int u = 1; u < P; u++) s += pre[q][u];
-    for (unsigned b = threadIdx.x + P * 256; b < G; b += 256) s += part[(size_t)q * G + b];
+    for (int u = 1; u < P; u++) s += pre[m][u];
+    if (q < NQ)
+      for (unsigned b = lane + P * 64; b < G; b += 64) s += part[(size_t)q * G + b];
     s = wave_sum(s);
-    if (lane == 0) red[q][wave] = s;
+    if (lane == 0 && q < NQ) red[q] = s;
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < NQ; q++) tot[q] = (red[q][0] + red[q][1]) + (red[q][2] + red[q][3]);
+  for (int q = 0; q < NQ; q++) tot[q] = red[q];
   __syncthreads();
+}
+
+// Wave sums of NQ values in one halving exchange: at each step a lane keeps
+// one half of its values and adds its partner's share of them, so NQ sums take
+// about NQ + 3 shuffles instead of 6 NQ.  The additions are those of wave_sum.
+template <int NQ>
+__device__ __forceinline__ void mr_wave_sums(double (&v)[NQ], double (*red)[4]) {
+  constexpr int L = NQ > 8 ? 4 : NQ > 4 ? 3 : NQ > 2 ? 2 : NQ > 1 ? 1 : 0, N2 = 1 << L;
+  static_assert(NQ <= 16, "at most 16 values");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double t[N2];
+#pragma unroll
+  for (int q = 0; q < N2; q++) t[q] = q < NQ ? v[q] : 0.0;
+#pragma unroll
+  for (int l = 0; l < L; l++) {
+    const int off = 32 >> l, half = N2 >> (l + 1);
+    const bool upper = lane & off;
+#pragma unroll
+    for (int q = 0; q < half; q++) {
+      const double send = upper ? t[q] : t[q + half], keep = upper ? t[q + half] : t[q];
+      t[q] = keep + __shfl_xor(send, off, MFS_WAVE);
+    }
+  }
+#pragma unroll
+  for (int off = 32 >> L; off > 0; off >>= 1) t[0] += __shfl_xor(t[0], off, MFS_WAVE);
+  const int q = lane >> (6 - L);
+  if ((lane & ((64 >> L) - 1)) == 0 && q < NQ) red[q][wave] = t[0];
 }
 
 // Per-block partials of NQ values into part[q*gridDim + blockIdx].
 template <int NQ>
 __device__ __forceinline__ void mr_block_partials(double (&v)[NQ], double* __restrict__ part) {
   __shared__ double red[NQ][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    const double s = wave_sum(v[q]);
-    if (lane == 0) red[q][wave] = s;
-  }
+  mr_wave_sums<NQ>(v, red);
   __syncthreads();
   if (threadIdx.x < NQ)
     part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
@@ -129,6 +154,112 @@ __device__ __forceinline__ void vstore(T* __restrict__ p, const T (&o)[KR]) {
     W u;
     __builtin_memcpy(&u, &o[v * (B / sizeof(T))], B);
     q[v] = u;
+  }
+}
+
+// N consecutive values from an 8-byte aligned address, 16 bytes per load.
+template <typename T, int N>
+__device__ __forceinline__ void vload_wide(const T* __restrict__ p, T (&o)[N]) {
+  typedef unsigned int word4 __attribute__((ext_vector_type(4), aligned(8)));
+  constexpr int bytes = N * sizeof(T), NV = bytes / 16;
+  static_assert(bytes % 8 == 0, "whole 8-byte words");
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    const word4 u = reinterpret_cast<const word4*>(p)[v];
+    __builtin_memcpy(&o[v * (16 / sizeof(T))], &u, 16);
+  }
+  if constexpr (bytes % 16) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p + NV * (16 / sizeof(T)));
+    __builtin_memcpy(&o[NV * (16 / sizeof(T))], &u, 8);
+  }
+}
+
+// Rows [component a][j] of the 3x3-block products of one slice by the four
+// waves of a block, P = Z + beta P_old formed on the way.  A block row's 3*KR
+// values of Z and P_old lie together and are gathered once, by the wave that
+// an entry falls to (whole 16-byte words: a 64-lane gather costs a line
+// lookup per lane whatever its width, and those lookups bound this kernel);
+// the waves a < 3 then take the operands from LDS and add component a in the
+// order of sell_row_multi.  The next G entries' gathers are in flight during
+// the products.  us per iteration with a wave per slice and 8-byte gathers,
+// and so: 6 systems in FP32, 245 slices 52.5, 22.7; 1077 slices 94.4, 60.7;
+// 3547 slices 152, 115; 2 systems, 1838 slices 57, 51; 6 in FP64, 245 slices
+// 63, 29.
+template <typename T, int KR>
+constexpr int mr_group() {
+  return sizeof(T) * KR > 32 ? 4 : 8;  // entries per round: at most 48 KB of LDS
+}
+template <typename T, int KR, typename CI>
+__device__ __forceinline__ void sell_slice_multi(const int64_t* __restrict__ slice_base,
+                                                 const int32_t* __restrict__ slice_width, const CI* __restrict__ col,
+                                                 const T* __restrict__ val, const T* __restrict__ Z,
+                                                 const T* __restrict__ P_old, const T (&beta)[KR], int64_t slice,
+                                                 T (&acc)[KR]) {
+  constexpr int C = 64, G = mr_group<T, KR>(), M = G / 4, N = 3 * KR;
+  __shared__ T sm[G][N][C];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t sb = slice_base[slice];
+  const int w = slice_width[slice];
+  const CI* cp = col + sb + lane;
+  const int32_t rbase = sizeof(CI) == 2 ? (int32_t)(slice * C + lane) : 0;
+  const T* vp = val + sb * 9 + 3 * wave * C + lane;
+  T z[M][N], p[M][N], v[G][3], vn[G][3];
+  int32_t c[M];
+#pragma unroll
+  for (int j = 0; j < KR; j++) acc[j] = 0;
+  // entry j0 + wave + 4 m is this wave's to gather; past the end the last one
+  auto columns = [&](int j0) {
+#pragma unroll
+    for (int m = 0; m < M; m++) c[m] = (int32_t)cp[(int64_t)min(j0 + wave + 4 * m, w - 1) * C] + rbase;
+  };
+  auto gather = [&]() {
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      vload_wide<T, N>(Z + (int64_t)c[m] * N, z[m]);
+      vload_wide<T, N>(P_old + (int64_t)c[m] * N, p[m]);
+    }
+  };
+  auto values = [&](int j0, T (&o)[G][3]) {
+    if (wave == 3) return;
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int j = min(j0 + u, w - 1);
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        const T t = __builtin_nontemporal_load(vp + ((int64_t)j * 9 + b) * C);
+        o[u][b] = j0 + u < w ? t : (T)0;
+      }
+    }
+  };
+  if (w > 0) {
+    columns(0);
+    values(0, v);
+    gather();
+    columns(G);
+  }
+  for (int j0 = 0; j0 < w; j0 += G) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int e = 0; e < N; e++) sm[wave + 4 * m][e][lane] = z[m][e] + beta[e % KR] * p[m][e];
+    __syncthreads();
+    if (j0 + G < w) {
+      gather();
+      values(j0 + G, vn);
+      columns(j0 + 2 * G);
+    }
+    if (wave < 3)
+#pragma unroll
+      for (int u = 0; u < G; u++)
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+#pragma unroll
+          for (int j = 0; j < KR; j++) acc[j] += v[u][b] * sm[u][b * KR + j][lane];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < G; u++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) v[u][b] = vn[u][b];
   }
 }
 
@@ -325,11 +456,21 @@ __global__ __launch_bounds__(256) void k_mr_dir_spmm(const int64_t* __restrict__
     st->alldone = all;
   }
   if (all) return;
-  const int64_t slice = (int64_t)xcd_block(xcd) * 4 + threadIdx.x / 64;
+  // 3x3 blocks: one slice per block, wave a < 3 holds component a
+  constexpr int NA = BS == 3 ? 1 : BS;
+  const int wave = threadIdx.x / 64;
+  const int64_t slice = BS == 3 ? (int64_t)xcd_block(xcd) : (int64_t)xcd_block(xcd) * 4 + wave;
   const int lane = threadIdx.x & 63;
   const int64_t row = slice * 64 + lane;
-  T acc[BS][KR];
-  if (slice < n_slices) {
+  const int a0 = BS == 3 ? wave : 0;
+  T acc[NA][KR];
+#pragma unroll
+  for (int a = 0; a < NA; a++)
+#pragma unroll
+    for (int j = 0; j < KR; j++) acc[a][j] = 0;
+  if constexpr (BS == 3) {
+    sell_slice_multi<T, KR>(slice_base, slice_width, col, val, Z, P_old, beta, slice, acc[0]);
+  } else if (slice < n_slices) {
     sell_row_multi<T, BS, KR>(slice_base, slice_width, col, val, slice, lane,
                               [&](int64_t i, T (&o)[KR]) {
                                 T zz[KR], pp[KR];
@@ -339,19 +480,14 @@ __global__ __launch_bounds__(256) void k_mr_dir_spmm(const int64_t* __restrict__
                                 for (int j = 0; j < KR; j++) o[j] = zz[j] + beta[j] * pp[j];
                               },
                               acc);
-  } else {
-#pragma unroll
-    for (int a = 0; a < BS; a++)
-#pragma unroll
-      for (int j = 0; j < KR; j++) acc[a][j] = 0;
   }
   double red[KR];
 #pragma unroll
   for (int j = 0; j < KR; j++) red[j] = 0;
-  if (row < nb) {
+  if (row < nb && (BS != 3 || wave < 3)) {
 #pragma unroll
-    for (int a = 0; a < BS; a++) {
-      const int64_t e0 = (BS * row + a) * KR;
+    for (int a = 0; a < NA; a++) {
+      const int64_t e0 = (BS * row + a0 + a) * KR;
       T zz[KR], pp[KR], pn[KR];
       vload<T, KR>(Z + e0, zz);
       vload<T, KR>(P_old + e0, pp);
@@ -482,7 +618,7 @@ struct MrEngine {
     dinv = precond ? (f64 ? (const T*)A->d_dinv64 : (const T*)A->d_dinv32) : nullptr;
     for (T** b : {&X, &R, &Z, &Q, &P[0], &P[1]}) MFS_TRY(dmalloc((void**)b, sizeof(T) * n * KR));
     MFS_TRY(dmalloc((void**)&st, sizeof(MrState)));
-    g_spmv = (unsigned)spmv_grid(A);
+    g_spmv = (unsigned)(A->bs == 3 ? A->sell.n_slices : spmv_grid(A));
     g_vec = mr_grid(n);
     MFS_TRY(dmalloc((void**)&part_rz, sizeof(double) * 2 * KR * std::max(g_spmv, g_vec)));
     MFS_TRY(dmalloc((void**)&part_pq, sizeof(double) * KR * g_spmv));
@@ -535,7 +671,7 @@ struct MrEngine {
                                                               A->xcd_map);
     if (fin) k_finish_sums<<<KR, 256, 0, s>>>(part_pq, g_spmv, tot_pq);
     k_mr_update<T, KR><<<g_vec, 256, 0, s>>>(X, p_new, R, Z, Q, dinv, n, st, fin ? tot_pq : part_pq,
-                                             fin ? 1u : g_spmv, part_rz, A->xcd_map, g_spmv, 256 * A->bs);
+                                             fin ? 1u : g_spmv, part_rz, A->xcd_map, g_spmv, A->bs == 3 ? 192 : 256);
     finish_rz(s);
   }
 

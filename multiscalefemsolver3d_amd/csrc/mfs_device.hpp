@@ -319,6 +319,99 @@ __device__ __forceinline__ T sell_row_component(const int64_t* __restrict__ slic
   return acc;
 }
 
+// 3x3-block row products of one slice by the four waves of a block: an entry's
+// operand (from xl) is gathered once, by the wave it falls to, and reaches the
+// waves a < 3 through LDS; they return component a, by the operations of
+// sell_row_x in the same order.  The next G entries are in flight during the
+// products.
+template <typename T, int G, typename XL, typename CI>
+__device__ __forceinline__ T sell_slice_x(const int64_t* __restrict__ slice_base,
+                                          const int32_t* __restrict__ slice_width, const CI* __restrict__ col,
+                                          const T* __restrict__ val, int64_t slice, XL xl) {
+  constexpr int C = 64, M = G / 4;
+  __shared__ T sm[G][3][C];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t sb = slice_base[slice];
+  const int w = slice_width[slice];
+  const CI* cp = col + sb + lane;
+  const int32_t rbase = sizeof(CI) == 2 ? (int32_t)(slice * C + lane) : 0;
+  const T* vp = val + sb * 9 + 3 * wave * C + lane;
+  T x[M][3], v[G][3], vn[G][3];
+  int32_t c[M];
+  T acc = 0;
+  // entry j0 + wave + 4 m is this wave's to gather; past the end the last one
+  auto columns = [&](int j0) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+      c[m] = (int32_t)__builtin_nontemporal_load(cp + (int64_t)min(j0 + wave + 4 * m, w - 1) * C) + rbase;
+  };
+  auto gather = [&]() {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) x[m][b] = xl((int64_t)3 * c[m] + b);
+  };
+  auto values = [&](int j0, T (&o)[G][3]) {
+    if (wave == 3) return;
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int j = min(j0 + u, w - 1);
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        const T t = __builtin_nontemporal_load(vp + ((int64_t)j * 9 + b) * C);
+        o[u][b] = j0 + u < w ? t : (T)0;
+      }
+    }
+  };
+  if (w > 0) {
+    columns(0);
+    values(0, v);
+    gather();
+    columns(G);
+  }
+  for (int j0 = 0; j0 < w; j0 += G) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) sm[wave + 4 * m][b][lane] = x[m][b];
+    __syncthreads();
+    if (j0 + G < w) {
+      gather();
+      values(j0 + G, vn);
+      columns(j0 + 2 * G);
+    }
+    if (wave < 3)
+#pragma unroll
+      for (int u = 0; u < G; u++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) acc += v[u][b] * sm[u][b][lane];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < G; u++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) v[u][b] = vn[u][b];
+  }
+  return acc;
+}
+
+// One slice per block: component `wave` (< 3; else 0) of its rows.  FP64
+// shares the gathers, FP32 makes them three times: the exchange's barriers
+// cost 0.3 us more there than the repeated 4-byte gathers (12.5 -> 10.7 and
+// 11.0 us per PCG iteration at 77 slices); in FP64 it takes 27.0 us where the
+// repeated gathers take 32.0 (1,077 slices).
+template <typename T, typename XL, typename CI>
+__device__ __forceinline__ T slice_component(const int64_t* __restrict__ slice_base,
+                                             const int32_t* __restrict__ slice_width, const CI* __restrict__ col,
+                                             const T* __restrict__ val, int64_t slice, XL xl) {
+  if constexpr (sizeof(T) == 8) {
+    return sell_slice_x<T, 8>(slice_base, slice_width, col, val, slice, xl);
+  } else {
+    const int wave = threadIdx.x >> 6;
+    if (wave == 3) return 0;
+    return sell_row_component<T, 9>(slice_base, slice_width, col, val, slice, threadIdx.x & 63, wave, xl);
+  }
+}
+
 template <typename T, int BS, typename CI>
 __device__ __forceinline__ void sell_row(const int64_t* __restrict__ slice_base, const int32_t* __restrict__ slice_width,
                                          const CI* __restrict__ col, const T* __restrict__ val,

@@ -708,13 +708,14 @@ int64_t spmv_grid(mfs_mat A) { return (A->sell.n_slices + 3) / 4; }
 // waves to hide a row's chain of index, gather and value latencies.  us per
 // PCG iteration, a wave per slice -> a wave per component, over the slices:
 //   FP32:  77 12.5 -> 10.7   145 12.0 ->  9.8 (MINRES)   562 13.9 -> 14.4
-//   FP64:  77 18.2 -> 12.5   245 22.0 -> 12.7           1077 37.3 -> 32.0
-//        2073 54.5 -> 54.8  3547 78.5 -> 92.6
-// Past the line the operand gathers, made three times, cost more.
+//   FP64:  77 18.2 -> 11.9   245 22.0 -> 11.8   1077 37.0 -> 27.0
+//        2073 54.5 -> 46.0  3547 78.6 -> 79.2
+// Past the line the other form's waves fill the chip, and its longer rows of
+// loads per wave stream the matrix at the same or a better rate.
 bool sell_component_waves(mfs_mat A, bool f64) {
   if (A->bs != 3) return false;
   if (const char* e = std::getenv("MFS_COMPONENT_WAVES")) return e[0] == '1';  // force either way (tests)
-  return A->sell.n_slices <= (f64 ? 1200 : 400);
+  return A->sell.n_slices <= (f64 ? 2100 : 400);
 }
 }  // namespace mfs
 

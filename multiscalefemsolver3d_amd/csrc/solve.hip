@@ -109,7 +109,6 @@ __device__ __forceinline__ void component_dot(const T (&v)[2], T& dot) {
     dot = 0;
   }
 }
-constexpr int kCompGroup = 9;  // entries per latency of sell_row_component
 
 // K1: from K2's partials (r.z, r.r): stop test, beta = rz / rz_prev;
 // p_new = z + beta p_old (own rows written), q = A p_new, per-block partial
@@ -187,9 +186,8 @@ __global__ __launch_bounds__(256) void k_cg_dir_spmv(const int64_t* __restrict__
       }
     }
     if constexpr (CW) {
-      if (wave < BS)
-        az[0] = sell_row_component<T, kCompGroup>(slice_base, slice_width, col, val, slice, lane, wave,
-                                                  [&](int64_t i) { return z[i] + beta * p_old[i]; });
+      az[0] = slice_component<T>(slice_base, slice_width, col, val, slice,
+                                 [&](int64_t i) { return z[i] + beta * p_old[i]; });
     } else if (slice < n_slices) {
       sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb,
                         [&](int64_t i) { return z[i] + beta * p_old[i]; }, az);
@@ -755,9 +753,7 @@ __global__ __launch_bounds__(256) void k_mr_spmv(const int64_t* __restrict__ sli
       xo[a] = x[i];
     }
   if constexpr (CW) {
-    if (wave < BS)
-      acc[0] = sell_row_component<T, kCompGroup>(slice_base, slice_width, col, val, slice, lane, wave,
-                                                 [&](int64_t i) { return u[i]; });
+    acc[0] = slice_component<T>(slice_base, slice_width, col, val, slice, [&](int64_t i) { return u[i]; });
   } else if (slice < n_slices) {
     sell_row_x<T, BS>(slice_base, slice_width, col, val, slice, lane, nb, [&](int64_t i) { return u[i]; }, acc);
   }

@@ -41,7 +41,7 @@ def spd(ctx, nb, bs, wide, seed):
     return mfs.Mat.bsr3(ctx, blk.indptr, blk.indices, blk.data), A
 
 
-LINE, LINE64 = 400 * 64, 1200 * 64  # block rows at the lines of the default rule, FP32 and FP64
+LINE, LINE64 = 400 * 64, 2100 * 64  # block rows at the lines of the default rule, FP32 and FP64
 
 
 @pytest.mark.parametrize("bs,nb,wide", [(1, 1, 0), (1, 64, 30), (1, 65, 9), (1, 1000, 40),(3, 1, 0), (3, 63, 14), (3, 300, 30), (3, LINE, 2), (3, LINE + 1, 2), (3, LINE64 + 1, 2)])

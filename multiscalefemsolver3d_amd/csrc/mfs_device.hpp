@@ -4,6 +4,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -52,6 +53,10 @@ struct mfs_ctx_s {
   // array (mfs_solve_noalloc), resolved once per device at context creation
   void* noalloc_scratch = nullptr;
   size_t noalloc_scratch_bytes = 0;
+  // mfs_dot's partial sums and result, kept from the first call on; the lock
+  // is held until the result has been read back
+  std::mutex dot_lock;
+  double* dot_scratch = nullptr;
 };
 
 struct mfs_vec_s {

@@ -148,6 +148,7 @@ void ctx_release(mfs_ctx c) {
   (void)hipStreamSynchronize(c->stream);
   (void)hipStreamDestroy(c->stream);
   (void)hipHostFree(c->pinned);
+  dfree(c->dot_scratch);
   delete c;
 }
 }  // namespace mfs
@@ -751,7 +752,7 @@ extern "C" int mfs_spmv_time(mfs_mat A, int prec, mfs_vec x, mfs_vec y, int reps
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void k_dot(const T* __restrict__ x, const T* __restrict__ y, int64_t n,
-                                             double* partials, unsigned* counter, double* out) {
+                                             double* partials) {
   T v[1] = {0};
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     v[0] += x[i] * y[i];
@@ -770,18 +771,18 @@ extern "C" int mfs_dot(mfs_vec x, mfs_vec y, double* result) {
   MFS_CHECK_ARG(result && x->n == y->n && x->prec == y->prec, "mfs_dot: size/precision mismatch");
   hipStream_t s = x->ctx->stream;
   const unsigned g = std::min<unsigned>(grid_for(x->n), 1024);
-  ReduceScratch rs;
-  MFS_TRY(reduce_scratch_alloc(rs, 1024 + 8));
-  double* out = rs.partials + 1024;
+  // allocating, clearing and freeing this per call took longer than the sum
+  std::lock_guard<std::mutex> hold(x->ctx->dot_lock);
+  if (!x->ctx->dot_scratch) MFS_TRY(dmalloc((void**)&x->ctx->dot_scratch, sizeof(double) * (1024 + 8)));
+  double *part = x->ctx->dot_scratch, *out = part + 1024;
   if (x->prec == MFS_F64)
-    k_dot<double><<<g, 256, 0, s>>>((const double*)x->d, (const double*)y->d, x->n, rs.partials, rs.counter, out);
+    k_dot<double><<<g, 256, 0, s>>>((const double*)x->d, (const double*)y->d, x->n, part);
   else
-    k_dot<float><<<g, 256, 0, s>>>((const float*)x->d, (const float*)y->d, x->n, rs.partials, rs.counter, out);
-  k_finish_sums<<<1, 256, 0, s>>>(rs.partials, g, out);
+    k_dot<float><<<g, 256, 0, s>>>((const float*)x->d, (const float*)y->d, x->n, part);
+  k_finish_sums<<<1, 256, 0, s>>>(part, g, out);
   MFS_HIP(hipGetLastError());
   MFS_HIP(hipMemcpyAsync(result, out, sizeof(double), hipMemcpyDeviceToHost, s));
   MFS_HIP(hipStreamSynchronize(s));
-  reduce_scratch_free(rs);
   return MFS_OK;
 }
 

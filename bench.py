@@ -38,12 +38,10 @@ HBM_PEAK_GBS = 8000.0
 # rocprofv3 --pmc FETCH_SIZE (13,300.2 KiB, x2.000 from a 512 MiB copy) and
 # WRITE_SIZE (2,179.2 KiB, x1.000), medians over 7,752 / 7,731 dispatches
 TRAFFIC_K1 = 29470310
-# HBM bytes of one k_batch_solve<float,1,true> launch on the headline
-# workload (learned guess, launch shape 384 / variant 3): rocprofv3 --pmc
-# FETCH_SIZE 57,946,409.9 KiB x2.000 + WRITE_SIZE 14,526,056.7 KiB x1.000
-# (the copy calibration above).  The register-resident kernel keeps r, q, d
-# and p on chip, so this is 0.058 of the algorithmic bytes.
-TRAFFIC_BATCH = 133548929536
+# HBM bytes of one k_batch_solve_mfma launch on the headline workload
+# (learned guess): rocprofv3 --pmc FETCH_SIZE 305,591,982.7 KiB x2.000 +
+# WRITE_SIZE 44,746,298.5 KiB x1.000 (the copy calibration above).
+TRAFFIC_BATCH = 671672590233
 
 
 def log(*a):
@@ -142,7 +140,7 @@ def main():
         "data": "synthetic (seeded lognormal moduli; the network is trained on cells the solver generates)",
         "config": head["config"],
         # FP64 GPU CG on the same problems: the batched register-resident
-        # kernel (same design as the mixed one, the ratio quoted), and plain
+        # kernel (on the vector unit; the ratio quoted), and plain
         # FP64 PCG through mfs_solve one problem at a time (sampled)
         "fp64_gpu_cg_ms": head["fp64_batched_zero_ms"],
         "speedup_vs_fp64_gpu_cg": round(head["fp64_batched_zero_ms"] / head["ms_per_step"], 3),
@@ -256,15 +254,15 @@ def bench_headline(mfs, ctx, args):
     }
     roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_BATCH,
-            "kernel": "k_batch_solve<float,R,REG> (persistent batched PCG, FP32 inner / FP64 refinement)",
+            "kernel": "k_batch_solve_mfma (persistent batched PCG, FP32 inner on the matrix cores / FP64 refinement)",
             "bytes_per_launch": nbytes, "avg_ms": round(kern_ms, 3),
             "measured_hbm_gbs": round(TRAFFIC_BATCH / (kern_ms * 1e6), 1),
             "note": "algorithmic bytes: per cell-iteration the 15-point stencil matrix once for all 24 "
                     "right-hand sides plus 11 vector passes per right-hand side and iteration; the "
-                    "register-resident kernel keeps the vectors on chip (registers, LDS, L2), so the "
+                    "kernel keeps the vectors on chip (registers, LDS, L2), so the "
                     "algorithmic rate is an effective one that can exceed the HBM peak, while the "
-                    "measured traffic (FETCH_SIZE/WRITE_SIZE) is far below it: the kernel is bound by "
-                    "FP32 VALU issue and latency, not by HBM"}
+                    "measured traffic (FETCH_SIZE/WRITE_SIZE) is 0.29 of those bytes: mostly K "
+                    "that the tasks of a cell no longer find in their L2"}
     # the GEMM of the network alone at a large size (MFMA utilisation)
     gms, gtf = mfs.gemm_bf16_time(ctx, 8192, 8192, 8192, reps=5)
     detail["gemm_bf16_kernel_8192cubed"] = {"ms": round(gms, 3), "tflops": round(gtf, 1),

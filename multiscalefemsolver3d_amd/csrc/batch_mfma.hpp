@@ -186,12 +186,9 @@ __device__ __forceinline__ void mfma_product(const MfmaK& K, f32x4_t (&kr)[MF_PF
     if (v < nint) {
       const float* pp = P + v * (3 * NR) + C * c;
 #pragma unroll
-      for (int j = 0; j < C; j++) {
-        float t = 0;
+      for (int j = 0; j < C; j++)
 #pragma unroll
-        for (int a = 0; a < 3; a++) t += Q[g][j][a] * pp[a * NR + j];
-        w[j] += (double)t;
-      }
+        for (int a = 0; a < 3; a++) w[j] += (double)(Q[g][j][a] * pp[a * NR + j]);
     }
   }
 }
@@ -524,9 +521,6 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
           for (int g = 0; g < G; g++) {
             const int v = row(g);
             if (v >= nint) continue;
-            float t[C];
-#pragma unroll
-            for (int j = 0; j < C; j++) t[j] = 0;
 #pragma unroll
             for (int a = 0; a < 3; a++) {
               const float dv = DV[3 * v + a];
@@ -539,11 +533,9 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
                   D[g][a][j - DJ] += alpha[j] * pe;
                 const float rv = R[g][a][j] - alpha[j] * Q[g][j][a];
                 R[g][a][j] = rv;
-                t[j] += rv * (dv * rv);
+                w[j] += (double)(rv * (dv * rv));
               }
             }
-#pragma unroll
-            for (int j = 0; j < C; j++) w[j] += (double)t[j];
           }
           mfma_wave_sums<C>(w, partA);
 #pragma unroll
@@ -552,12 +544,9 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
           for (int g = 0; g < G; g++) {
             if (row(g) >= nint) continue;
 #pragma unroll
-            for (int j = 0; j < C; j++) {
-              float t = 0;
+            for (int j = 0; j < C; j++)
 #pragma unroll
-              for (int a = 0; a < 3; a++) t += R[g][a][j] * R[g][a][j];
-              w[j] += (double)t;
-            }
+              for (int a = 0; a < 3; a++) w[j] += (double)(R[g][a][j] * R[g][a][j]);
           }
           mfma_wave_sums<C>(w, partA + 4 * C * W);
           const double rz_old = S.rz[par][sl], itol2 = S.itol2[sl], rrmin = S.rrmin[par][sl];

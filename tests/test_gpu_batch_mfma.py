@@ -50,6 +50,47 @@ def test_bases_match_oracle_at_class_and_tile_edges(ctx, sizes):
     B.close()
 
 
+def test_inner_products_add_every_product_in_fp64(ctx):
+    """r.z and p.q are FP64 sums of FP32 products.  Cells with one interior
+    node and one iteration show it: x = alpha p with alpha = r.z / p.q in
+    FP32, restated here operation by operation.  FP32 sums of the three
+    components would move alpha by one unit in the last place (6e-8) for a
+    good part of the problems; the restatement itself can part from the
+    kernel only where the last bit of an FP64 input decides an FP32 rounding
+    (odds of about 1e-7 a problem), so nearly every problem must agree."""
+    cells, h, f32 = 128, 0.25, np.float32
+    E = [np.exp(np.log(1e9) + 0.3 * np.random.default_rng([9, c]).standard_normal(48)) for c in range(cells)]
+    B = mfs.Batch(ctx, [2] * cells, [[c * h, 0, 0] for c in range(cells)], h, np.concatenate(E), 0.3,
+                  convention=mfs.ELEM_TEXTBOOK)
+    B.assemble()
+    rep = B.solve(check=False, precision=mfs.PREC_MIXED, tol=1e-12, maxit=1)
+    assert rep.max_iterations == 1 and rep.n_precision_fallback == 0
+    xyz, tets = mfs.mesh_box(2, h=(h / 2,) * 3)
+    inner = 3 * 13 + np.arange(3)
+    outer = np.setdiff1d(np.arange(81), inner)
+    agree = 0
+    for c in range(cells):
+        K = np.zeros((81, 81))
+        for t, T in enumerate(tets):
+            d = (3 * T[:, None] + np.arange(3)).ravel()
+            K[np.ix_(d, d)] += orc.elem_elastic(xyz[T], E[c][t], 0.3, mfs.ELEM_TEXTBOOK)
+        x = B.basis(c)
+        b = -K[np.ix_(inner, outer)] @ x[:, outer].T
+        Ki = K[np.ix_(inner, inner)]
+        scale = np.sqrt((b ** 2).sum(0))
+        r = (b.astype(f32).astype(float) * (1 / scale).astype(f32).astype(float)).astype(f32)
+        p = (1 / np.diag(Ki)).astype(f32)[:, None] * r
+        rz = (r * p).astype(float).sum(0)
+        q = np.zeros_like(p)
+        for k in range(3):  # fused multiply-adds
+            q = (Ki[:, k:k + 1].astype(f32).astype(float) * p[k].astype(float) + q).astype(f32)
+        alpha = (rz / (q * p).astype(float).sum(0)).astype(f32)
+        ref = scale * (alpha * p).astype(float)
+        agree += int((np.abs(x[:, inner].T - ref).max(0) <= 1e-12 * np.abs(ref).max(0)).sum())
+    assert agree >= 0.99 * 24 * cells, agree
+    B.close()
+
+
 def test_iteration_cap_and_failure_list(ctx):
     """Problems stopped by maxit are reported as such; problems that FP32
     cannot finish are handed over in groups of eight and end converged, the

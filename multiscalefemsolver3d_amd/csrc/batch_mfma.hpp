@@ -38,7 +38,8 @@
 // stored as its upper half, the lower blocks transposed by lane moves
 // (32.1 ms: a third less traffic beyond L2, but 126 more vector instructions
 // per 16 nodes); two workgroups of 4 waves with 12 right-hand sides per CU
-// (38.1 ms: K is read twice).
+// (38.1 ms: K is read twice).  Inner products added in FP32 per node first
+// were 4 % faster (17.1 against 17.8 ms) and are not used.
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -513,7 +514,8 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
         float beta[C];
         {
           // d, r and r.z group by group, then r.r from the new r: fewer sums
-          // are live beside q
+          // are live beside q.  (One conversion and FP64 products: 1.5 % less
+          // time than FP32 products converted one by one.)
           double w[C];
 #pragma unroll
           for (int j = 0; j < C; j++) w[j] = 0;
@@ -523,7 +525,7 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
             if (v >= nint) continue;
 #pragma unroll
             for (int a = 0; a < 3; a++) {
-              const float dv = DV[3 * v + a];
+              const double dvd = DV[3 * v + a];
 #pragma unroll
               for (int j = 0; j < C; j++) {
                 const float pe = P[v * (3 * NR) + a * NR + C * c + j];
@@ -533,7 +535,8 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
                   D[g][a][j - DJ] += alpha[j] * pe;
                 const float rv = R[g][a][j] - alpha[j] * Q[g][j][a];
                 R[g][a][j] = rv;
-                w[j] += (double)(rv * (dv * rv));
+                const double rd = rv;
+                w[j] += (rd * rd) * dvd;
               }
             }
           }
@@ -546,7 +549,7 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
 #pragma unroll
             for (int j = 0; j < C; j++)
 #pragma unroll
-              for (int a = 0; a < 3; a++) w[j] += (double)(R[g][a][j] * R[g][a][j]);
+              for (int a = 0; a < 3; a++) w[j] += (double)R[g][a][j] * (double)R[g][a][j];
           }
           mfma_wave_sums<C>(w, partA + 4 * C * W);
           const double rz_old = S.rz[par][sl], itol2 = S.itol2[sl], rrmin = S.rrmin[par][sl];

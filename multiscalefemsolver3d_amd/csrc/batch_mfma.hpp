@@ -3,7 +3,8 @@
 // and the stencil tables.
 //
 // One task holds NR right-hand sides of a cell (all 24 for cells of up to 384
-// interior nodes, 12 for up to 768).  The stencil product q = K p is a 3x3
+// interior nodes, 12 for up to 768; 8 or 12 in batches too small to fill the
+// chip so, see mfma_batch_rhs).  The stencil product q = K p is a 3x3
 // block per (node, stencil point) times 3 x NR values, and every node has
 // blocks of its own, so the product maps onto v_mfma_f32_4x4x1_16b_f32: 16
 // independent 4x4 outer products.  Block = node (16 consecutive nodes per
@@ -44,11 +45,28 @@
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // right-hand sides per lane whose correction lives in LDS
-constexpr int mfma_d_lds(int nr) { return nr == 24 ? 3 : 1; }
+constexpr int mfma_d_lds(int nr) { return nr == 24 ? 3 : nr == 12 ? 1 : 0; }
 // Right-hand sides per task of a cell: all 24 while r, q and half of d of 24
 // groups of 16 nodes fit the registers of 8 waves (n <= 8), else 12 (n = 9,
 // 10: up to 48 groups).
 __host__ __device__ constexpr int mfma_task_rhs(int nint) { return nint <= 384 ? 24 : 12; }
+
+// Time of a cell's task in units of about 0.3 us of a batch of its own: each
+// iteration costs a fixed part and one per node, and iterations grow with n.
+// (24 right-hand sides, n = 3..8: 0.13 0.17 0.21 0.38 0.65 0.98 ms.)
+inline int64_t mfma_task_weight(int n, int nint) { return 400 + (int64_t)n * nint; }
+// Right-hand sides per task of a whole batch (0: mfma_task_rhs of each cell).
+// A cell's wider tasks do less work in all (K is read once, the barriers are
+// shared), narrower ones end sooner: 8^3 0.98 / 0.64 / 0.46 ms with 24 / 12 /
+// 8, 5^3 0.21 / 0.16 / 0.12, 10^3 1.41 with 12, 1.00 with 8.  So the narrowest
+// width is taken whose tasks, counted as fractions of the largest cell's, all
+// run at once, one per CU: 85 cells of 8^3 1.08 -> 0.54 ms, 128 cells 1.11 ->
+// 0.75; with 100 cells 8 at a time would take a second turn (0.99 ms, 12: 0.73).
+inline int mfma_batch_rhs(int64_t weights, int64_t largest, int cus) {
+  for (int nr : {8, 12})
+    if (weights * (24 / nr) <= (int64_t)cus * largest) return nr;
+  return 0;
+}
 
 struct MfmaRhs {  // per right-hand side of the running task
   double bb[NB], rr64[NB], prev[NB], scale[NB], itol2[NB];
@@ -154,7 +172,7 @@ __device__ __forceinline__ void mfma_product(const MfmaK& K, f32x4_t (&kr)[MF_PF
       for (int j = 0; j < C; j++) Q[g][j] = f32x4_t{0, 0, 0, 0};
       // p from LDS PD entries ahead (an entry's C products take 8 C cycles, an
       // LDS read about 130); the scheduling barriers keep it that way
-      constexpr int PD = C >= 6 ? 2 : 4;
+      constexpr int PD = C >= 6 ? 2 : C >= 3 ? 4 : 8;
       float pv[PD + 1][C];
       const float* pu[2];
       auto request = [&](int t) {
@@ -652,14 +670,17 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
 // Launch classes by the batch's largest cell: 0: nint <= 64 and 1: nint <= 128
 // (4 waves of 1 / 2 groups, several workgroups per CU), 2: nint <= 384 (8
 // waves of up to 3 groups, one workgroup per CU: p and d take its LDS), 3:
-// nint <= 729 (tasks of 24 and of 12 right-hand sides in one launch).
-__host__ __device__ constexpr int mfma_class(int max_nint) {
-  return max_nint <= 64 ? 0 : max_nint <= 128 ? 1 : max_nint <= 384 ? 2 : 3;
+// nint <= 729 (up to 6 groups; tasks of 24 and of 12 right-hand sides in one
+// launch), 4: tasks of 8 with nint <= 512 (up to 4 groups: one cell of 9^3
+// 0.68 -> 0.65 ms; the wider tasks gain nothing from it).
+__host__ __device__ constexpr int mfma_class(int max_nint, int task_rhs) {
+  return max_nint <= 64 ? 0 : max_nint <= 128 ? 1 : max_nint <= 384 ? 2 : max_nint <= 512 && task_rhs == 8 ? 4 : 3;
 }
 constexpr int mfma_waves(int cls) { return cls <= 1 ? 4 : 8; }
 constexpr int mfma_eu(int cls) { return cls == 0 ? 3 : 2; }
 
-template <int CLS>
+// NRT: right-hand sides per task, 0 for mfma_task_rhs of the task's cell.
+template <int CLS, int NRT>
 __global__ __launch_bounds__(mfma_waves(CLS) * 64)
 __attribute__((amdgpu_waves_per_eu(mfma_eu(CLS), mfma_eu(CLS))))
 void k_batch_solve_mfma(SolveArgs A) {
@@ -693,13 +714,18 @@ void k_batch_solve_mfma(SolveArgs A) {
     const int cell = __builtin_amdgcn_readfirstlane(A.task_cell[task]);
     const int grp = __builtin_amdgcn_readfirstlane(A.task_group[task]);
     const Cell C = uniform_cell(A.cells, cell);
-    if constexpr (CLS == 3) {
+    constexpr int G = CLS == 3 ? 6 : CLS == 4 ? 4 : CLS == 2 ? 3 : CLS + 1;
+    if constexpr (NRT == 8) {
+      mfma_task<8, G, W>(A, C, cell, 8 * grp, P, P + C.nint * 24, P, partA, partB, S);
+    } else if constexpr (NRT == 12) {
+      mfma_task<12, G, W>(A, C, cell, 12 * grp, P, P + C.nint * 48, P + C.nint * 36, partA, partB, S);
+    } else if constexpr (CLS == 3) {
       if (C.nint > 384)
-        mfma_task<12, 6, W>(A, C, cell, 12 * grp, P, P + C.nint * 48, P + C.nint * 36, partA, partB, S);
+        mfma_task<12, G, W>(A, C, cell, 12 * grp, P, P + C.nint * 48, P + C.nint * 36, partA, partB, S);
       else
         mfma_task<24, 3, W>(A, C, cell, 0, P, P + C.nint * 108, P + C.nint * 72, partA, partB, S);
     } else {
-      mfma_task<24, CLS + 1, W>(A, C, cell, 0, P, P + C.nint * 108, P + C.nint * 72, partA, partB, S);
+      mfma_task<24, G, W>(A, C, cell, 0, P, P + C.nint * 108, P + C.nint * 72, partA, partB, S);
     }
   }
 }

@@ -2153,6 +2153,7 @@ struct mfs_batch_s {
   int seg[NQ + 1] = {};  // task ranges of the per-XCD queues
   bool tiled = false;    // every cell has n <= 10: mixed precision runs the matrix-core kernel
   int mseg[NQ + 1] = {};  // its task ranges
+  int task_rhs = 0;       // its right-hand sides per task (0: mfma_task_rhs of the cell)
   int64_t k32_total = 0;  // FP32 matrix values
   bool assembled = false;
   int tuned_wg[2] = {0, 0}, tuned_per_cu[2] = {0, 0};  // per precision (0 mixed, 1 FP64)
@@ -2282,10 +2283,17 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
   B->ntasks = (int)tc.size();
   std::vector<int> mc, mg;
   if (B->tiled) {
+    int64_t weights = 0, largest = 0;
+    for (const Cell& C : B->cells) {
+      const int64_t w = mfma_task_weight(C.n, C.nint);
+      weights += w;
+      largest = std::max(largest, w);
+    }
+    B->task_rhs = mfma_batch_rhs(weights, largest, ctx->cu_count);
     for (int q = 0; q < NQ; q++) {
       B->mseg[q] = (int)mc.size();
       for (size_t i = q; i < order.size(); i += NQ)
-        for (int g = 0; g < NB / mfma_task_rhs(B->cells[order[i]].nint); g++) {
+        for (int g = 0; g < NB / (B->task_rhs ? B->task_rhs : mfma_task_rhs(B->cells[order[i]].nint)); g++) {
           mc.push_back(order[i]);
           mg.push_back(g);
         }
@@ -2449,8 +2457,8 @@ static size_t lds_bytes(mfs_batch B, int prec, int var) {
 static size_t mfma_lds_bytes(mfs_batch B) {
   size_t need = 0;
   for (int n = 2; n <= B->max_n; n++) {
-    const int nint = (n - 1) * (n - 1) * (n - 1);
-    need = std::max(need, sizeof(float) * (size_t)nint * 3 * (mfma_task_rhs(nint) + 1 + 4 * mfma_d_lds(mfma_task_rhs(nint))));
+    const int nint = (n - 1) * (n - 1) * (n - 1), nr = B->task_rhs ? B->task_rhs : mfma_task_rhs(nint);
+    need = std::max(need, sizeof(float) * (size_t)nint * 3 * (nr + 1 + 4 * mfma_d_lds(nr)));
   }
   return need;
 }
@@ -2475,14 +2483,24 @@ static int batch_scratch(mfs_batch B, int precision, int per_cu, int var) {
 
 // Launch reset + persistent solve on the context stream (capturable: no
 // allocation, no memset; the queue and flags are cleared by a kernel).
+template <int NRT>
+static const void* mfma_kernel(int cls) {
+  switch (cls) {
+    case 0: return (const void*)k_batch_solve_mfma<0, NRT>;
+    case 1: return (const void*)k_batch_solve_mfma<1, NRT>;
+    case 2: return (const void*)k_batch_solve_mfma<2, NRT>;
+    case 4:
+      if constexpr (NRT == 8) return (const void*)k_batch_solve_mfma<4, NRT>;
+      [[fallthrough]];
+    default: return (const void*)k_batch_solve_mfma<3, NRT>;
+  }
+}
 static const void* batch_kernel(mfs_batch B, int precision, int var) {
   if (use_mfma(B, precision)) {
-    switch (mfma_class(B->max_nint)) {
-      case 0: return (const void*)k_batch_solve_mfma<0>;
-      case 1: return (const void*)k_batch_solve_mfma<1>;
-      case 2: return (const void*)k_batch_solve_mfma<2>;
-      default: return (const void*)k_batch_solve_mfma<3>;
-    }
+    const int cls = mfma_class(B->max_nint, B->task_rhs);
+    if (B->task_rhs == 8) return mfma_kernel<8>(cls);
+    if (B->task_rhs == 12) return mfma_kernel<12>(cls);
+    return mfma_kernel<0>(cls);
   }
   if (precision == MFS_PREC_F64) {
     switch (var) {
@@ -2497,7 +2515,7 @@ static const void* batch_kernel(mfs_batch B, int precision, int var) {
 }
 // Threads and dynamic LDS of a launch (the matrix-core kernel's are its own).
 static int launch_threads(mfs_batch B, int precision, int wg) {
-  return use_mfma(B, precision) ? 64 * mfma_waves(mfma_class(B->max_nint)) : wg;
+  return use_mfma(B, precision) ? 64 * mfma_waves(mfma_class(B->max_nint, B->task_rhs)) : wg;
 }
 static size_t launch_lds(mfs_batch B, int precision, int var) {
   return use_mfma(B, precision) ? mfma_lds_bytes(B) : lds_bytes(B, precision, var);

@@ -1,6 +1,6 @@
 """The matrix-core kernel of the mixed batched solve at the edges of its
 launch classes and tiles (16 nodes per instruction; 64 / 128 / 384 / 729
-interior nodes; 24 or 12 right-hand sides per task), against the oracle's
+interior nodes; 24, 12 or 8 right-hand sides per task), against the oracle's
 per-cell FP64 bases.
 
 Tolerance: every problem is solved to a true relative residual of 1e-10, and
@@ -48,6 +48,37 @@ def test_bases_match_oracle_at_class_and_tile_edges(ctx, sizes):
     assert rep.n_not_converged == 0 and rep.n_fallback == 24 * len(sizes)
     assert np.array_equal(B.iterations(), it0)
     B.close()
+
+
+@pytest.mark.parametrize("width", [12, 24])
+@pytest.mark.parametrize("sizes", [[2, 3, 4], [5, 3], [6, 5, 2], [7, 8, 4], [9, 6], [10, 8, 2, 9]])
+def test_wide_tasks_match_oracle_at_class_and_tile_edges(ctx, sizes, width):
+    """The lists above are batches small enough for tasks of 8 right-hand
+    sides.  Repeated until the tasks, counted as fractions of the largest
+    cell's (400 + n nint), come to 110 and to 160 cells, they run 12 and 24
+    per task (256 CUs); cells of n = 9, 10 keep 12."""
+    w = [400 + n * (n - 1) ** 3 for n in sizes]
+    copies = int(np.ceil({12: 110, 24: 160}[width] * max(w) / sum(w)))
+    B, origin, h, E = batch(ctx, sizes * copies, 5)
+    rep = B.solve(precision=mfs.PREC_MIXED, tol=1e-10)
+    assert rep.n_not_converged == 0 and rep.max_true_relres <= 1e-10
+    for c in list(range(len(sizes))) + list(range(B.ncells - len(sizes), B.ncells)):
+        ref, _, _ = orc.msfem_cell(B.cell_n[c], origin[c], h, E[c], 0.3, tol=1e-13)
+        err = np.linalg.norm(B.basis(c) - ref) / np.linalg.norm(ref)
+        assert err < 1e-8, (c, err)
+    B.close()
+
+
+@pytest.mark.parametrize("n", [7, 8])
+def test_few_cells_are_spread_over_the_chip(ctx, n):
+    """16 cells: with all right-hand sides of a cell in one task the mixed
+    solve took 1.4 (n = 7) and 1.6 (n = 8) times as long as the FP64 one,
+    which runs three tasks per cell; it must not be the slower one."""
+    B, *_ = batch(ctx, [n] * 16, 10)
+    t = [min(B.solve(precision=p, tol=1e-8).kernel_seconds for _ in range(5))
+         for p in (mfs.PREC_MIXED, mfs.PREC_F64)]
+    B.close()
+    assert t[0] < t[1], t
 
 
 def test_inner_products_add_every_product_in_fp64(ctx):

@@ -2149,6 +2149,7 @@ struct mfs_batch_s {
   std::vector<Cell> cells;
   int64_t total_int = 0, total_tets = 0;
   int max_n = 0, max_nint = 0;
+  int64_t sum_n = 0, sum_n5 = 0;  // over the cells: n, and n (n - 1)^4
   int ntasks = 0;
   int seg[NQ + 1] = {};  // task ranges of the per-XCD queues
   bool tiled = false;    // every cell has n <= 10: mixed precision runs the matrix-core kernel
@@ -2254,6 +2255,8 @@ extern "C" int mfs_batch_create(mfs_ctx ctx, const mfs_batch_desc* d, mfs_batch*
     i0 += C.nint;
     B->max_n = std::max(B->max_n, C.n);
     B->max_nint = std::max(B->max_nint, C.nint);
+    B->sum_n += C.n;
+    B->sum_n5 += (int64_t)C.n * (C.n - 1) * C.nint;
   }
   B->total_tets = t0;
   B->total_int = i0;
@@ -2635,17 +2638,38 @@ static int resident_per_cu(mfs_batch B, int precision, int wg, int var) {
   return std::max(1, std::min(nb, 8));
 }
 
-static int pick_shape(mfs_batch B, const mfs_batch_solve_desc* d, int* wg, int* per_cu, int* var) {
+// Register-resident kernel (a thread per row of the largest cell) or slab
+// kernel on 256 threads for an FP64 batch of several sizes.  Above 125 rows
+// the register form runs one workgroup per CU, and a task takes 0.06 ms x n
+// whatever its rows.  The slab form runs two; with all CUs busy a task costs
+// 0.06 ms x n x (0.55 + (n - 1)^4 / 620) of a CU (n = 3..8: 0.11 0.16 0.25 0.51
+// 1.1 2.1 ms), alone it takes 0.06 ms x n x (1.2 + nint / 230).  So registers
+// pay where the mean of (n - 1)^4, weighted by n, reaches 310, or where the slab
+// form's largest cell alone takes longer than all tasks in registers.
+//   registers / slab, ms: 512 cells of 8^3 5.1 / 15.7, of n = 3..7 (weighted
+//   mean 579) 3.9 / 6.0, 1,000 of 6^3 and one of 8^3 (630) 4.9 / 6.0, 3,600 of
+//   3^3 and 400 of 8^3 (560) 10.8 / 14.4, 2,000 of 5^3 and one of 8^3 (258)
+//   8.0 / 5.9, 3,000 of 4^3 and 200 of 7^3 (208) 8.9 / 8.4, 4,096 of 3^3 and one
+//   of 8^3 (18) 8.8 / 5.3, 250 of 3^3 and six of 8^3 0.76 / 1.6.  Up to 125 rows
+//   several workgroups fit a CU: 4,096 cells of 3^3 and one of 6^3 4.0 / 5.3.
+static bool f64_registers_pay(mfs_batch B) {
+  if (B->max_nint <= 125) return true;
+  if (B->sum_n5 >= 310 * B->sum_n) return true;
+  const double largest = B->max_n * (1.2 + B->max_nint / 230.0);
+  return (double)(NB / RG) * B->sum_n <= largest * B->ctx->cu_count;
+}
+
+// short_list: the FP64 pass over the problems that FP32 left, a few tasks
+static int pick_shape(mfs_batch B, const mfs_batch_solve_desc* d, bool short_list, int* wg, int* per_cu, int* var) {
   const int t = d->precision == MFS_PREC_F64 ? 1 : 0;
   int wgs = d->wg_size ? d->wg_size : (B->tuned_wg[t] ? B->tuned_wg[t] : 256);
   *var = d->variant > 0 ? d->variant - 1 : (B->tuned_var[t] >= 0 ? B->tuned_var[t] : 0);
   // FP64 with nothing asked for and nothing tuned: the register-resident
-  // kernel with a thread per row wherever every cell fits it (n <= 8; d and p
-  // take 143 KB of LDS there).  Against the slab kernel on 256 threads: 512
-  // cells of 8^3 5.1 / 15.7 ms, 1,000 cells of 5^3 1.17 / 3.29 ms, of n =
-  // 3..7 3.9 / 6.0 ms.
+  // kernel with a thread per row of the largest cell, where that one fits it
+  // (n <= 8; d and p take 143 KB of LDS there) and the others fill it
   const int rows = (B->max_nint + 63) / 64 * 64;
-  if (t == 1 && !d->wg_size && d->variant <= 0 && B->tuned_var[t] < 0 && variant_fits(B, d->precision, 2, rows)) {
+  if (t == 1 && !d->wg_size && d->variant <= 0 && B->tuned_var[t] < 0 && variant_fits(B, d->precision, 2, rows) &&
+      (short_list || f64_registers_pay(B))) {
     wgs = rows;
     *var = 2;
   }
@@ -2717,7 +2741,7 @@ extern "C" int mfs_batch_solve(mfs_batch B, const mfs_batch_solve_desc* d, mfs_b
   MFS_TRY(batch_check_desc(B, d));
   MFS_CHECK_ARG(rep, "mfs_batch_solve: report is NULL");
   int wg, pc, var;
-  MFS_TRY(pick_shape(B, d, &wg, &pc, &var));
+  MFS_TRY(pick_shape(B, d, false, &wg, &pc, &var));
   // Problems the FP32 inner iteration cannot solve (the reference's
   // indefinite local operators, see k_batch_solve) are solved again in FP64,
   // as the reference falls back to another solver (FEM/FEM.h:3726-3737),
@@ -2734,7 +2758,7 @@ extern "C" int mfs_batch_solve(mfs_batch B, const mfs_batch_solve_desc* d, mfs_b
   d64.wg_size = d->fallback_wg_size;
   int wg64 = 0, pc64 = 0, var64 = 0;
   if (mixed) {
-    MFS_TRY(pick_shape(B, &d64, &wg64, &pc64, &var64));
+    MFS_TRY(pick_shape(B, &d64, true, &wg64, &pc64, &var64));
     MFS_TRY(batch_scratch(B, MFS_PREC_F64, pc64, var64));
   }
   MFS_TRY(batch_scratch(B, d->precision, pc, var));

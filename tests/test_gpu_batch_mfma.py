@@ -190,3 +190,16 @@ def test_fp64_default_shape_matches_the_slab_kernel(ctx, sizes):
         ref = B.basis(c)
         assert np.linalg.norm(x[c] - ref) <= 1e-8 * np.linalg.norm(ref)
     B.close()
+
+
+@pytest.mark.parametrize("sizes", [[3] * 2000 + [8], [4] * 1000 + [7], [8] * 64])
+def test_fp64_default_is_not_slower_than_the_slab_kernel(ctx, sizes):
+    """A single large cell sized every workgroup of the register-resident
+    kernel for itself: 1.4 to 1.7 times the slab kernel's time in the first
+    two batches.  The default may not cost more than run-to-run noise; where
+    the cells fill its threads (the third) it is more than twice as fast."""
+    B, *_ = batch(ctx, sizes, 12)
+    t = [min(B.solve(precision=mfs.PREC_F64, tol=1e-8, **kw).kernel_seconds for _ in range(4))
+         for kw in ({}, dict(variant=1, wg_size=256))]
+    B.close()
+    assert t[0] <= (0.7 if sizes[0] == 8 else 1.15) * t[1], t

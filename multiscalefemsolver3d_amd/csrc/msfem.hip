@@ -279,7 +279,7 @@ __device__ __forceinline__ void elastic_block(const double* dI, const double* dJ
 }
 
 // ---------------------------------------------------------------------------
-// Cell assembly: one workgroup per cell, one thread per interior node.
+// Cell assembly: one thread per interior node.
 //
 // A tet steps from a hex corner along its three axes p0, p1, p2; times h the
 // gradients of its hat functions are -e_p0, e_p0 - e_p1, e_p1 - e_p2, e_p2.
@@ -294,9 +294,8 @@ __device__ __forceinline__ void elastic_block(const double* dI, const double* dJ
 // that the 72 sums of b exist once in the code).
 //
 // Bound by its stores (2.3 KB per node: K in FP64 and FP32, b) and, at nodes
-// next to the boundary, by b.  16^3 cells of n = 6..10: 2.7 ms (3.0 with the
-// moduli read from global memory instead of LDS); the gather over per-template
-// lists with the element recomputed per contribution took 3.9 ms.
+// next to the boundary, by b.  16^3 cells of n = 6..10: 2.6 ms; the gather over
+// per-template lists with the element recomputed per contribution took 3.9 ms.
 // ---------------------------------------------------------------------------
 // corner of local vertex I of tet p (bits x, y, z), and its gradient's signs
 __host__ __device__ constexpr int tet_axis(int p, int s) {
@@ -422,115 +421,154 @@ __device__ __forceinline__ void store_points(const CellK& C, const double (&w)[2
   }
 }
 
+// One node: its rows of K, the inverse diagonal and b.  weight(t) is the
+// modulus of the cell's tet t times h / 6.
+template <typename W>
+__device__ __forceinline__ void assemble_node(const Cell& C, const CellK& ck, int v, W weight,
+                                              const double* __restrict__ ft, float* __restrict__ dinv32,
+                                              double* __restrict__ dinv64, double* __restrict__ b64) {
+  const int n = C.n, m = n - 1;
+  const double rn = 1.0 / n;
+  const int i = v % m + 1, j = (v / m) % m + 1, k = v / (m * m) + 1;
+  {
+    double w[24];
+#pragma unroll
+    for (int p = 0; p < 6; p++)
+#pragma unroll
+      for (int I = 0; I < 4; I++) {
+        const int c = tet_corner(p, I);
+        const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
+        w[4 * p + I] = weight(6 * hex + p);
+      }
+    float pend[3][12];
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int q = 0; q < 12; q++) pend[a][q] = 0.f;
+    double diag[3];
+    store_points<0>(ck, w, v, i, j, k, pend, diag);
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      dinv64[(C.int0 + v) * 3 + a] = 1.0 / diag[a];
+      dinv32[(C.int0 + v) * 3 + a] = (float)(1.0 / diag[a]);
+    }
+  }
+  double bacc[3][NB];
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int q = 0; q < NB; q++) bacc[a][q] = 0.0;
+  if (i == 1 || i == m || j == 1 || j == m || k == 1 || k == m) {
+#pragma unroll 1
+    for (int s = 0; s < NS; s++) {
+      const int ni = i + c_stencil[s][0], nj = j + c_stencil[s][1], nk = k + c_stencil[s][2];
+      if (ni >= 1 && ni <= m && nj >= 1 && nj <= m && nk >= 1 && nk <= m) continue;
+      double S[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+      for (int e = 0; e < 6; e++) {
+        const uint32_t code = c_tets.pt[s].code[e];
+        const int p = code & 7, c = (code >> 3) & 7;
+        const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
+        const double w = weight(6 * hex + p);
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          const double wa = w * (double)((int)((code >> (6 + 2 * a)) & 3) - 1);
+#pragma unroll
+          for (int b = 0; b < 3; b++) S[a][b] += wa * (double)((int)((code >> (12 + 2 * b)) & 3) - 1);
+        }
+      }
+      double Kb[3][3];
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) Kb[a][b] = block_entry(ck, S, a, b);
+      if (ft == nullptr) {
+        // g for basis (c, d) at this boundary node: hat_c(x) e_d
+        const double X = ni == n ? 1.0 : ni * rn, Y = nj == n ? 1.0 : nj * rn, Z = nk == n ? 1.0 : nk * rn;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+          const double hat = ((c & 1) ? X : 1 - X) * ((c & 2) ? Y : 1 - Y) * ((c & 4) ? Z : 1 - Z);
+#pragma unroll
+          for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int a = 0; a < 3; a++) bacc[a][3 * c + d] -= Kb[a][d] * hat;
+        }
+      } else {
+        // g from the face traces (reference-trace mode): full vectors
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+          const double* g = face_trace_of(ft + C.ft0, n, ni, nj, nk, c);
+          if (!g) continue;
+#pragma unroll
+          for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+              bacc[a][3 * c + d] -= Kb[a][0] * g[d] + Kb[a][1] * g[12 + d] + Kb[a][2] * g[24 + d];
+        }
+      }
+    }
+  }
+  double2* bv = reinterpret_cast<double2*>(b64 + (C.int0 + v) * (3 * NB));
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int q = 0; q < NB; q += 2) bv[(a * NB + q) / 2] = make_double2(bacc[a][q], bacc[a][q + 1]);
+}
+__device__ __forceinline__ CellK cell_matrix(const Cell& C, double nu, int conv, int tiled, float* K32, double* K64) {
+  const double lam = nu / ((1.0 + nu) * (1.0 - 2.0 * nu)), mu = 1.0 / (2.0 * (1.0 + nu));
+  CellK ck;
+  ck.K64 = K64 + C.int0 * (NS * 9);
+  ck.K32 = K32 + C.kt0;
+  ck.nint = C.nint;
+  ck.m = C.n - 1;
+  ck.tiled = tiled;
+  ck.F = conv == MFS_ELEM_TEXTBOOK ? lam : mu;
+  ck.H = conv == MFS_ELEM_TEXTBOOK ? mu : lam;
+  ck.mu = mu;
+  return ck;
+}
+
 constexpr int kAsmThreads = 128;  // 125 .. 729 nodes per cell: few idle lanes
+// A workgroup per cell, its moduli staged in LDS: every one is read 4 times
+// by the nodes of its tet and again for b.
 __global__ __launch_bounds__(kAsmThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_cell_assemble(const Cell* __restrict__ cells, const double* __restrict__ E, double nu, double h, int conv,
                      const double* __restrict__ ft, int tiled, float* __restrict__ K32, double* __restrict__ K64,
                      float* __restrict__ dinv32, double* __restrict__ dinv64, double* __restrict__ b64) {
   const Cell C = uniform_cell(cells, blockIdx.x);
-  const int n = C.n, m = n - 1, nint = C.nint;
-  const double hf = h / n, rn = 1.0 / n;
-  const double lam = nu / ((1.0 + nu) * (1.0 - 2.0 * nu)), mu = 1.0 / (2.0 * (1.0 + nu));
-  CellK ck;
-  ck.K64 = K64 + C.int0 * (NS * 9);
-  ck.K32 = K32 + C.kt0;
-  ck.nint = nint;
-  ck.m = m;
-  ck.tiled = tiled;
-  ck.F = conv == MFS_ELEM_TEXTBOOK ? lam : mu;
-  ck.H = conv == MFS_ELEM_TEXTBOOK ? mu : lam;
-  ck.mu = mu;
-  // the cell's moduli, times h / 6, in LDS: every one is read 4 times by the
-  // nodes of its tet and again for b
+  const int n = C.n;
+  const double hf = h / n;
+  const CellK ck = cell_matrix(C, nu, conv, tiled, K32, K64);
   extern __shared__ double w_lds[];
   for (int t = threadIdx.x; t < 6 * n * n * n; t += kAsmThreads) w_lds[t] = E[C.tet0 + t] * (hf / 6.0);
   __syncthreads();
-  for (int v = threadIdx.x; v < nint; v += kAsmThreads) {
-    const int i = v % m + 1, j = (v / m) % m + 1, k = v / (m * m) + 1;
-    {
-      double w[24];
-#pragma unroll
-      for (int p = 0; p < 6; p++)
-#pragma unroll
-        for (int I = 0; I < 4; I++) {
-          const int c = tet_corner(p, I);
-          const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
-          w[4 * p + I] = w_lds[6 * hex + p];
-        }
-      float pend[3][12];
-#pragma unroll
-      for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int q = 0; q < 12; q++) pend[a][q] = 0.f;
-      double diag[3];
-      store_points<0>(ck, w, v, i, j, k, pend, diag);
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        dinv64[(C.int0 + v) * 3 + a] = 1.0 / diag[a];
-        dinv32[(C.int0 + v) * 3 + a] = (float)(1.0 / diag[a]);
-      }
-    }
-    double bacc[3][NB];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int q = 0; q < NB; q++) bacc[a][q] = 0.0;
-    if (i == 1 || i == m || j == 1 || j == m || k == 1 || k == m) {
-#pragma unroll 1
-      for (int s = 0; s < NS; s++) {
-        const int ni = i + c_stencil[s][0], nj = j + c_stencil[s][1], nk = k + c_stencil[s][2];
-        if (ni >= 1 && ni <= m && nj >= 1 && nj <= m && nk >= 1 && nk <= m) continue;
-        double S[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll
-        for (int e = 0; e < 6; e++) {
-          const uint32_t code = c_tets.pt[s].code[e];
-          const int p = code & 7, c = (code >> 3) & 7;
-          const int hex = (i - (c & 1)) + n * ((j - ((c >> 1) & 1)) + n * (k - (c >> 2)));
-          const double w = w_lds[6 * hex + p];
-#pragma unroll
-          for (int a = 0; a < 3; a++) {
-            const double wa = w * (double)((int)((code >> (6 + 2 * a)) & 3) - 1);
-#pragma unroll
-            for (int b = 0; b < 3; b++) S[a][b] += wa * (double)((int)((code >> (12 + 2 * b)) & 3) - 1);
-          }
-        }
-        double Kb[3][3];
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-#pragma unroll
-          for (int b = 0; b < 3; b++) Kb[a][b] = block_entry(ck, S, a, b);
-        if (ft == nullptr) {
-          // g for basis (c, d) at this boundary node: hat_c(x) e_d
-          const double X = ni == n ? 1.0 : ni * rn, Y = nj == n ? 1.0 : nj * rn, Z = nk == n ? 1.0 : nk * rn;
-#pragma unroll
-          for (int c = 0; c < 8; c++) {
-            const double hat = ((c & 1) ? X : 1 - X) * ((c & 2) ? Y : 1 - Y) * ((c & 4) ? Z : 1 - Z);
-#pragma unroll
-            for (int d = 0; d < 3; d++)
-#pragma unroll
-              for (int a = 0; a < 3; a++) bacc[a][3 * c + d] -= Kb[a][d] * hat;
-          }
-        } else {
-          // g from the face traces (reference-trace mode): full vectors
-#pragma unroll
-          for (int c = 0; c < 8; c++) {
-            const double* g = face_trace_of(ft + C.ft0, n, ni, nj, nk, c);
-            if (!g) continue;
-#pragma unroll
-            for (int d = 0; d < 3; d++)
-#pragma unroll
-              for (int a = 0; a < 3; a++)
-                bacc[a][3 * c + d] -= Kb[a][0] * g[d] + Kb[a][1] * g[12 + d] + Kb[a][2] * g[24 + d];
-          }
-        }
-      }
-    }
-    double2* bv = reinterpret_cast<double2*>(b64 + (C.int0 + v) * (3 * NB));
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int q = 0; q < NB; q += 2) bv[(a * NB + q) / 2] = make_double2(bacc[a][q], bacc[a][q + 1]);
+  for (int v = threadIdx.x; v < C.nint; v += kAsmThreads)
+    assemble_node(C, ck, v, [&](int t) { return w_lds[t]; }, ft, dinv32, dinv64, b64);
+}
+// A thread per node of the whole batch, the moduli read through the caches.
+__global__ __launch_bounds__(kAsmThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_node_assemble(const Cell* __restrict__ cells, int ncells, int64_t total_int, const double* __restrict__ E,
+                     double nu, double h, int conv, const double* __restrict__ ft, int tiled, float* __restrict__ K32,
+                     double* __restrict__ K64, float* __restrict__ dinv32, double* __restrict__ dinv64,
+                     double* __restrict__ b64) {
+  const int64_t gv = blockIdx.x * (int64_t)kAsmThreads + threadIdx.x;
+  if (gv >= total_int) return;
+  int lo = 0, hi = ncells - 1;  // the cell: the last one that starts at or before gv
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (cells[mid].int0 <= gv)
+      lo = mid;
+    else
+      hi = mid - 1;
   }
+  const Cell C = cells[lo];
+  const double hf = h / C.n;
+  const double* Ec = E + C.tet0;
+  auto weight = [&](int t) {
+#pragma clang fp contract(off)  // rounded before it is added, as the staged one is
+    return Ec[t] * (hf / 6.0);
+  };
+  assemble_node(C, cell_matrix(C, nu, conv, tiled, K32, K64), (int)(gv - C.int0), weight, ft, dinv32, dinv64, b64);
 }
 
 // ---------------------------------------------------------------------------
@@ -2366,6 +2404,26 @@ extern "C" int mfs_batch_cell_dofs(mfs_batch B, int cell, int64_t* n_interior, i
   return MFS_OK;
 }
 
+// A workgroup per cell leaves lanes idle in cells smaller than the largest,
+// takes a cell's passes of 128 nodes one after the other, and its LDS is sized
+// by the largest cell; a thread per node has none of that but reads the moduli
+// through the caches and searches for its cell.  ms by cell / by node, with
+// transfers of the call:
+//   one pass: 512 cells of 2^3 0.060 / 0.076, 4,096 0.207 / 0.079; 4,096 of 6^3
+//   (lanes 98 % used) 0.94 / 1.01, of 5^3 (50 %) 0.47 / 0.53, 1,000 of 3..6 (44 %)
+//   0.146 / 0.113, 20,000 of 3^3 (6 %) 0.92 / 0.41, of 2^3 0.87 / 0.10, these and
+//   one of 12^3 3.2 / 0.11;
+//   more: 1 cell of 12^3 0.41 / 0.06, 256 of 8^3 0.167 / 0.141, 384 0.23 / 0.28
+//   and 512 0.28 / 0.34 (here a thread per node needs a second, mostly empty
+//   round of blocks), 1,024 0.64 / 0.63, 4,096 2.59 / 2.40, 384 of 12^3 0.99 /
+//   0.80, 4,096 of 6..10 2.70 / 2.63.
+static bool assemble_by_cell(mfs_batch B) {
+  const int64_t cus = B->ctx->cu_count, passes = (B->max_nint + kAsmThreads - 1) / kAsmThreads;
+  const double used = (double)B->total_int / ((double)B->ncells * passes * kAsmThreads);
+  if (passes == 1) return used >= 0.48 || B->ncells <= 3 * cus;
+  return used >= 0.6 && 2 * B->ncells >= (passes <= 6 ? 3 : 4) * cus && B->ncells <= 4 * cus;
+}
+
 extern "C" int mfs_batch_assemble(mfs_batch B) {
   MFS_CHECK_ARG(B, "mfs_batch_assemble: NULL batch");
   hipStream_t s = B->ctx->stream;
@@ -2396,11 +2454,17 @@ extern "C" int mfs_batch_assemble(mfs_batch B) {
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
   }
-  const size_t asm_lds = sizeof(double) * 6 * B->max_n * B->max_n * B->max_n;  // 83 KB at n = 12
-  (void)hipFuncSetAttribute((const void*)k_cell_assemble, hipFuncAttributeMaxDynamicSharedMemorySize, (int)asm_lds);
-  k_cell_assemble<<<B->ncells, kAsmThreads, asm_lds, s>>>(B->d_cells, B->d_E, B->nu, B->h, B->conv, B->d_ft,
-                                                    B->tiled ? 1 : 0, B->d_K32, B->d_K64, B->d_dinv32, B->d_dinv64,
-                                                    B->d_b64);
+  if (!assemble_by_cell(B)) {
+    k_node_assemble<<<(unsigned)((B->total_int + kAsmThreads - 1) / kAsmThreads), kAsmThreads, 0, s>>>(
+        B->d_cells, B->ncells, B->total_int, B->d_E, B->nu, B->h, B->conv, B->d_ft, B->tiled ? 1 : 0, B->d_K32,
+        B->d_K64, B->d_dinv32, B->d_dinv64, B->d_b64);
+  } else {
+    const size_t lds = sizeof(double) * 6 * B->max_n * B->max_n * B->max_n;  // 83 KB at n = 12
+    (void)hipFuncSetAttribute((const void*)k_cell_assemble, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    k_cell_assemble<<<B->ncells, kAsmThreads, lds, s>>>(B->d_cells, B->d_E, B->nu, B->h, B->conv, B->d_ft,
+                                                        B->tiled ? 1 : 0, B->d_K32, B->d_K64, B->d_dinv32,
+                                                        B->d_dinv64, B->d_b64);
+  }
   MFS_HIP(hipGetLastError());
   MFS_HIP(hipStreamSynchronize(s));
   B->assembled = true;

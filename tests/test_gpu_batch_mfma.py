@@ -203,3 +203,41 @@ def test_fp64_default_is_not_slower_than_the_slab_kernel(ctx, sizes):
          for kw in ({}, dict(variant=1, wg_size=256))]
     B.close()
     assert t[0] <= (0.7 if sizes[0] == 8 else 1.15) * t[1], t
+
+
+@pytest.mark.parametrize("by_cell,by_node", [([5] * 6, [5] * 6 + [2] * 3000), ([8] * 600, [8] * 300),
+                                             ([10] * 600, [10] * 300)])
+def test_both_assembly_forms_give_the_same_bits(ctx, by_cell, by_node):
+    """The first batch is assembled by a workgroup per cell, the second by a
+    thread per node (256 CUs).  A node's operations are the same, and so are
+    then the iterates of its cell, in FP64 (K64, b, the FP64 diagonal) and,
+    where both batches run tasks of the same width, in mixed precision."""
+    x = []
+    for sizes in (by_cell, by_node):
+        B, *_ = batch(ctx, sizes, 13)
+        for kw in (dict(precision=mfs.PREC_F64, variant=1, wg_size=256), dict(precision=mfs.PREC_MIXED)):
+            if sizes[0] == 5 and kw["precision"] == mfs.PREC_MIXED:
+                continue
+            B.solve(check=False, tol=1e-8, maxit=30, **kw)
+            x.append([B.basis(c) for c in (0, 5)])
+        B.close()
+    half = len(x) // 2
+    assert all(np.array_equal(p, q) for p, q in zip(x[:half], x[half:]))
+
+
+def test_one_large_cell_does_not_slow_the_assembly(ctx):
+    """One cell of 12^3 behind 20,000 of 2^3 sized every workgroup's LDS and
+    made the assembly 3.7 times as slow."""
+    import time
+    t = []
+    for sizes in ([2] * 20000, [2] * 20000 + [12]):
+        B = mfs.Batch(ctx, sizes, [[c, 0, 0] for c in range(len(sizes))], 1.0,
+                      np.full(sum(6 * k ** 3 for k in sizes), 1e9), 0.3)
+        best = 1.0
+        for _ in range(6):
+            t0 = time.perf_counter()
+            B.assemble()
+            best = min(best, time.perf_counter() - t0)
+        t.append(best)
+        B.close()
+    assert t[1] <= 2 * t[0], t

@@ -413,17 +413,27 @@ __global__ void k_mr_state(MrState* st, const double* tol2, int k, int maxit) {
   }
 }
 
+// Waves per SIMD of k_mr_dir_spmm.  The scalar FP64 products are bound by
+// gathers of 32 to 64 bytes per entry and operand, and more waves than these
+// evict each other's lines: 6 systems 64^3 106 us per iteration with 5 waves,
+// 85 with 4; 100^3 302 and 234; 8 systems 417 with 4, 344 with 3; 4 systems
+// 169 with 8, 154 with 6.  The other forms run what their registers allow.
+template <typename T, int BS, int KR>
+constexpr int mr_max_waves() {
+  return BS == 1 && sizeof(T) == 8 ? (KR <= 4 ? 6 : KR <= 6 ? 4 : 3) : 8;
+}
+
 // K1: stop tests and beta per system from K2's partials; P_new = Z + beta
 // P_old (own rows written, gathered rows formed on the fly); Q = A P_new;
 // partials p.q per system.
 template <typename T, int BS, int KR, typename CI>
-__global__ __launch_bounds__(256) void k_mr_dir_spmm(const int64_t* __restrict__ slice_base,
-                                                     const int32_t* __restrict__ slice_width,
-                                                     const CI* __restrict__ col, const T* __restrict__ val,
-                                                     const T* __restrict__ Z, const T* __restrict__ P_old,
-                                                     T* __restrict__ P_new, T* __restrict__ Q, int64_t nb,
-                                                     int64_t n_slices, MrState* st, const double* __restrict__ part_rz,
-                                                     unsigned g_rz, double* __restrict__ part_pq, int xcd) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, (mr_max_waves<T, BS, KR>()))))
+void k_mr_dir_spmm(const int64_t* __restrict__ slice_base, const int32_t* __restrict__ slice_width,
+                   const CI* __restrict__ col, const T* __restrict__ val,
+                   const T* __restrict__ Z, const T* __restrict__ P_old,
+                   T* __restrict__ P_new, T* __restrict__ Q, int64_t nb,
+                   int64_t n_slices, MrState* st, const double* __restrict__ part_rz,
+                   unsigned g_rz, double* __restrict__ part_pq, int xcd) {
   if (st->alldone) return;
   double t[2 * KR];
   mr_sum_partials<2 * KR, 4>(part_rz, g_rz, t);

@@ -991,14 +991,19 @@ struct MinresEngine {
     for (hipEvent_t& e : ev)
       if (!e) MFS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     MinresState* hs = (MinresState*)A->ctx->pinned;
+    int64_t left = (int64_t)maxsteps + 1;  // k_mr_spmv launches until the cap stops the run
     auto submit = [&](int slot) -> int {
-      if (use_graph) {
+      // a cap inside the chunk: the launches past it would find nothing to do
+      // (3 steps of a 100^3 scalar system 0.51 ms with them, 0.43 without)
+      const int steps = (int)std::min<int64_t>(kChunk, left);
+      left -= steps;
+      if (use_graph && steps == kChunk) {
         MFS_HIP(hipGraphLaunch(exec, s));
       } else {
-        for (int t = 0; t < kChunk; t++) launch_step(s, t);
+        for (int t = 0; t < steps; t++) launch_step(s, t);
         MFS_HIP(hipGetLastError());
       }
-      MFS_HIP(hipMemcpyAsync(hs + slot, st, sizeof(MinresState), hipMemcpyDeviceToHost, s));  // kChunk is even
+      MFS_HIP(hipMemcpyAsync(hs + slot, st + steps % 2, sizeof(MinresState), hipMemcpyDeviceToHost, s));
       MFS_HIP(hipEventRecord(ev[slot], s));
       return MFS_OK;
     };

@@ -41,11 +41,13 @@ def test_bases_match_oracle(ctx, small, precision):
     (p, v, w) for p in (mfs.PREC_MIXED, mfs.PREC_F64)
     for v, w in ((1, 64), (1, 256), (2, 64), (2, 192), (3, 64), (3, 512), (4, 64), (4, 192))])
 def test_kernel_variants_and_shapes_match_oracle(ctx, small, precision, variant, wg):
-    """Every kernel variant (rows carried per thread; variants 3 and 4 keep
-    the rows' vectors in registers) at small and large workgroups, where
+    """FP64: every kernel variant (rows carried per thread; variants 3 and 4
+    keep the rows' vectors in registers) at small and large workgroups, where
     rows per thread exceed or fall short of the variant's interleave (with
     192 or 512 threads most threads of variants 3 and 4 own no row of these
-    cells), gives the oracle's bases."""
+    cells), gives the oracle's bases.  MIXED: these shapes are accepted, and
+    the matrix-core kernel, which has a shape of its own, gives the oracle's
+    bases for each (its vector kernels are tested on larger cells below)."""
     p, B = small
     rep = B.solve(precision=precision, tol=1e-10, use_graph=False, variant=variant, wg_size=wg)
     assert rep.n_not_converged == 0 and rep.max_true_relres <= 1e-10
@@ -56,11 +58,53 @@ def test_kernel_variants_and_shapes_match_oracle(ctx, small, precision, variant,
         assert err < 1e-8, (c, err)
 
 
+@pytest.fixture(scope="module")
+def large(ctx):
+    """Cells too large for the matrix-core kernel (n > 10), and a small one."""
+    sizes = [12, 3, 11]
+    g = np.random.default_rng(17)
+    E = [np.exp(np.log(1e9) + 0.3 * g.standard_normal(6 * n ** 3)) for n in sizes]
+    origin = np.array([[0, 0, 0], [0.25, 0, 0], [0.5, 0, 0]])
+    B = mfs.Batch(ctx, sizes, origin, 0.25, np.concatenate(E), 0.3)
+    B.assemble()
+    yield B, [orc.msfem_cell(n, o, 0.25, e, 0.3, tol=1e-13)[0] for n, o, e in zip(sizes, origin, E)]
+    B.close()
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2])
+@pytest.mark.parametrize("wg", [0, 64, 192, 256])
+def test_mixed_vector_kernels_match_oracle(large, variant, wg):
+    """MIXED on cells of n = 11, 12: two and three rows per thread, small and
+    large workgroups and the default shape.  The true residuals are 1e-10 and
+    the Jacobi-scaled condition numbers below 1e2 for these moduli."""
+    B, ref = large
+    rep = B.solve(precision=mfs.PREC_MIXED, tol=1e-10, variant=variant, wg_size=wg)
+    assert rep.n_not_converged == 0 and rep.max_true_relres <= 1e-10
+    for c, r in enumerate(ref):
+        assert np.linalg.norm(B.basis(c) - r) / np.linalg.norm(r) < 1e-8, c
+
+
+def test_mixed_vector_kernels_are_autotuned(large):
+    """The autotuner times both variants on these cells and the solve that
+    follows runs the shape it chose."""
+    B, ref = large
+    wg, per_cu, variant, ms = B.autotune(precision=mfs.PREC_MIXED, tol=1e-8)
+    assert wg in (64, 128, 192, 256) and per_cu >= 1 and variant in (0, 1) and ms > 0
+    rep = B.solve(precision=mfs.PREC_MIXED, tol=1e-10)
+    assert rep.n_not_converged == 0
+    for c, r in enumerate(ref):
+        assert np.linalg.norm(B.basis(c) - r) / np.linalg.norm(r) < 1e-8, c
+    for kw in (dict(variant=3, wg_size=512), dict(variant=4, wg_size=256), dict(variant=1, wg_size=320)):
+        with pytest.raises(mfs.MfsError, match="register-resident"):
+            B.solve(precision=mfs.PREC_MIXED, tol=1e-8, **kw)
+
+
 def test_register_variant_rejects_cells_larger_than_the_workgroup(ctx):
     """Variants 3 and 4 hold each row of a cell in one thread's registers: a
     cell of 8^3 hexes (343 interior nodes) does not fit 256 threads x 1 row
-    or 64 threads x 2 rows, and such solves are refused instead of run; the
-    shapes that fit give the slab variant's solution in both precisions."""
+    or 64 threads x 2 rows, and such shapes are refused in both precisions,
+    though mixed precision runs a kernel of its own shape here; the shapes
+    that fit give the slab variant's solution."""
     p = problems.msfem_cells(1, n_fixed=8, seed_E=3)
     B = make_batch(ctx, p)
     for var, wg in ((3, 256), (4, 64), (4, 384)):

@@ -74,30 +74,6 @@ struct MfmaRhs {  // per right-hand side of the running task
   int itmin[2][NB], done[NB], failed[NB], warm[NB], itbase[NB], it[NB];
 };
 
-// lane l of every row of 16 gets lane (l + 4) % 16's (or l ^ 8's) value
-__device__ __forceinline__ double row_ror4_f64(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x124, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x124, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-// x + y after swapping the upper half (32) or the odd rows (16) of x with the
-// lower half / even rows of y: with x = y every lane gets the sum over the
-// two halves, else the halves keep the sums of x and of y
-template <int O>
-__device__ __forceinline__ double swap_add(double x, double y) {
-  const unsigned xl = (unsigned)__double2loint(x), xh = (unsigned)__double2hiint(x);
-  const unsigned yl = (unsigned)__double2loint(y), yh = (unsigned)__double2hiint(y);
-  if constexpr (O == 32) {
-    const auto l = __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
-    const auto h = __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
-  } else {
-    const auto l = __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
-    const auto h = __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
-  }
-}
-
 // Workgroup sums of C values per lane (v[j] of right-hand side C c + j) over
 // the 16 blocks of a wave and over the waves, in two steps: mfma_wave_sums
 // leaves the wave's sums in part[wave][j][c], and after a barrier
@@ -114,8 +90,8 @@ __device__ __forceinline__ void mfma_wave_sums(const double (&v)[C], double* par
   for (int i = 0; i < N; i++) {
     a[i] = swap_add<32>(v[i], split ? v[N + i] : v[i]);
     a[i] = swap_add<16>(a[i], a[i]);
-    a[i] += row_ror8_f64(a[i]);
-    a[i] += row_ror4_f64(a[i]);
+    a[i] += row_rotated<0x128>(a[i]);
+    a[i] += row_rotated<0x124>(a[i]);
   }
   if ((lane & 28) == 0 && (split || lane < 32))
 #pragma unroll
@@ -340,7 +316,7 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
 #pragma unroll
           for (int q = 0; q < 3; q++)
 #pragma unroll
-            for (int e = 0; e < 9; e++) kn[q][e] = buffer_load<double>(rs64, 8 * vi, (9 * q + e) * stride);
+            for (int e = 0; e < 9; e++) kn[q][e] = buffer_load_f64(rs64, 8 * vi, (9 * q + e) * stride);
 #pragma unroll 1
           for (int s0 = 0; s0 < NS; s0 += 3) {
 #pragma unroll
@@ -356,7 +332,7 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
                 }
               const int next = min(s0 + q + 3, NS - 1) * 9;  // (past the last point: not used)
 #pragma unroll
-              for (int e = 0; e < 9; e++) kn[q][e] = buffer_load<double>(rs64, 8 * vi, (next + e) * stride);
+              for (int e = 0; e < 9; e++) kn[q][e] = buffer_load_f64(rs64, 8 * vi, (next + e) * stride);
               __builtin_amdgcn_sched_barrier(0);
             }
           }

@@ -136,35 +136,44 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// The FP64 sum in registers: the same additions without the LDS crossbar's
-// six round trips, which stand in every reduction of an iteration kernel.
-// lane ^ 32 and lane ^ 16 by the half and row swaps; the sums are then equal
-// in the lanes 8 (then 4, 2) apart, so rotating a row by 8, 4, 2, 1 reaches
-// the value of lane ^ 8, ^ 4, ^ 2, ^ 1.  All 64 lanes must be active.
-// PCG solve 12^3 FP64 9.9 -> 9.1 us per iteration, 64^3 mixed 14.7 -> 13.8.
+// Lane exchanges of FP64 values without the LDS crossbar; all 64 lanes must be
+// active.
+// Rotation of the rows of 16 lanes (CTRL 0x120 + k: by k lanes).
 template <int CTRL>
 __device__ __forceinline__ double row_rotated(double v) {
   const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
   return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
-__device__ __forceinline__ double wave_sum(double v) {
+// x + y after swapping the upper half (O = 32) or the odd rows (O = 16) of x
+// with the lower half / even rows of y: with x = y every lane gets the sum over
+// the two halves, else the halves keep the sums of x and of y.
+template <int O>
+__device__ __forceinline__ double swap_add(double x, double y) {
+  const unsigned long long xb = __builtin_bit_cast(unsigned long long, x), yb = __builtin_bit_cast(unsigned long long, y);
   auto pair = [](unsigned lo, unsigned hi) {
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
   };
-  {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    v = pair(lo[0], hi[0]) + pair(lo[1], hi[1]);
+  if constexpr (O == 32) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)xb, (unsigned)yb, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(xb >> 32), (unsigned)(yb >> 32), false, false);
+    return pair(lo[0], hi[0]) + pair(lo[1], hi[1]);
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)xb, (unsigned)yb, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(xb >> 32), (unsigned)(yb >> 32), false, false);
+    return pair(lo[0], hi[0]) + pair(lo[1], hi[1]);
   }
-  {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    v = pair(lo[0], hi[0]) + pair(lo[1], hi[1]);
-  }
+}
+// The FP64 sum in registers: the same additions without the crossbar's six
+// round trips, which stand in every reduction of an iteration kernel.
+// lane ^ 32 and lane ^ 16 by the half and row swaps; the sums are then equal
+// in the lanes 8 (then 4, 2) apart, so rotating a row by 8, 4, 2, 1 reaches
+// the value of lane ^ 8, ^ 4, ^ 2, ^ 1.
+// PCG solve 12^3 FP64 9.9 -> 9.1 us per iteration, 64^3 mixed 14.7 -> 13.8.
+__device__ __forceinline__ double wave_sum(double v) {
+  v = swap_add<32>(v, v);
+  v = swap_add<16>(v, v);
   v += row_rotated<0x128>(v);
   v += row_rotated<0x124>(v);
   v += row_rotated<0x122>(v);

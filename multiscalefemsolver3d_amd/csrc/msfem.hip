@@ -71,8 +71,9 @@ constexpr int MAXN = 12; // largest supported cell subdivision (FP32 inner; FP64
 // registers for two waves per SIMD), and whether the per-row vectors r, d, q
 // live in registers (FP64 variants 3 and 4; only for batches whose cells all
 // have nint <= rows * workgroup size) or in a global scratch slab.  In mixed
-// precision variants 3 and 4 exist for cells that the matrix-core kernel
-// takes (n <= 10), which then serves all four.
+// precision variants 3 and 4 are numbers that callers may pass for cells of
+// n <= 8, within the limits of a register form's rows and workgroup; the
+// matrix-core kernel serves every shape accepted on cells of n <= 10.
 constexpr int kRptF32[4] = {2, 3, 1, 2}, kRptF64[4] = {1, 2, 1, 2};
 constexpr bool kRegVar[4] = {false, false, true, true};
 constexpr int kVariants[2] = {4, 4};  // per precision: FP32 inner, FP64 inner
@@ -172,9 +173,10 @@ __host__ __device__ __forceinline__ void hat_trace_at(int n, int i, int j, int k
 }
 
 // Task queues: one per XCD.  Workgroups are dispatched round-robin over the
-// 8 XCDs, so workgroup b pulls from queue b % 8 first; all three tasks of a
-// cell sit in the same queue, so the cell matrix they stream stays in one
-// XCD's L2.  An exhausted queue sends the workgroup on to the next one.
+// 8 XCDs, so workgroup b pulls from queue b % 8 first; a cell's tasks (three in
+// k_batch_solve, one to three in the matrix-core kernel) sit in one queue, so
+// where there are several they read the cell matrix through one XCD's L2.  An
+// exhausted queue sends the workgroup on to the next one.
 constexpr int NQ = 8;
 constexpr int QSTRIDE = 32;  // counters 128 bytes apart
 
@@ -586,14 +588,7 @@ constexpr uint32_t kOffI = pack_offsets(0), kOffJ = pack_offsets(1), kOffK = pac
 // Loads through a raw buffer resource (gfx9 descriptor word 3; the range
 // check returns 0 beyond num_records).
 constexpr int kBufferRsrcWord3 = 0x00020000;
-template <typename KT>
-__device__ __forceinline__ KT buffer_load(__amdgpu_buffer_rsrc_t rs, int voff, int soff);
-template <>
-__device__ __forceinline__ float buffer_load<float>(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, 0));
-}
-template <>
-__device__ __forceinline__ double buffer_load<double>(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+__device__ __forceinline__ double buffer_load_f64(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
 }
 
@@ -770,25 +765,26 @@ __device__ __forceinline__ void phase_direction(int nint, const T* __restrict__ 
 }
 
 // K of one cell through a buffer resource: the row's byte offset is the
-// (per-thread) VGPR offset and the entry's byte offset (s*9+e)*nint*sizeof(KT)
+// (per-thread) VGPR offset and the entry's byte offset (s*9+e)*nint*8
 // the (uniform) SGPR offset, so a load costs no vector address arithmetic.
 // The stride is redefined for the compiler on every call, so the 135 entry
 // offsets are formed where they are used instead of being hoisted out of
 // the iteration loop.
-template <typename KT, int RPT>
+template <int RPT>
 struct KRows {
   __amdgpu_buffer_rsrc_t rs;
   int vo[RPT];
   int stride;
-  __device__ __forceinline__ KRows(const KT* Kc, int nint, const int (&vi)[RPT]) {
-    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<KT*>(Kc), (short)0, NS * 9 * nint * (int)sizeof(KT),
-                                           kBufferRsrcWord3);
+  __device__ __forceinline__ KRows(const double* Kc, int nint, const int (&vi)[RPT]) {
+    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(Kc), (short)0, NS * 9 * nint * 8, kBufferRsrcWord3);
 #pragma unroll
-    for (int q = 0; q < RPT; q++) vo[q] = vi[q] * (int)sizeof(KT);
-    stride = nint * (int)sizeof(KT);
+    for (int q = 0; q < RPT; q++) vo[q] = vi[q] * 8;
+    stride = nint * 8;
     asm volatile("" : "+s"(stride));
   }
-  __device__ __forceinline__ KT at(int q, int s, int e) const { return buffer_load<KT>(rs, vo[q], (s * 9 + e) * stride); }
+  __device__ __forceinline__ double at(int q, int s, int e) const {
+    return buffer_load_f64(rs, vo[q], (s * 9 + e) * stride);
+  }
 };
 
 template <int RPT>
@@ -799,12 +795,12 @@ __device__ __forceinline__ void clamp_rows(const int (&v)[RPT], const bool (&ok)
 
 // Requests the K values of stencil points 0 .. PF-1 into the ring that
 // stencil_rows_pf consumes.
-template <typename KT, int RPT, int PF>
-__device__ __forceinline__ void k_ring_request(const KT* __restrict__ Kc, int nint, const int (&v)[RPT],
-                                               const bool (&ok)[RPT], KT (&ring)[PF][RPT][9]) {
+template <int RPT, int PF>
+__device__ __forceinline__ void k_ring_request(const double* __restrict__ Kc, int nint, const int (&v)[RPT],
+                                               const bool (&ok)[RPT], double (&ring)[PF][RPT][9]) {
   int vi[RPT];
   clamp_rows<RPT>(v, ok, vi);
-  const KRows<KT, RPT> kr(Kc, nint, vi);
+  const KRows<RPT> kr(Kc, nint, vi);
 #pragma unroll
   for (int p = 0; p < PF; p++)
 #pragma unroll
@@ -823,10 +819,10 @@ __device__ __forceinline__ void k_ring_request(const KT* __restrict__ Kc, int ni
 // copies.  A wave then waits for a K load once per PF points instead of
 // once per point; PF x RPT x 9 stays below the 63 vector loads a wave can
 // have outstanding.  Same arithmetic, in the same order, as stencil_rows_pp.
-template <typename KT, typename VT, int RPT, int PF, typename Load>
-__device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int nint, const int (&v)[RPT],
-                                                const bool (&ok)[RPT], int m, Load load, KT (&ring)[PF][RPT][9],
-                                                VT (&acc)[RPT][3][RG]) {
+template <int RPT, int PF, typename Load>
+__device__ __forceinline__ void stencil_rows_pf(const double* __restrict__ Kc, int nint, const int (&v)[RPT],
+                                                const bool (&ok)[RPT], int m, Load load, double (&ring)[PF][RPT][9],
+                                                double (&acc)[RPT][3][RG]) {
   static_assert(PF >= 1 && NS % PF == 0 && PF * RPT * 9 <= 63, "prefetch ring: PF must divide 15, <= 63 loads");
   int vi[RPT];
   clamp_rows<RPT>(v, ok, vi);
@@ -836,7 +832,7 @@ __device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int n
     for (int a = 0; a < 3; a++)
 #pragma unroll
       for (int r = 0; r < RG; r++) acc[q][a][r] = 0;
-  const KRows<KT, RPT> kr(Kc, nint, vi);
+  const KRows<RPT> kr(Kc, nint, vi);
 #pragma unroll
   for (int s0 = 0; s0 < NS; s0 += PF) {
 #pragma unroll
@@ -848,13 +844,13 @@ __device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int n
         const int u = neighbour_row(vi[q], off, nint);
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-          VT pv[RG];
+          double pv[RG];
           load(u, b, pv);
 #pragma unroll
           for (int r = 0; r < RG; r++) {
-            acc[q][0][r] += (VT)ring[p][q][0 * 3 + b] * pv[r];
-            acc[q][1][r] += (VT)ring[p][q][1 * 3 + b] * pv[r];
-            acc[q][2][r] += (VT)ring[p][q][2 * 3 + b] * pv[r];
+            acc[q][0][r] += ring[p][q][0 * 3 + b] * pv[r];
+            acc[q][1][r] += ring[p][q][1 * 3 + b] * pv[r];
+            acc[q][2][r] += ring[p][q][2 * 3 + b] * pv[r];
           }
         }
       }
@@ -871,14 +867,15 @@ __device__ __forceinline__ void stencil_rows_pf(const KT* __restrict__ Kc, int n
 
 // Register-resident forms of the three phases: thread t owns rows
 // t + q * blockDim.x (q < RPT) for the whole task, and keeps their r, q and
-// diagonal inverses in registers (d in registers or in LDS behind p), so an
-// inner iteration reads only K from memory (p stays in LDS: the stencil
-// reads the neighbours' entries).  Rows at or beyond nint (ok false) carry
+// diagonal inverses in registers (d in LDS behind p), so an inner iteration
+// reads only K from memory (p stays in LDS: the stencil reads the
+// neighbours' entries).  FP64 only.  Rows at or beyond nint (ok false) carry
 // values that are never used.
-template <typename T, int RPT, int PF>
-__device__ __forceinline__ void phase_spmv_reg(const T* __restrict__ K, int nint, int m, const T* P, T (&ring)[PF][RPT][9], T (&Qr)[RPT][3][RG],
+template <int RPT, int PF>
+__device__ __forceinline__ void phase_spmv_reg(const double* __restrict__ K, int nint, int m, const double* P,
+                                               double (&ring)[PF][RPT][9], double (&Qr)[RPT][3][RG],
                                                double (&w)[RG]) {
-  auto ld = [&](int u, int b, T (&pv)[RG]) {
+  auto ld = [&](int u, int b, double (&pv)[RG]) {
 #pragma unroll
     for (int r = 0; r < RG; r++) pv[r] = P[lds_at(u, b, r)];
   };
@@ -889,56 +886,55 @@ __device__ __forceinline__ void phase_spmv_reg(const T* __restrict__ K, int nint
     vr[q] = threadIdx.x + q * blockDim.x;
     ok[q] = vr[q] < nint;
   }
-  stencil_rows_pf<T, T, RPT, PF>(K, nint, vr, ok, m, ld, ring, Qr);
-  // the row's three components are summed in T before the FP64 partial
-  // (one conversion and FP64 add per right-hand side instead of three)
+  stencil_rows_pf<RPT, PF>(K, nint, vr, ok, m, ld, ring, Qr);
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
     if (!ok[q]) continue;
 #pragma unroll
     for (int r = 0; r < RG; r++) {
-      T t = 0;
+      double t = 0;
 #pragma unroll
       for (int a = 0; a < 3; a++) t += Qr[q][a][r] * P[lds_at(vr[q], a, r)];
-      w[r] += (double)t;
+      w[r] += t;
     }
   }
 }
 
-template <typename T, int RPT>
-__device__ __forceinline__ void phase_update_reg(int nint, const T (&dv)[RPT][3], const T* P, const T (&Qr)[RPT][3][RG],
-                                                 T (&Rr)[RPT][3][RG], T* DL, const T (&alpha)[RG],
-                                                 double (&w)[2 * RG]) {
+template <int RPT>
+__device__ __forceinline__ void phase_update_reg(int nint, const double (&dv)[RPT][3], const double* P,
+                                                 const double (&Qr)[RPT][3][RG], double (&Rr)[RPT][3][RG], double* DL,
+                                                 const double (&alpha)[RG], double (&w)[2 * RG]) {
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
     const int v = threadIdx.x + q * blockDim.x;
     if (v >= nint) continue;
-    T tz[RG], tr[RG];  // the row's three components summed in T first
+    double tz[RG], tr[RG];
 #pragma unroll
     for (int r = 0; r < RG; r++) tz[r] = tr[r] = 0;
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
       for (int r = 0; r < RG; r++) {
-        const T pe = P[lds_at(v, a, r)];
+        const double pe = P[lds_at(v, a, r)];
         DL[lds_at(v, a, r)] += alpha[r] * pe;
-        const T rv = Rr[q][a][r] - alpha[r] * Qr[q][a][r];
+        const double rv = Rr[q][a][r] - alpha[r] * Qr[q][a][r];
         Rr[q][a][r] = rv;
-        const T z = dv[q][a] * rv;
+        const double z = dv[q][a] * rv;
         tz[r] += rv * z;
         tr[r] += rv * rv;
       }
 #pragma unroll
     for (int r = 0; r < RG; r++) {
-      w[r] += (double)tz[r];
-      w[RG + r] += (double)tr[r];
+      w[r] += tz[r];
+      w[RG + r] += tr[r];
     }
   }
 }
 
-template <typename T, int RPT>
-__device__ __forceinline__ void phase_direction_reg(int nint, const T (&dv)[RPT][3], T* P, const T (&Rr)[RPT][3][RG],
-                                                    const T (&beta)[RG], int on) {
+template <int RPT>
+__device__ __forceinline__ void phase_direction_reg(int nint, const double (&dv)[RPT][3], double* P,
+                                                    const double (&Rr)[RPT][3][RG], const double (&beta)[RG],
+                                                    int on) {
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
     const int v = threadIdx.x + q * blockDim.x;
@@ -982,12 +978,6 @@ __device__ __forceinline__ int dpp_partner_i32(int v, int o) {
     default: return __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, false); // row_mirror (o = 8)
   }
 }
-// lane l of every row of 16 gets lane l ^ 8's value (DPP row_ror:8)
-__device__ __forceinline__ double row_ror8_f64(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x128, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x128, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
 __device__ __forceinline__ double partner_f64(double v, int o) {
   if (o >= 16) return __shfl_xor(v, o, 64);
   const int lo = dpp_partner_i32(__double2loint(v), o);
@@ -1016,23 +1006,7 @@ __device__ __forceinline__ double wg_reduce_to_lanes(double (&v)[N], double* par
       // of that value in the other: one swap per 32-bit half and an add,
       // with no selects and no LDS round trip
 #pragma unroll
-      for (int i = 0; i < h; i++) {
-        const unsigned al = (unsigned)__double2loint(a[i]), ah = (unsigned)__double2hiint(a[i]);
-        const unsigned bl = (unsigned)__double2loint(a[h + i]), bh = (unsigned)__double2hiint(a[h + i]);
-        double x0, x1;
-        if (o == 32) {
-          const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
-          const auto hh = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
-          x0 = __hiloint2double((int)hh[0], (int)l[0]);
-          x1 = __hiloint2double((int)hh[1], (int)l[1]);
-        } else {
-          const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
-          const auto hh = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
-          x0 = __hiloint2double((int)hh[0], (int)l[0]);
-          x1 = __hiloint2double((int)hh[1], (int)l[1]);
-        }
-        a[i] = x0 + x1;
-      }
+      for (int i = 0; i < h; i++) a[i] = o == 32 ? swap_add<32>(a[i], a[h + i]) : swap_add<16>(a[i], a[h + i]);
       continue;
     }
 #pragma unroll
@@ -1262,8 +1236,8 @@ void k_batch_solve(SolveArgs A) {
             double acc[1][3][RG];
             // unrolled, with the next point's K in flight
             double kr1[1][1][9];
-            k_ring_request<double, 1, 1>(K64, nint, vr, ok, kr1);
-            stencil_rows_pf<double, double, 1, 1>(K64, nint, vr, ok, m, lds_ld, kr1, acc);
+            k_ring_request<1, 1>(K64, nint, vr, ok, kr1);
+            stencil_rows_pf<1, 1>(K64, nint, vr, ok, m, lds_ld, kr1, acc);
             if (!ok[0]) continue;
 #pragma unroll
             for (int a = 0; a < 3; a++)
@@ -1508,7 +1482,7 @@ void k_batch_solve(SolveArgs A) {
             vr[q] = tid + q * nth;
             ok[q] = vr[q] < nint;
           }
-          if constexpr (fp64) k_ring_request<double, RQ, kPrefetch>(K64, nint, vr, ok, kring);
+          if constexpr (fp64) k_ring_request<RQ, kPrefetch>(K64, nint, vr, ok, kring);
         }
       }
       if (act && inner_cap > 0) do {
@@ -1519,7 +1493,7 @@ void k_batch_solve(SolveArgs A) {
 #pragma unroll
           for (int r = 0; r < RG; r++) w[r] = 0;
           if constexpr (REG)
-            phase_spmv_reg<T, RQ, kPrefetch>(K64, nint, m, P, kring, Qr, w);
+            phase_spmv_reg<RQ, kPrefetch>(K64, nint, m, P, kring, Qr, w);
           else
             phase_spmv<T, RPT>(K32, K64, nint, m, P, Q, w);
           // alpha of right-hand side r computed in lane r, then broadcast
@@ -1540,7 +1514,7 @@ void k_batch_solve(SolveArgs A) {
 #pragma unroll
           for (int r = 0; r < 2 * RG; r++) w[r] = 0;
           if constexpr (REG)
-            phase_update_reg<T, RQ>(nint, dvr, P, Qr, Rr, DL, alpha, w);
+            phase_update_reg<RQ>(nint, dvr, P, Qr, Rr, DL, alpha, w);
           else
             phase_update<T, RPT>(nint, dinv, P, Q, R, D, alpha, w);
           // lane r < RG decides right-hand side r from its r.z (lane r) and
@@ -1552,7 +1526,7 @@ void k_batch_solve(SolveArgs A) {
           const double rz_old = S.rz[par][sl], itol2 = S.itol2[sl], rrmin = S.rrmin[par][sl];
           const int itbase = S.itbase[sl], itmin = S.itmin[par][sl];
           const double rzl = wg_reduce_to_lanes<2 * RG>(w, partA);
-          const double rrl = row_ror8_f64(rzl);
+          const double rrl = row_rotated<0x128>(rzl);
           const bool mine = lane < RG && ((act >> lane) & 1);
           bool cont = false, stag = false;
           T be = 0;
@@ -1591,7 +1565,7 @@ void k_batch_solve(SolveArgs A) {
         }
         // p = z + beta p (continuing RHS only)
         if constexpr (REG)
-          phase_direction_reg<T, RQ>(nint, dvr, P, Rr, beta, act2);
+          phase_direction_reg<RQ>(nint, dvr, P, Rr, beta, act2);
         else
           phase_direction<T, RPT>(nint, dinv, P, R, beta, act2);
         __syncthreads();
@@ -1948,11 +1922,6 @@ __host__ __device__ __forceinline__ int face_bw(int m) { return 3 * (m + 1) + 2;
 size_t face_lds_bytes(int max_n) {
   const int m = max_n - 1, N = 3 * m * m, bw = face_bw(m);
   return sizeof(double) * ((size_t)N * (bw + 1) + (size_t)N * FRHS + 2 * FRHS);
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
 }
 
 __global__ __launch_bounds__(F_THREADS) void k_face_traces(const Cell* __restrict__ cells,

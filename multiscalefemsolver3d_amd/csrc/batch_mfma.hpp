@@ -507,12 +507,15 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
         unsigned act2;
         float beta[C];
         {
-          // d, r and r.z group by group, then r.r from the new r: fewer sums
-          // are live beside q.  (One conversion and FP64 products: 1.5 % less
-          // time than FP32 products converted one by one.)
-          double w[C];
+          // d, r, r.z and r.r group by group; where q and d leave no registers
+          // for both sums, r.r afterwards from the new r (8^3 cells 17.8 ms,
+          // both at once 18.4; 10^3 cells 13.0 and 12.8, 6^3 4.50 and 4.38).
+          // One conversion and FP64 products: 1.5 % less time than FP32
+          // products converted one by one.
+          constexpr bool both = NR < 24 || G < 3;
+          double w[C], w2[C];
 #pragma unroll
-          for (int j = 0; j < C; j++) w[j] = 0;
+          for (int j = 0; j < C; j++) w[j] = w2[j] = 0;
 #pragma unroll
           for (int g = 0; g < G; g++) {
             const int v = row(g);
@@ -529,23 +532,24 @@ __device__ __forceinline__ void mfma_task(const SolveArgs& A, const Cell& C_, in
                   D[g][a][j - DJ] += alpha[j] * pe;
                 const float rv = R[g][a][j] - alpha[j] * Q[g][j][a];
                 R[g][a][j] = rv;
-                const double rd = rv;
-                w[j] += (rd * rd) * dvd;
+                const double rd = rv, r2 = rd * rd;
+                w[j] += r2 * dvd;
+                if (both) w2[j] += r2;
               }
             }
           }
           mfma_wave_sums<C>(w, partA);
+          if constexpr (!both) {
 #pragma unroll
-          for (int j = 0; j < C; j++) w[j] = 0;
+            for (int g = 0; g < G; g++) {
+              if (row(g) >= nint) continue;
 #pragma unroll
-          for (int g = 0; g < G; g++) {
-            if (row(g) >= nint) continue;
+              for (int j = 0; j < C; j++)
 #pragma unroll
-            for (int j = 0; j < C; j++)
-#pragma unroll
-              for (int a = 0; a < 3; a++) w[j] += (double)R[g][a][j] * (double)R[g][a][j];
+                for (int a = 0; a < 3; a++) w2[j] += (double)R[g][a][j] * (double)R[g][a][j];
+            }
           }
-          mfma_wave_sums<C>(w, partA + 4 * C * W);
+          mfma_wave_sums<C>(w2, partA + 4 * C * W);
           const double rz_old = S.rz[par][sl], itol2 = S.itol2[sl], rrmin = S.rrmin[par][sl];
           const int itbase = S.itbase[sl], itmin = S.itmin[par][sl];
           __syncthreads();

@@ -39,9 +39,9 @@ HBM_PEAK_GBS = 8000.0
 # WRITE_SIZE (2,179.2 KiB, x1.000), medians over 7,752 / 7,731 dispatches
 TRAFFIC_K1 = 29470310
 # HBM bytes of one k_batch_solve_mfma launch on the headline workload
-# (learned guess): rocprofv3 --pmc FETCH_SIZE 305,591,982.7 KiB x2.000 +
-# WRITE_SIZE 44,746,298.5 KiB x1.000 (the copy calibration above).
-TRAFFIC_BATCH = 671672590233
+# (learned guess): rocprofv3 --pmc FETCH_SIZE 305,459,659.1 KiB x2.000 +
+# WRITE_SIZE 44,612,162.0 KiB x1.000 (the copy calibration above).
+TRAFFIC_BATCH = 671264235745
 
 
 def log(*a):
@@ -71,7 +71,8 @@ def main():
     ap.add_argument("--train-cells", type=int, default=20000)
     ap.add_argument("--epochs", type=int, default=20)
     ap.add_argument("--shape", default="", help="headline batch-solve launch shape WG,VARIANT for both precisions, "
-                                               "or WG,VARIANT,WG64,VARIANT64, instead of the autotuner (counter runs)")
+                                               "or WG,VARIANT,WG64,VARIANT64, instead of the autotuner (counter runs; "
+                                               "the mixed launch on these cells has a shape of its own)")
     ap.add_argument("--n", type=int, default=64, help="Laplace leg: mesh hexes per edge")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline legs")
     ap.add_argument("--cpu-budget", type=float, default=20.0, help="seconds of CPU baseline work per leg")
@@ -261,8 +262,8 @@ def bench_headline(mfs, ctx, args):
                     "right-hand sides plus 11 vector passes per right-hand side and iteration; the "
                     "kernel keeps the vectors on chip (registers, LDS, L2), so the "
                     "algorithmic rate is an effective one that can exceed the HBM peak, while the "
-                    "measured traffic (FETCH_SIZE/WRITE_SIZE) is 0.29 of those bytes: mostly K "
-                    "that the tasks of a cell no longer find in their L2"}
+                    "measured traffic (FETCH_SIZE/WRITE_SIZE) is 0.29 of those bytes: mostly K, "
+                    "203 KB per cell and iteration (32 cells at a time exceed an XCD's 4 MB L2)"}
     # the GEMM of the network alone at a large size (MFMA utilisation)
     gms, gtf = mfs.gemm_bf16_time(ctx, 8192, 8192, 8192, reps=5)
     detail["gemm_bf16_kernel_8192cubed"] = {"ms": round(gms, 3), "tflops": round(gtf, 1),

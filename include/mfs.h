@@ -338,17 +338,21 @@ typedef struct {
   int maxit;       /* inner iteration cap per problem                         */
   double inner_tol;/* MIXED: FP32 inner relative tolerance                    */
   int use_graph;   /* capture the persistent launch in a hipGraph             */
-  int wg_size;     /* workgroup size (0 = autotuned; 64..256, 512 for
-                      variant 3)                                             */
+  int wg_size;     /* workgroup size (0 = autotuned or default; 64..256, 512
+                      for variant 3)                                         */
   int use_guess;   /* start from mfs_batch_set_guess values                   */
   int variant;     /* kernel variant: 0 = autotuned/default; rows carried
                       per thread: FP32 inner 1 -> 2 rows, 2 -> 3 rows;
                       FP64 inner 1 -> 1 row, 2 -> 2 rows; with r, d, q
                       kept in registers: 3 -> 1 row (wg_size up to 512),
                       4 -> 2 rows (these need nint <= rows * wg_size for
-                      every cell, else MFS_ERR_ARG).  MIXED on cells of
-                      n <= 10 runs the matrix-core kernel, which has one
-                      shape, for every variant and wg_size accepted        */
+                      every cell, else MFS_ERR_ARG).  A batch whose cells
+                      all have n <= 10 solves MIXED with the matrix-core
+                      kernel, whose shape follows from the cells; variant
+                      and wg_size then select nothing, and the same ones
+                      are refused as for the vector kernels: variants 1, 2
+                      and 4 with wg_size > 256, 3 with nint > wg_size, 4
+                      with nint > 2 wg_size                                 */
   int fallback_wg_size;  /* MIXED: shape of the FP64 pass over the problems  */
   int fallback_variant;  /* the FP32 launch could not solve (0 = the FP64
                             autotuned shape, else as wg_size / variant)      */
@@ -393,7 +397,8 @@ int mfs_batch_set_guess(mfs_batch B, const double* guess);
 /* Download basis of one cell: 24 x n_total (full fine vectors, boundary
  * traces included), basis index 3*coarse_node + direction. */
 int mfs_batch_get_basis(mfs_batch B, int cell, double* basis);
-/* Coarse element matrices Kc = Phi^T K Phi, 24x24 per cell, all cells. */
+/* Coarse element matrices Kc = Phi^T K Phi, 24x24 per cell, all cells (the
+ * batch keeps a device buffer of them, 4.6 KB per cell, from the first call). */
 int mfs_batch_coarse_matrices(mfs_batch B, double* Kc);
 /* Per-problem inner iteration counts, 24 per cell. */
 int mfs_batch_iterations(mfs_batch B, int32_t* iters);

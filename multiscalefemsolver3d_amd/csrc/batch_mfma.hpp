@@ -17,19 +17,24 @@
 //
 // What else it buys: one task per cell instead of three reads K once per
 // iteration for all 24 right-hand sides, and the three barriers and the
-// scalar work of an iteration are shared by them too.
+// scalar work of an iteration are shared by them too.  (With one task per
+// cell nothing shares K in L2: 32 cells at a time hold 6.5 MB of it, an XCD's
+// L2 4 MB, so K comes from the fabric in every iteration.)
 //
 // K is stored for it in lane order (k32_tile_index).  Lanes with
 // lane % 4 == 3 read their neighbour's 16 bytes again.
 //
 // Bound and measurements (8^3 cells, one workgroup per CU, core cycles per
-// iteration of a cell): the product takes 14,200, against 13,000 of MFMA
+// iteration of a cell): the product took 14,200, against 13,000 of MFMA
 // issue on the fullest SIMD; the update 5,100, the two reductions 8,500, the
-// new direction 3,400.  An FP64 residual pass costs as much as 4 to 7
-// iterations (K64 comes from HBM).  32,768 cells of 8^3 from zero: 151 ms,
-// against 215 ms for the one-row-per-thread vector kernel it replaces and
-// 490 ms for the slab kernel (2 rows per thread) that untuned calls ran;
-// 16^3 cells of n = 6..10: 29.6 against 85.1 ms.
+// new direction 3,400; the FP64 sums of single products have since added
+// about 1,200.  No unit is saturated over a launch (matrix cores busy 25 %,
+// vector issue 35 %, LDS 38 %; a wave waits 46 % of its time): the phases
+// follow each other behind barriers.  An FP64 residual pass costs as much as
+// 4 to 7 iterations (K64 comes from HBM, twice).  32,768 cells of 8^3 from
+// zero: 160 ms, against 215 ms for the one-row-per-thread vector kernel it
+// replaces and 490 ms for the slab kernel (2 rows per thread) that untuned
+// calls ran; 16^3 cells of n = 6..10: 29.1 against 85.1 ms.
 //
 // What decided it, one at a time at 4,096 cells of 8^3: everything in
 // registers, spilled d 38.9 ms; half of d in LDS, addresses formed where they
